@@ -1,5 +1,7 @@
 /*
- * Direct cross-correlation kernel for gfx950 (the "plain" visibility path).
+ * Direct cross-correlation kernel for gfx950 (the "plain" visibility path)
+ * with a Gaussian or smearing factor per baseline; without one the sum is a
+ * matrix product (xcorr_product.hip).
  *
  * Computes, for every baseline (p > q) outside the uv filter,
  *     V_pq += sum_s smear_s(pq) * J_first(s) B_s J_second(s)^H
@@ -40,6 +42,7 @@
 #include "device_common.h"
 #include "private.h"
 #include "workspace.h"
+#include "xcorr_common.h"
 
 using namespace oskar_amd;
 
@@ -57,57 +60,6 @@ namespace {
 constexpr int BLOCK_A = 32;    /* "first" stations per workgroup */
 constexpr int BLOCK_B = 16;    /* "second" stations per workgroup */
 constexpr int THREADS = 256;
-constexpr double OMEGA_EARTH = 7.272205217e-5; /* rad/s, define_correlate_utils.h:3 */
-
-template <typename FP>
-struct XcorrArgs
-{
-    int num_sources, num_stations, offset_out, use_casa;
-    int src_per_split, num_splits;
-    const void* jones;
-    const FP *I, *Q, *U, *V, *l, *m, *n, *a, *b, *c;
-    const FP *st_u, *st_v, *st_w, *st_x, *st_y;
-    FP uv_min, uv_max, inv_wl, frac_bw, time_int, gha0, dec0;
-    void* vis;
-    double* partial;
-};
-
-/* Baseline-dependent terms, written exactly as OSKAR_BASELINE_TERMS and
- * OSKAR_BASELINE_DELTAS (define_correlate_utils.h:5-26) with p = SP, q = SQ. */
-template <typename FP, bool TS>
-struct BaselineTerms
-{
-    FP uu, vv, ww, uu2, vv2, uuvv, uv_len, du, dv, dw;
-
-    __device__ __forceinline__ void init(const XcorrArgs<FP>& A, int sp,
-            int sq)
-    {
-        uu = (A.st_u[sp] - A.st_u[sq]) * A.inv_wl;
-        vv = (A.st_v[sp] - A.st_v[sq]) * A.inv_wl;
-        ww = (A.st_w[sp] - A.st_w[sq]) * A.inv_wl;
-        uu2 = uu * uu;
-        vv2 = vv * vv;
-        uv_len = sqrt(uu2 + vv2);
-        uuvv = 2 * uu * vv;
-        const FP f = pi_v<FP>() * A.frac_bw;
-        uu *= f; vv *= f; ww *= f;
-        du = dv = dw = (FP) 0;
-        if (TS)
-        {
-            FP sin_ha, cos_ha, sin_dec, cos_dec;
-            sincos_v<FP>(A.gha0, &sin_ha, &cos_ha);
-            sincos_v<FP>(A.dec0, &sin_dec, &cos_dec);
-            FP temp = pi_v<FP>() * A.inv_wl;
-            const FP xx = (A.st_x[sp] - A.st_x[sq]) * temp;
-            const FP yy = (A.st_y[sp] - A.st_y[sq]) * temp;
-            const FP rot = ((FP) OMEGA_EARTH) * A.time_int;
-            temp = (xx * sin_ha + yy * cos_ha) * rot;
-            du = (xx * cos_ha - yy * sin_ha) * rot;
-            dv = temp * sin_dec;
-            dw = -temp * cos_dec;
-        }
-    }
-};
 
 template <typename FP, bool GAUSS, bool BS, bool TS>
 __device__ __forceinline__ FP smearing(const BaselineTerms<FP, TS>& t,
@@ -124,9 +76,8 @@ __device__ __forceinline__ FP smearing(const BaselineTerms<FP, TS>& t,
  * value is moved as VPE vectors of VR reals (16 bytes, or 8 for a float
  * complex scalar); TILE * VPE = 64, so one wave loads one station row of
  * a tile with consecutive lanes on consecutive bytes. */
-/* Matrix kernels stage 16 sources per tile: with the FP32 inner loop
- * taking two sources per iteration for point sources without smearing
- * and one otherwise, every FP32 matrix variant fits 128 VGPRs and 26 KB of
+/* Matrix kernels stage 16 sources per tile: with one source per iteration
+ * of the inner loop every FP32 matrix variant fits 128 VGPRs and 26 KB of
  * LDS, four waves per SIMD. */
 template <typename FP, bool MATRIX> struct Geometry
 {
@@ -137,11 +88,6 @@ template <typename FP, bool MATRIX> struct Geometry
     /* Station rows of a tile moved by one wave instruction. */
     static constexpr int RPI = 64 / (TILE * VPE);
     static_assert(RPI * TILE * VPE == 64, "whole station rows per wave");
-};
-
-template <typename FP, int VR> struct alignas(VR * sizeof(FP)) Vec
-{
-    FP v[VR];
 };
 
 /* Four source values, read from LDS as one vector. */
@@ -276,10 +222,8 @@ void xcorr_direct_kernel(XcorrArgs<FP> A)
         if constexpr (MATRIX)
         {
             /* M = J_first * B once per (source, first station) of the tile,
-             * in place of J_first: B = [[I+Q, U+iV], [U-iV, I-Q]]
-             * (define_correlate_utils.h:36-39), M = J B
-             * (define_multiply.h:69-87).  Each entry is read and written
-             * by one thread. */
+             * in place of J_first.  Each entry is read and written by one
+             * thread. */
             for (int i = tid; i < TILE * BLOCK_A; i += THREADS)
             {
                 const int s = i / BLOCK_A, a = i - s * BLOCK_A;
@@ -288,20 +232,9 @@ void xcorr_direct_kernel(XcorrArgs<FP> A)
                 FP ja[8];
 #pragma unroll
                 for (int r = 0; r < 8; ++r) ja[r] = e[r];
-                const FP Ii = fl.x, Qi = fl.y, Ui = fl.z, Vi = fl.w;
-                const FP ba = Ii + Qi, bd = Ii - Qi;
-                /* M.a = a*ba + b*conj(U+iV) */
-                e[0] = ja[0] * ba + (ja[2] * Ui + ja[3] * Vi);
-                e[1] = ja[1] * ba + (ja[3] * Ui - ja[2] * Vi);
-                /* M.b = b*bd + a*(U+iV) */
-                e[2] = ja[2] * bd + (ja[0] * Ui - ja[1] * Vi);
-                e[3] = ja[3] * bd + (ja[0] * Vi + ja[1] * Ui);
-                /* M.c = c*ba + d*conj(U+iV) */
-                e[4] = ja[4] * ba + (ja[6] * Ui + ja[7] * Vi);
-                e[5] = ja[5] * ba + (ja[7] * Ui - ja[6] * Vi);
-                /* M.d = d*bd + c*(U+iV) */
-                e[6] = ja[6] * bd + (ja[4] * Ui - ja[5] * Vi);
-                e[7] = ja[7] * bd + (ja[4] * Vi + ja[5] * Ui);
+                row_times_brightness<FP>(ja, fl.x, fl.y, fl.z, fl.w, e);
+                row_times_brightness<FP>(ja + 4, fl.x, fl.y, fl.z, fl.w,
+                        e + 4);
             }
             __syncthreads();
         }
@@ -312,11 +245,10 @@ void xcorr_direct_kernel(XcorrArgs<FP> A)
 #pragma unroll
             for (int r = 0; r < NR; ++r) t[k][r] = (FP) 0;
 
-        /* Two sources per iteration in FP32, except in the matrix form
-         * with a smearing or Gaussian factor: one there (the factor's
-         * registers would leave three waves per SIMD); one in FP64. */
-        constexpr int UNROLL = (sizeof(FP) == 4 &&
-                (!MATRIX || !(GAUSS || BS || TS))) ? 2 : 1;
+        /* Two sources per iteration in the FP32 scalar form; one in the
+         * matrix form (more registers would leave three waves per SIMD)
+         * and in FP64. */
+        constexpr int UNROLL = (sizeof(FP) == 4 && !MATRIX) ? 2 : 1;
 #pragma unroll UNROLL
         for (int s = 0; s < TILE; ++s)
         {
@@ -542,10 +474,14 @@ template <typename FP, bool MATRIX>
 hipError_t dispatch(const XcorrArgs<FP>& A, bool gauss, bool bs, bool ts,
         hipStream_t s, double* fixed)
 {
+    /* No factor depends on the baseline: one matrix product. */
+    if (!gauss && !bs && !ts)
+        return xcorr_product_launch<FP, MATRIX>(A, s, fixed,
+                XCORR_SCRATCH_BYTES);
 #define XC_CASE(G_, B_, T_) if (gauss == G_ && bs == B_ && ts == T_) \
         return launch_t<FP, MATRIX, G_, B_, T_>(A, s, fixed);
-    XC_CASE(false, false, false) XC_CASE(false, false, true)
-    XC_CASE(false, true, false)  XC_CASE(false, true, true)
+    XC_CASE(false, false, true)  XC_CASE(false, true, false)
+    XC_CASE(false, true, true)
     XC_CASE(true, false, false)  XC_CASE(true, false, true)
     XC_CASE(true, true, false)   XC_CASE(true, true, true)
 #undef XC_CASE
