@@ -92,8 +92,9 @@ void oskar_cross_correlate_factorised_jones(
         oskar_Mem* vis,
         int* status);
 
-/* Sources per part of oskar_cross_correlate_factorised_jones() (default
- * and maximum 2048; multiple of 4).  Returns the previous value. */
+/* Most sources per part of oskar_cross_correlate_factorised_jones()
+ * (default and maximum 2048; multiple of 4).  A call takes fewer where that
+ * keeps more of the chip busy.  Returns the previous value. */
 OSKAR_EXPORT int oskar_cross_correlate_factorised_jones_set_part_size(
         int sources);
 
@@ -103,8 +104,9 @@ OSKAR_EXPORT int oskar_cross_correlate_factorised_jones_set_part_size(
 OSKAR_EXPORT int oskar_cross_correlate_factorised_jones_last_times(
         double ms[3]);
 
-/* Sources accumulated in FP32 by one workgroup before the FP64 sum
- * (default 8192; multiple of 8).  Returns the previous value. */
+/* Most sources accumulated in FP32 by one workgroup before the FP64 sum
+ * (default 8192; multiple of 8).  A call takes fewer where that keeps more
+ * of the chip busy.  Returns the previous value. */
 OSKAR_EXPORT int oskar_cross_correlate_factorised_set_part_size(int sources);
 
 /* Tile shape of oskar_cross_correlate_factorised(), as for batches

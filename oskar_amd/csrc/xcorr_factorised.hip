@@ -59,6 +59,7 @@
 #include <vector>
 
 #include "device_common.h"
+#include "fact_parts.h"
 #include "private.h"
 #include "workspace.h"
 
@@ -930,31 +931,35 @@ __device__ __forceinline__ void block_max_to(float mx, unsigned int* cmax,
                 __HIP_MEMORY_SCOPE_AGENT);
 }
 
-/* Sum over parts in FP64 of one station row p (q from thread, stepping by
- * the workgroup size), scale removal, and accumulation into
- * vis[offset_out + b] for baselines inside the uv filter.  Consecutive
- * threads read consecutive partials. */
+/* Sum over parts in FP64 of 64 baselines (p, q0 + 0..63) of station row p,
+ * scale removal, and accumulation into vis[offset_out + b] for baselines
+ * inside the uv filter.  Wave g of the workgroup adds the g-th quarter of
+ * the parts (consecutive lanes read consecutive partials) and the quarters
+ * are added in order, so that a row of a small array keeps 256 threads
+ * busy. */
+constexpr int RED_Q = 64;
+
 template <typename FP, class TL>
-__device__ __forceinline__ void reduce_row(int N, int p, int tiles,
+__device__ __forceinline__ void reduce_row(int N, int p, int q0, int tiles,
         int parts, int use_casa, const float* partial,
         const unsigned int* cmax, const double* st_uvw, double uv_min,
-        double uv_max, int offset_out, Cplx<FP>* vis)
+        double uv_max, int offset_out, Cplx<FP>* vis,
+        double (*sums)[8][RED_Q])
 {
     constexpr int TP = TL::TP, TQ = TL::TQ, TW = TL::TW;
+    const int lane = threadIdx.x % RED_Q, quarter = threadIdx.x / RED_Q;
+    const int q = q0 + lane;
     const int ib = p / TP, pl = p - ib * TP;
     const int t0 = row_first_tile(ib, N, TP, TQ);
-    const double inv = 1.0 / ((double) c_scale(cmax) * (double) K_SCALE);
-    for (int q = threadIdx.x; q < p; q += blockDim.x)
+    double vr[4] = {0, 0, 0, 0}, vi[4] = {0, 0, 0, 0};
+    if (q < p)
     {
-        /* uv filter on the baseline length in wavelengths. */
-        const double du = gld(st_uvw + 3 * p) - gld(st_uvw + 3 * q);
-        const double dv = gld(st_uvw + 3 * p + 1) - gld(st_uvw + 3 * q + 1);
-        const double len = sqrt(du * du + dv * dv);
-        if (len < uv_min || len > uv_max) continue;
         const int jb = q / TQ, ql = q - jb * TQ;
         const int t = t0 + jb;
-        double vr[4] = {0, 0, 0, 0}, vi[4] = {0, 0, 0, 0};
-        for (int k = 0; k < parts; ++k)
+        const int per = (parts + 3) / 4;
+        const int k1 = min(parts, (quarter + 1) * per);
+#pragma unroll 2
+        for (int k = quarter * per; k < k1; ++k)
         {
             const float* b = partial + ((size_t) k * tiles + t) *
                     (size_t) (2 * TP * TW) + (size_t) pl * TW + ql;
@@ -965,18 +970,43 @@ __device__ __forceinline__ void reduce_row(int N, int p, int tiles,
                 vi[ik] += (double) gld(b + TP * TW + ik * TQ);
             }
         }
-        const int bl = q * (N - 1) - (q - 1) * q / 2 + p - q - 1;
-        FP* o = (FP*) (vis + 4 * (size_t) (offset_out + bl));
+    }
+    if (quarter > 0)
+    {
 #pragma unroll
         for (int ik = 0; ik < 4; ++ik)
         {
-            /* CASA: V = (J_p B J_q^H)^H -> element [i][k] = conj(V[k][i]). */
-            const int sidx = use_casa ? ((ik & 1) * 2 + (ik >> 1)) : ik;
-            const double r = vr[sidx] * inv;
-            const double i = (use_casa ? -vi[sidx] : vi[sidx]) * inv;
-            gst(o + 2 * ik, (FP) (gld(o + 2 * ik) + (FP) r));
-            gst(o + 2 * ik + 1, (FP) (gld(o + 2 * ik + 1) + (FP) i));
+            sums[quarter - 1][ik][lane] = vr[ik];
+            sums[quarter - 1][4 + ik][lane] = vi[ik];
         }
+    }
+    __syncthreads();
+    if (quarter > 0 || q >= p) return;
+    /* uv filter on the baseline length in wavelengths. */
+    const double du = gld(st_uvw + 3 * p) - gld(st_uvw + 3 * q);
+    const double dv = gld(st_uvw + 3 * p + 1) - gld(st_uvw + 3 * q + 1);
+    const double len = sqrt(du * du + dv * dv);
+    if (len < uv_min || len > uv_max) return;
+#pragma unroll
+    for (int h = 0; h < 3; ++h)
+#pragma unroll
+        for (int ik = 0; ik < 4; ++ik)
+        {
+            vr[ik] += sums[h][ik][lane];
+            vi[ik] += sums[h][4 + ik][lane];
+        }
+    const double inv = 1.0 / ((double) c_scale(cmax) * (double) K_SCALE);
+    const int bl = q * (N - 1) - (q - 1) * q / 2 + p - q - 1;
+    FP* o = (FP*) (vis + 4 * (size_t) (offset_out + bl));
+#pragma unroll
+    for (int ik = 0; ik < 4; ++ik)
+    {
+        /* CASA: V = (J_p B J_q^H)^H -> element [i][k] = conj(V[k][i]). */
+        const int sidx = use_casa ? ((ik & 1) * 2 + (ik >> 1)) : ik;
+        const double r = vr[sidx] * inv;
+        const double i = (use_casa ? -vi[sidx] : vi[sidx]) * inv;
+        gst(o + 2 * ik, (FP) (gld(o + 2 * ik) + (FP) r));
+        gst(o + 2 * ik + 1, (FP) (gld(o + 2 * ik + 1) + (FP) i));
     }
 }
 
@@ -1085,8 +1115,11 @@ void fact_reduce_kernel(int N, int num_tiles, int num_parts, int use_casa,
         const float* partial, const unsigned int* cmax, const double* st_uvw,
         double uv_min, double uv_max, int offset_out, Cplx<FP>* vis)
 {
-    reduce_row<FP, TL>(N, blockIdx.x, num_tiles, num_parts, use_casa,
-            partial, cmax, st_uvw, uv_min, uv_max, offset_out, vis);
+    __shared__ double sums[3][8][RED_Q];
+    const int p = blockIdx.x, q0 = blockIdx.y * RED_Q;
+    if (q0 >= p) return;
+    reduce_row<FP, TL>(N, p, q0, num_tiles, num_parts, use_casa, partial,
+            cmax, st_uvw, uv_min, uv_max, offset_out, vis, sums);
 }
 
 /* ---------------------------------------------------------------------- */
@@ -1094,8 +1127,8 @@ void fact_reduce_kernel(int N, int num_tiles, int num_parts, int use_casa,
 
 struct BatchHeader
 {
-    int num_units, num_stations, num_tiles, src_per_part;
-    int total_items, prep_total, use_casa, pad0;
+    int num_units, num_stations, num_tiles, total_items;
+    int prep_total, use_casa, pad0, pad1;
 };
 
 struct UnitDesc
@@ -1113,7 +1146,7 @@ struct UnitDesc
     int item_start;              /* first work item (prefix over units) */
     int num_parts;
     int prep_start;              /* first prepare slot (256-aligned) */
-    int pad0;
+    int src_per_part;
 };
 
 /* x, through an empty asm the compiler must assume changes it: values
@@ -1201,7 +1234,6 @@ void fact_batch_kernel(const BatchHeader* H, const UnitDesc* D, int* counter)
     __shared__ int s_item;
     const int total = H->total_items, nu = H->num_units;
     const int N = H->num_stations, tiles = H->num_tiles;
-    const int spp = H->src_per_part;
     for (;;)
     {
         __syncthreads();          /* every thread has read s_item */
@@ -1213,7 +1245,7 @@ void fact_batch_kernel(const BatchHeader* H, const UnitDesc* D, int* counter)
         const int u = find_unit(nu, item,
                 [&](int k) { return D[k].item_start; });
         const UnitDesc& d = D[u];
-        const int local = item - d.item_start;
+        const int local = item - d.item_start, spp = d.src_per_part;
         const int part = local / tiles, tile = local - part * tiles;
         int ib, jb;
         tile_coords(tile, N, TL::TP, TL::TQ, &ib, &jb);
@@ -1238,15 +1270,20 @@ template <typename FP, class TL>
 __global__ __launch_bounds__(256)
 void fact_batch_reduce_kernel(const BatchHeader* H, const UnitDesc* D)
 {
+    __shared__ double sums[3][8][RED_Q];
     const int N = H->num_stations, rows = H->num_units * N;
     for (int r = blockIdx.x; r < rows; r += gridDim.x)
     {
         const int u = r / N, p = r - u * N;
         const UnitDesc& d = D[u];
         if (d.num_parts == 0) continue;      /* no sources: untouched */
-        reduce_row<FP, TL>(N, p, H->num_tiles, d.num_parts, H->use_casa,
-                d.partial, d.cmax, d.st, d.uv_min, d.uv_max, d.offset_out,
-                (Cplx<FP>*) d.vis);
+        for (int q0 = 0; q0 < p; q0 += RED_Q)
+        {
+            reduce_row<FP, TL>(N, p, q0, H->num_tiles, d.num_parts,
+                    H->use_casa, d.partial, d.cmax, d.st, d.uv_min,
+                    d.uv_max, d.offset_out, (Cplx<FP>*) d.vis, sums);
+            __syncthreads();              /* sums is reused */
+        }
     }
 }
 
@@ -1408,6 +1445,7 @@ int fact_launch_shape(int dev, int precision, int mode, int use_casa,
     A.cmax = cmax;
     A.partial = partial;
     const dim3 grid(tiles, parts);
+    const dim3 rgrid(N, (N + RED_Q - 1) / RED_Q);
     mark(dev, 1, stream);
     if (mode == 1)
         hipLaunchKernelGGL((fact_xcorr_kernel<BodyB>), grid,
@@ -1420,11 +1458,11 @@ int fact_launch_shape(int dev, int precision, int mode, int use_casa,
 
     mark(dev, 2, stream);
     if (precision == OSKAR_DOUBLE)
-        hipLaunchKernelGGL((fact_reduce_kernel<double, TL>), dim3(N),
+        hipLaunchKernelGGL((fact_reduce_kernel<double, TL>), rgrid,
                 dim3(256), 0, stream, N, tiles, parts, use_casa, partial,
                 cmax, st, uv_min, uv_max, offset_out, (Cplx<double>*) vis);
     else
-        hipLaunchKernelGGL((fact_reduce_kernel<float, TL>), dim3(N),
+        hipLaunchKernelGGL((fact_reduce_kernel<float, TL>), rgrid,
                 dim3(256), 0, stream, N, tiles, parts, use_casa, partial,
                 cmax, st, uv_min, uv_max, offset_out, (Cplx<float>*) vis);
     mark(dev, 3, stream);
@@ -1468,6 +1506,7 @@ extern "C" int oskar_amd_fact_launch(int precision, int mode, int use_casa,
     if (dev < 0 || dev >= 64) return (int) hipErrorInvalidDevice;
     if (src_per_part <= 0) src_per_part = 8192;
     src_per_part = ((src_per_part + KSRC - 1) / KSRC) * KSRC;
+    src_per_part = part_sources(S, N, src_per_part, KSRC);
 #define FACT_ARGS dev, precision, mode, use_casa, S, N, beam, I, Q, U, V, \
         l, m, n, st_u, st_v, st_w, frequency_hz, uv_min_lambda, \
         uv_max_lambda, offset_out, vis, src_per_part, stream
@@ -1594,10 +1633,25 @@ hipError_t batch_upload(Batch* b, int nu, int use_casa,
     const int N = b->N, TP = SHAPE_TP[b->cfg.shape],
             TQ = SHAPE_TQ[b->cfg.shape];
     const int tiles = num_tiles(N, TP, TQ);
-    const int spp = b->cfg.src_per_part;
+    const int max_part = b->cfg.src_per_part;
     const size_t tile_bytes = 2 * (size_t) TP * 4 * TQ * sizeof(float);
     const size_t nb = (size_t) N * (N - 1) / 2;
     const size_t vis_elem = (b->precision == OSKAR_DOUBLE ? 64 : 32);
+
+    /* A batch of less than two rounds of workgroups at the configured part
+     * size takes the one-call path's part sizes (smaller ones, which cost
+     * more partial sums, for units that leave the chip idle). */
+    long long full = 0;
+    for (int u = 0; u < nu; ++u)
+        full += part_tiles(N) * ((b->units[u].num_sources + max_part - 1) /
+                max_part);
+    std::vector<int> part(nu);
+    for (int u = 0; u < nu; ++u)
+    {
+        const int S = b->units[u].num_sources;
+        part[u] = full < 2 * PART_SLOTS && S > 0 ?
+                part_sources(S, N, max_part, KSRC) : max_part;
+    }
 
     /* Workspace layout per unit: [cmax 256 B][stations][src][cmat][partial]. */
     size_t bytes = 0;
@@ -1606,7 +1660,7 @@ hipError_t batch_upload(Batch* b, int nu, int use_casa,
     for (int u = 0; u < nu; ++u)
     {
         const int S = b->units[u].num_sources;
-        const int parts = (S + spp - 1) / spp;
+        const int parts = (S + part[u] - 1) / part[u];
         off[u] = bytes;
         bytes += 256 + align256(3 * (size_t) N * 8) +
                 align256(sizeof(Src) * (size_t) pad8(S)) +
@@ -1638,7 +1692,6 @@ hipError_t batch_upload(Batch* b, int nu, int use_casa,
     h->num_units = nu;
     h->num_stations = N;
     h->num_tiles = tiles;
-    h->src_per_part = spp;
     h->total_items = (int) items;
     h->prep_total = (int) prep;
     h->use_casa = use_casa;
@@ -1647,7 +1700,8 @@ hipError_t batch_upload(Batch* b, int nu, int use_casa,
     {
         UnitDesc d = b->units[u];
         const int S = d.num_sources;
-        const int parts = (S + spp - 1) / spp;
+        const int parts = (S + part[u] - 1) / part[u];
+        d.src_per_part = part[u];
         char* w = base + off[u];
         d.cmax = (unsigned int*) w;
         w += 256;

@@ -46,6 +46,7 @@
 #include <stdint.h>
 
 #include "device_common.h"
+#include "fact_parts.h"
 #include "private.h"
 #include "workspace.h"
 
@@ -667,25 +668,32 @@ void fs_product_kernel(int N, int S4, int SP, int tiles, const uint4* planes,
 /* ---------------------------------------------------------------------- */
 /* Reduction: FP64 sum over parts of each baseline's 2x2 block.            */
 
+/* Workgroup (p, q / 64): wave g adds the g-th quarter of the parts of 64
+ * baselines (p, q), the quarters are added in order. */
+constexpr int RED_Q = 64;
+
 template <typename FP>
 __global__ __launch_bounds__(NT)
 void fs_reduce_kernel(int N, int tiles, int parts, int use_casa,
         const float* partial, const float* scales, const double* st,
         double uv_min, double uv_max, int offset_out, Cplx<FP>* vis)
 {
+    __shared__ double sums[3][8][RED_Q];
     const int p = blockIdx.x;
+    const int lane = threadIdx.x % RED_Q, quarter = threadIdx.x / RED_Q;
+    const int q = blockIdx.y * RED_Q + lane;
+    if ((int) blockIdx.y * RED_Q >= p) return;
     const int ib = p / TS, pl = p - ib * TS;
     const int t0 = ib * (ib + 1) / 2;
-    for (int q = threadIdx.x; q < p; q += blockDim.x)
+    double vr[4] = {0, 0, 0, 0}, vi[4] = {0, 0, 0, 0};
+    if (q < p)
     {
-        const double du = st[3 * p] - st[3 * q];
-        const double dv = st[3 * p + 1] - st[3 * q + 1];
-        const double len = sqrt(du * du + dv * dv);
-        if (len < uv_min || len > uv_max) continue;
         const int jb = q / TS, ql = q - jb * TS;
         const int t = t0 + jb;
-        double vr[4] = {0, 0, 0, 0}, vi[4] = {0, 0, 0, 0};
-        for (int k = 0; k < parts; ++k)
+        const int per = (parts + 3) / 4;
+        const int k1 = min(parts, (quarter + 1) * per);
+#pragma unroll 2
+        for (int k = quarter * per; k < k1; ++k)
         {
             const double inv = 1.0 / ((double) scales[(size_t) k * N + p] *
                     (double) scales[(size_t) k * N + q]);
@@ -703,16 +711,39 @@ void fs_reduce_kernel(int N, int tiles, int parts, int use_casa,
                 vi[2 * i + 1] += (double) m.y * inv;
             }
         }
-        const int bl = q * (N - 1) - (q - 1) * q / 2 + p - q - 1;
-        FP* o = (FP*) (vis + 4 * (size_t) (offset_out + bl));
+    }
+    if (quarter > 0)
+    {
 #pragma unroll
         for (int ik = 0; ik < 4; ++ik)
         {
-            /* CASA: element [i][k] = conj(V[k][i]). */
-            const int sidx = use_casa ? ((ik & 1) * 2 + (ik >> 1)) : ik;
-            o[2 * ik] += (FP) vr[sidx];
-            o[2 * ik + 1] += (FP) (use_casa ? -vi[sidx] : vi[sidx]);
+            sums[quarter - 1][ik][lane] = vr[ik];
+            sums[quarter - 1][4 + ik][lane] = vi[ik];
         }
+    }
+    __syncthreads();
+    if (quarter > 0 || q >= p) return;
+    const double du = st[3 * p] - st[3 * q];
+    const double dv = st[3 * p + 1] - st[3 * q + 1];
+    const double len = sqrt(du * du + dv * dv);
+    if (len < uv_min || len > uv_max) return;
+#pragma unroll
+    for (int h = 0; h < 3; ++h)
+#pragma unroll
+        for (int ik = 0; ik < 4; ++ik)
+        {
+            vr[ik] += sums[h][ik][lane];
+            vi[ik] += sums[h][4 + ik][lane];
+        }
+    const int bl = q * (N - 1) - (q - 1) * q / 2 + p - q - 1;
+    FP* o = (FP*) (vis + 4 * (size_t) (offset_out + bl));
+#pragma unroll
+    for (int ik = 0; ik < 4; ++ik)
+    {
+        /* CASA: element [i][k] = conj(V[k][i]). */
+        const int sidx = use_casa ? ((ik & 1) * 2 + (ik >> 1)) : ik;
+        o[2 * ik] += (FP) vr[sidx];
+        o[2 * ik + 1] += (FP) (use_casa ? -vi[sidx] : vi[sidx]);
     }
 }
 
@@ -795,7 +826,8 @@ int fs_launch_t(int dev, int use_casa, int S, int N, const void* E,
     err = hipGetLastError();
     if (err != hipSuccess) return (int) err;
     mark(dev, 2, stream);
-    hipLaunchKernelGGL(fs_reduce_kernel<FP>, dim3(N), dim3(NT), 0, stream,
+    hipLaunchKernelGGL(fs_reduce_kernel<FP>, dim3(N,
+            (N + RED_Q - 1) / RED_Q), dim3(NT), 0, stream,
             N, tiles, parts, use_casa, partial, scales, st, uv_min, uv_max,
             offset_out, (Cplx<FP>*) vis);
     mark(dev, 3, stream);
@@ -824,6 +856,7 @@ extern "C" int oskar_amd_fact_stations_launch(int precision, int mode,
     if (dev < 0 || dev >= 64) return (int) hipErrorInvalidDevice;
     int SP = src_per_part <= 0 ? MAX_SP : src_per_part;
     SP = std::min(MAX_SP, std::max(KS, SP / KS * KS));
+    SP = part_sources(S, N, SP, KS);
 #define FS_ARGS dev, use_casa, S, N, E, ld_e, I, Q, U, V, l, m, n, st_u, \
         st_v, st_w, frequency_hz, uv_min_lambda, uv_max_lambda, offset_out, \
         vis, SP, stream
