@@ -55,7 +55,7 @@ void oskar_cross_correlate(
  * device memory: code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc.  Arguments, checks, errors and results
  * as oskar_cross_correlate(); the split-source partial sums go to a fixed
- * 64 MiB array that every device holds until the process ends, instead of
+ * 256 MiB array that every device holds until the process ends, instead of
  * a workspace the library allocates.  No input is rejected for its size:
  * when the partials of the usual split count do not fit, the sources are
  * split fewer times (down to one split, which adds to vis directly and

@@ -15,6 +15,11 @@ namespace oskar_amd {
 
 constexpr double OMEGA_EARTH = 7.272205217e-5; /* rad/s, define_correlate_utils.h:3 */
 
+/* Most FP64 partial sums of a call: they stay in the Infinity Cache, and
+ * the allocation-free entry point's array holds as many, so that it splits
+ * the sources as oskar_cross_correlate does. */
+constexpr size_t XCORR_PARTIAL_BYTES = (size_t) 256 << 20;
+
 template <typename FP>
 struct XcorrArgs
 {
@@ -93,11 +98,11 @@ __device__ __forceinline__ int baseline_index(int N, int p, int q)
 }
 
 /* xcorr_product.hip: the launch of the matrix-core product.  fixed: the
- * allocation-free entry point's scratch array of fixed_bytes, or NULL for
+ * allocation-free entry point's array of XCORR_PARTIAL_BYTES, or NULL for
  * the per-stream workspace. */
 template <typename FP, bool MATRIX>
 hipError_t xcorr_product_launch(XcorrArgs<FP> A, hipStream_t stream,
-        double* fixed, size_t fixed_bytes);
+        double* fixed);
 
 } /* namespace oskar_amd */
 

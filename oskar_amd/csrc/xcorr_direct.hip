@@ -17,22 +17,34 @@
  *    second stations t%8 and t%8 + 8.  In the matrix form M = J_first * B
  *    is formed once per (source, first station) of a staged tile, in LDS
  *    in place of J_first, and read by the 16 baselines that need it.
+ *  - Only blocks that hold a baseline are launched, as one list of (split,
+ *    block) items that the XCDs share evenly.
  *  - Sources are streamed in tiles of TILE sources.  The Jones values of the
  *    48 stations are loaded as 16-byte vectors, one station row of the tile
  *    per wave and instruction (64 lanes on consecutive bytes), and stored
- *    transposed in LDS as [source][station], so the inner loop reads a
- *    first-station value that is broadcast to 8 lanes and 16 consecutive
- *    second-station values.  Source parameters are stored as 4-value
- *    vectors, one LDS read each.
- *  - The second-station Jones is scaled by the smearing factor, and every
- *    term of M J^H is one fused multiply-add into the tile sum.
+ *    transposed in LDS as [source][vector][station], so the inner loop
+ *    reads a first-station value that is broadcast to 8 lanes and
+ *    consecutive second-station vectors, without bank conflicts.  Source
+ *    parameters are stored as 4-value vectors, one LDS read each.
+ *  - The factors of a baseline and source: the Gaussian only for sources
+ *    that are extended (a wave's sources are the same), the smearing by the
+ *    polynomials of Sinc (device_common.h).  The second-station Jones is
+ *    scaled by their product, and every term of M J^H is one fused
+ *    multiply-add into the tile sum.
  *  - Single precision: each tile is summed in FP32 registers, then folded
  *    into FP64 accumulators (cross-tile sums in FP64).  Double precision
  *    accumulates in FP64 throughout.
- *  - The source range is split over gridDim.z workgroups (split-K) so a
- *    call fills all 256 CUs; partial sums go to an FP64 workspace and a
- *    second kernel adds them to vis in a fixed order.  No atomics are used,
- *    so results are identical from run to run.
+ *  - The source range is split over workgroups; partial sums go to an FP64
+ *    workspace and a second kernel adds them to vis in a fixed order.  No
+ *    atomics are used, so results are identical from run to run.
+ *
+ * Bound: vector instructions.  FP32 matrices with all factors take 92 per
+ * evaluation, 40 of them the contraction (163 with library sines, divisions
+ * and both sinc branches), and the vector unit is busy throughout: 512
+ * stations x 20,000 sources 10.97 -> 5.84 ms.  FP64 with both smearings
+ * takes 82 (565), vector unit 64 % busy at three waves per SIMD: 255 x
+ * 10,007 sources 4.69 -> 1.19 ms.  Scalars with bandwidth smearing in FP32,
+ * 351 x 50,001: 2.54 -> 1.41 ms.
  */
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -46,14 +58,12 @@
 
 using namespace oskar_amd;
 
-/* Split partials of the allocation-free entry point: a fixed 64 MiB array
- * in every device's code object (8 splits of 512 stations' 130,816
- * baselines x 8 FP64 values fit).  Host code never passes this name to a
+/* Split partials of the allocation-free entry point: a fixed array in
+ * every device's code object.  Host code never passes this name to a
  * kernel: it is a host-side stand-in, not a device address; the device
  * address comes from hipGetSymbolAddress (scratch_address below). */
-constexpr size_t XCORR_SCRATCH_BYTES = (size_t) 64 << 20;
 static __device__ __align__(256)
-        double scratch[XCORR_SCRATCH_BYTES / sizeof(double)];
+        double scratch[XCORR_PARTIAL_BYTES / sizeof(double)];
 
 namespace {
 
@@ -61,15 +71,55 @@ constexpr int BLOCK_A = 32;    /* "first" stations per workgroup */
 constexpr int BLOCK_B = 16;    /* "second" stations per workgroup */
 constexpr int THREADS = 256;
 
-template <typename FP, bool GAUSS, bool BS, bool TS>
-__device__ __forceinline__ FP smearing(const BaselineTerms<FP, TS>& t,
-        FP l, FP m, FP n1, FP sa, FP sb, FP sc)
+/* exp2 of a Gaussian's exponent, whose a, b, c carry -log2(e) (FP32: the
+ * hardware's exp2), or exp of it with a, b, c negated (FP64). */
+__device__ __forceinline__ float gauss_scale(float) { return -1.44269504f; }
+__device__ __forceinline__ double gauss_scale(double) { return -1.0; }
+__device__ __forceinline__ float gauss_exp(float x)
 {
-    FP s = (FP) 1;
-    if (GAUSS) s = exp_v<FP>(-(sa * t.uu2 + sb * t.uuvv + sc * t.vv2));
-    if (BS) s *= sinc_v<FP>(t.uu * l + t.vv * m + t.ww * n1);
-    if (TS) s *= sinc_v<FP>(t.du * l + t.dv * m + t.dw * n1);
-    return s;
+    return __builtin_amdgcn_exp2f(x);
+}
+__device__ __forceinline__ double gauss_exp(double x) { return exp(x); }
+
+/* The smearing factors of a thread's two baselines for one source, times
+ * the Gaussian factors already in sm.  The sinc form is chosen by the
+ * largest argument in the wave: long baselines and sources far from the
+ * phase centre take the wider forms. */
+template <typename FP, bool BS, bool TS>
+__device__ __forceinline__ void smear_factors(
+        const BaselineTerms<FP, TS> (&t)[2], FP l, FP m, FP n1, FP (&sm)[2])
+{
+    using S = Sinc<FP>;
+    FP xb[2], xt[2], most = (FP) 0;
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+    {
+        if (BS)
+        {
+            xb[k] = t[k].uu * l + t[k].vv * m + t[k].ww * n1;
+            most = fmax(most, fabs(xb[k]));
+        }
+        if (TS)
+        {
+            xt[k] = t[k].du * l + t[k].dv * m + t[k].dw * n1;
+            most = fmax(most, fabs(xt[k]));
+        }
+    }
+    auto apply = [&](auto f) __attribute__((always_inline))
+    {
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+        {
+            if (BS) sm[k] *= f(xb[k]);
+            if (TS) sm[k] *= f(xt[k]);
+        }
+    };
+    if (!__any(most > S::SMALL))
+        apply([](FP x) { return S::small(x); });
+    else if (!__any(most > S::MID))
+        apply([](FP x) { return S::mid(x); });
+    else
+        apply([](FP x) { return S::large(x); });
 }
 
 /* Number of reals per Jones value and the source-tile length.  A Jones
@@ -96,9 +146,32 @@ template <typename FP> struct alignas(4 * sizeof(FP)) Quad
     FP x, y, z, w;
 };
 
+/* The station blocks that hold a baseline with the required index order:
+ * for first block ia (stations 32 ia ..), second blocks *ib0 .. *ib0 +
+ * count - 1 (stations 16 ib ..). */
+__host__ __device__ inline int blocks_in_row(int N, bool casa, int ia,
+        int* ib0)
+{
+    const int a0 = ia * BLOCK_A;
+    const int a_last = (a0 + BLOCK_A < N ? a0 + BLOCK_A : N) - 1;
+    if (casa)
+    {
+        /* first < second */
+        *ib0 = a0 / BLOCK_B;
+        return a0 < N - 1 ? (N + BLOCK_B - 1) / BLOCK_B - *ib0 : 0;
+    }
+    /* first > second */
+    *ib0 = 0;
+    return a_last > 0 ? (a_last - 1) / BLOCK_B + 1 : 0;
+}
+
+/* FP64 matrices without the Gaussian factor fit three waves per SIMD (168
+ * VGPRs and 52 KB of LDS: 1.25 -> 1.19 ms for 255 stations x 10,007
+ * sources); with it they would spill (30 x 277 sources: 21.7 -> 24.6 us). */
 template <typename FP, bool MATRIX, bool GAUSS, bool BS, bool TS>
-__global__ __launch_bounds__(THREADS)
-void xcorr_direct_kernel(XcorrArgs<FP> A)
+__global__ __launch_bounds__(THREADS, MATRIX && !GAUSS && sizeof(FP) == 8 ?
+        3 : 1)
+void xcorr_direct_kernel(XcorrArgs<FP> A, int blocks)
 {
     using G = Geometry<FP, MATRIX>;
     constexpr int NR = G::NR;
@@ -106,22 +179,35 @@ void xcorr_direct_kernel(XcorrArgs<FP> A)
     constexpr int VPE = G::VPE;
     constexpr int VR = G::VR;
     using V = Vec<FP, VR>;
-    /* Padding of one station row spreads the transposed stores over banks. */
-    __shared__ FP sJa[TILE][BLOCK_A + 1][NR];
-    __shared__ FP sJb[TILE][BLOCK_B + 1][NR];
+    /* A station's value as vectors in planes of their own, so that lanes on
+     * consecutive stations read consecutive vectors; the odd number of
+     * stations per plane spreads the transposed stores over banks. */
+    __shared__ V sJa[TILE][VPE][BLOCK_A + 1];
+    __shared__ V sJb[TILE][VPE][BLOCK_B + 1];
     __shared__ Quad<FP> sFlux[TILE];      /* I, Q, U, V */
     __shared__ Quad<FP> sDir[TILE];       /* l, m, n - 1 */
     __shared__ Quad<FP> sExt[TILE];       /* a, b, c */
 
     const int N = A.num_stations;
-    const int a0 = blockIdx.x * BLOCK_A;
-    const int b0 = blockIdx.y * BLOCK_B;
-    /* Skip blocks that hold no baseline with the required index order. */
+    /* Workgroup w runs on XCD w % 8; each XCD takes a contiguous range of
+     * (split, block) items, so that all have the same work (with a grid of
+     * all blocks, XCDs held whole block rows: 2x the average on 255
+     * stations) and the blocks of a split share an L2. */
+    const int total = (int) gridDim.x, wg = (int) blockIdx.x;
+    const int xq = total / 8, xr = total % 8, xcd = wg % 8;
+    const int item = xcd * xq + min(xcd, xr) + wg / 8;
+    const int split = item / blocks;
+    int a0, b0;
     {
-        const int a_last = min(a0 + BLOCK_A, N) - 1;
-        const int b_last = min(b0 + BLOCK_B, N) - 1;
-        const bool valid = A.use_casa ? (a0 < b_last) : (a_last > b0);
-        if (!valid || a0 >= N || b0 >= N) return;
+        int block = item % blocks, ia = 0, ib0 = 0;
+        for (;; ++ia)
+        {
+            const int c = blocks_in_row(N, A.use_casa != 0, ia, &ib0);
+            if (block < c) break;
+            block -= c;
+        }
+        a0 = ia * BLOCK_A;
+        b0 = (ib0 + block) * BLOCK_B;
     }
     const int tid = threadIdx.x;
     const int la = tid >> 3;
@@ -151,7 +237,7 @@ void xcorr_direct_kernel(XcorrArgs<FP> A)
                 !(bt[k].uv_len < A.uv_min || bt[k].uv_len > A.uv_max);
     }
 
-    const int s_begin = blockIdx.z * A.src_per_split;
+    const int s_begin = split * A.src_per_split;
     const int s_end = min(A.num_sources, s_begin + A.src_per_split);
 
     double acc[2][NR];
@@ -183,8 +269,7 @@ void xcorr_direct_kernel(XcorrArgs<FP> A)
             const int st = (wave + 4 * i) * RPI + lr;
             const bool first = st < BLOCK_A;
             const int station = first ? a0 + st : b0 + (st - BLOCK_A);
-            FP* dst = first ? &sJa[ls][st][lq * VR] :
-                    &sJb[ls][st - BLOCK_A][lq * VR];
+            V* dst = first ? &sJa[ls][lq][st] : &sJb[ls][lq][st - BLOCK_A];
             const FP* src = J + ((size_t) station * A.num_sources + s0 +
                     ls) * NR + lq * VR;
             V x;
@@ -200,7 +285,7 @@ void xcorr_direct_kernel(XcorrArgs<FP> A)
                     for (int r = 0; r < VR; ++r) x.v[r] = src[r];
                 }
             }
-            *(V*) dst = x;
+            *dst = x;
         }
         for (int s = tid; s < TILE; s += THREADS)
         {
@@ -215,8 +300,14 @@ void xcorr_direct_kernel(XcorrArgs<FP> A)
                 sDir[s] = Quad<FP>{in ? A.l[g] : z, in ? A.m[g] : z,
                         in ? A.n[g] - (FP) 1 : z, z};
             if (GAUSS)
-                sExt[s] = Quad<FP>{in ? A.a[g] : z, in ? A.b[g] : z,
-                        in ? A.c[g] : z, z};
+            {
+                /* .w: whether the source is extended. */
+                const FP f = gauss_scale(z);
+                const FP ea = in ? A.a[g] : z, eb = in ? A.b[g] : z;
+                const FP ec = in ? A.c[g] : z;
+                sExt[s] = Quad<FP>{f * ea, f * eb, f * ec,
+                        (FP) (ea != z || eb != z || ec != z)};
+            }
         }
         __syncthreads();
         if constexpr (MATRIX)
@@ -226,15 +317,23 @@ void xcorr_direct_kernel(XcorrArgs<FP> A)
              * thread. */
             for (int i = tid; i < TILE * BLOCK_A; i += THREADS)
             {
-                const int s = i / BLOCK_A, a = i - s * BLOCK_A;
-                FP* e = sJa[s][a];
+                const int s = i / BLOCK_A, a = i % BLOCK_A;
                 const Quad<FP> fl = sFlux[s];
-                FP ja[8];
+                FP ja[8], M[8];
 #pragma unroll
-                for (int r = 0; r < 8; ++r) ja[r] = e[r];
-                row_times_brightness<FP>(ja, fl.x, fl.y, fl.z, fl.w, e);
+                for (int r = 0; r < 8; ++r)
+                    ja[r] = sJa[s][r / VR][a].v[r % VR];
+                row_times_brightness<FP>(ja, fl.x, fl.y, fl.z, fl.w, M);
                 row_times_brightness<FP>(ja + 4, fl.x, fl.y, fl.z, fl.w,
-                        e + 4);
+                        M + 4);
+#pragma unroll
+                for (int v = 0; v < VPE; ++v)
+                {
+                    V x;
+#pragma unroll
+                    for (int r = 0; r < VR; ++r) x.v[r] = M[v * VR + r];
+                    sJa[s][v][a] = x;
+                }
             }
             __syncthreads();
         }
@@ -253,23 +352,40 @@ void xcorr_direct_kernel(XcorrArgs<FP> A)
         for (int s = 0; s < TILE; ++s)
         {
             const Quad<FP> fl = sFlux[s];
-            FP sm[2];
-            if (GAUSS || BS || TS)
+            FP sm[2] = {(FP) 1, (FP) 1};
+            if (GAUSS)
             {
-                const Quad<FP> d = (BS || TS) ? sDir[s] : Quad<FP>{};
-                const Quad<FP> e = GAUSS ? sExt[s] : Quad<FP>{};
+                const Quad<FP> e = sExt[s];
+                if (__any(e.w != (FP) 0))
+                {
 #pragma unroll
-                for (int k = 0; k < 2; ++k)
-                    sm[k] = smearing<FP, GAUSS, BS, TS>(bt[k], d.x, d.y, d.z,
-                            e.x, e.y, e.z);
+                    for (int k = 0; k < 2; ++k)
+                        sm[k] = gauss_exp(e.x * bt[k].uu2 +
+                                e.y * bt[k].uuvv + e.z * bt[k].vv2);
+                }
             }
-            const FP* ja = sJa[s][la];
+            if (BS || TS)
+            {
+                const Quad<FP> d = sDir[s];
+                smear_factors<FP, BS, TS>(bt, d.x, d.y, d.z, sm);
+            }
+            /* The values of this thread's stations. */
+            auto get = [](const V* planes, int pitch, FP* x)
+            {
+#pragma unroll
+                for (int v = 0; v < VPE; ++v)
+                {
+                    const V y = planes[v * pitch];
+#pragma unroll
+                    for (int r = 0; r < VR; ++r) x[v * VR + r] = y.v[r];
+                }
+            };
+            FP ja[NR];
+            get(&sJa[s][0][la], BLOCK_A + 1, ja);
             if (MATRIX)
             {
                 /* The tile holds M = J_first * B (formed after staging). */
-                FP M[8];
-#pragma unroll
-                for (int r = 0; r < 8; ++r) M[r] = ja[r];
+                const FP* M = ja;
 #pragma unroll
                 for (int k = 0; k < 2; ++k)
                 {
@@ -277,11 +393,11 @@ void xcorr_direct_kernel(XcorrArgs<FP> A)
                      * (M J^H).a = M.a conj(J.a) + M.b conj(J.b), etc.  The
                      * smearing factor scales J_second; each term is one
                      * fused multiply-add into the tile sum. */
-                    const FP* jb = sJb[s][lb + 8 * k];
-                    FP w[8];
+                    FP jb[8], w[8];
+                    get(&sJb[s][0][lb + 8 * k], BLOCK_B + 1, jb);
 #pragma unroll
                     for (int r = 0; r < 8; ++r)
-                        w[r] = (GAUSS || BS || TS) ? jb[r] * sm[k] : jb[r];
+                        w[r] = jb[r] * sm[k];
                     FP* T = t[k];
                     T[0] += M[0] * w[0]; T[0] += M[1] * w[1];
                     T[0] += M[2] * w[2]; T[0] += M[3] * w[3];
@@ -307,9 +423,10 @@ void xcorr_direct_kernel(XcorrArgs<FP> A)
 #pragma unroll
                 for (int k = 0; k < 2; ++k)
                 {
-                    const FP* jb = sJb[s][lb + 8 * k];
+                    FP jb[2];
+                    get(&sJb[s][0][lb + 8 * k], BLOCK_B + 1, jb);
                     /* J_first * conj(J_second) * (smear * I) */
-                    const FP w = (GAUSS || BS || TS) ? sm[k] * Ii : Ii;
+                    const FP w = sm[k] * Ii;
                     const FP re = ja[0] * jb[0] + ja[1] * jb[1];
                     const FP im = ja[1] * jb[0] - ja[0] * jb[1];
                     t[k][0] += re * w;
@@ -339,41 +456,57 @@ void xcorr_direct_kernel(XcorrArgs<FP> A)
         else
         {
             const size_t nb = (size_t) N * (N - 1) / 2;
-            double* w = A.partial + ((size_t) blockIdx.z * nb + bl) * NR;
+            double* w = A.partial + ((size_t) split * nb + bl) * NR;
 #pragma unroll
             for (int r = 0; r < NR; ++r) w[r] = acc[k][r];
         }
     }
 }
 
-/* Adds the split partial sums to vis in split order, skipping baselines
- * outside the uv filter.  Grid: x over the higher station index p, y = the
- * lower index q. */
-template <typename FP, int NR>
+/* Adds the split partial sums to vis in a fixed order, skipping baselines
+ * outside the uv filter.  Grid: y = the lower station index q, x over the
+ * consecutive reals of its baselines (p, q).  GROUPS groups of a workgroup
+ * add a share of the splits each (consecutive threads on consecutive
+ * partials), and the shares are added in order: 4 where there are many
+ * splits, so that a small array's sums are not one long chain (60 stations,
+ * 205 splits: 66 us with a thread per baseline). */
+template <typename FP, int NR, int GROUPS>
 __global__ __launch_bounds__(256)
 void xcorr_reduce_kernel(XcorrArgs<FP> A)
 {
+    constexpr int VALUES = 256 / GROUPS;
+    __shared__ double sums[GROUPS > 1 ? GROUPS - 1 : 1][VALUES];
     const int N = A.num_stations;
     const size_t nb = (size_t) N * (N - 1) / 2;
     const int q = blockIdx.y;
-    const int p = q + 1 + blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= N) return;
-    BaselineTerms<FP, false> t;
-    t.init(A, p, q);
-    if (t.uv_len < A.uv_min || t.uv_len > A.uv_max) return;
-    const int bl = q * (N - 1) - (q - 1) * q / 2 + p - q - 1;
-    double sum[NR];
-#pragma unroll
-    for (int r = 0; r < NR; ++r) sum[r] = 0.0;
-    for (int k = 0; k < A.num_splits; ++k)
+    const int at = threadIdx.x % VALUES, group = threadIdx.x / VALUES;
+    const int e = blockIdx.x * VALUES + at;
+    const int count = (N - 1 - q) * NR;
+    if ((int) blockIdx.x * VALUES >= count) return;
+    const size_t first = (size_t) baseline_index(N, q + 1, q) * NR;
+    double sum = 0.0;
+    if (e < count)
     {
-        const double* w = A.partial + ((size_t) k * nb + bl) * NR;
-#pragma unroll
-        for (int r = 0; r < NR; ++r) sum[r] += w[r];
+        const int per = (A.num_splits + GROUPS - 1) / GROUPS;
+        const int k1 = min(A.num_splits, (group + 1) * per);
+        const double* w = A.partial + first + e;
+#pragma unroll 4
+        for (int k = group * per; k < k1; ++k) sum += w[k * nb * NR];
     }
-    FP* v = (FP*) A.vis + (size_t) (A.offset_out + bl) * NR;
+    if (GROUPS > 1)
+    {
+        if (group > 0) sums[group - 1][at] = sum;
+        __syncthreads();
+        if (group > 0) return;
 #pragma unroll
-    for (int r = 0; r < NR; ++r) v[r] += (FP) sum[r];
+        for (int g = 0; g < GROUPS - 1; ++g) sum += sums[g][at];
+    }
+    if (e >= count) return;
+    BaselineTerms<FP, false> t;
+    t.init(A, q + 1 + e / NR, q);
+    if (t.uv_len < A.uv_min || t.uv_len > A.uv_max) return;
+    FP* v = (FP*) A.vis + (size_t) A.offset_out * NR + first + e;
+    *v += (FP) sum;
 }
 
 /* FP64 workspace for the split partial sums, one per (device, stream),
@@ -411,40 +544,31 @@ hipError_t scratch_address(double** out)
     return hipSuccess;
 }
 
-/* fixed: the device's scratch array (allocation-free entry point), whose
- * capacity caps the split count; NULL: the per-stream workspace. */
+/* fixed: the device's scratch array (allocation-free entry point); NULL:
+ * the per-stream workspace. */
 template <typename FP, bool MATRIX, bool GAUSS, bool BS, bool TS>
 hipError_t launch_t(XcorrArgs<FP> A, hipStream_t stream, double* fixed)
 {
     using G = Geometry<FP, MATRIX>;
     const int N = A.num_stations;
     const int na = (N + BLOCK_A - 1) / BLOCK_A;
-    const int nbk = (N + BLOCK_B - 1) / BLOCK_B;
-    /* Count the blocks that do work, then split the sources so the launch
-     * holds about 2048 working workgroups (8 per CU) with at least 4 tiles
-     * of sources each. */
-    int valid = 0;
+    int blocks = 0, ib0 = 0;
     for (int ia = 0; ia < na; ++ia)
-        for (int ib = 0; ib < nbk; ++ib)
-        {
-            const int a0 = ia * BLOCK_A, b0 = ib * BLOCK_B;
-            const int a_last = min(a0 + BLOCK_A, N) - 1;
-            const int b_last = min(b0 + BLOCK_B, N) - 1;
-            if (A.use_casa ? (a0 < b_last) : (a_last > b0)) ++valid;
-        }
-    if (valid == 0 || A.num_sources <= 0) return hipSuccess;
-    const int min_per_split = 4 * G::TILE;
-    int splits = (2048 + valid - 1) / valid;
-    const int max_splits = max(1, A.num_sources / min_per_split);
+        blocks += blocks_in_row(N, A.use_casa != 0, ia, &ib0);
+    if (blocks == 0 || A.num_sources <= 0) return hipSuccess;
+    /* Splits: about 12 rounds of four workgroups per CU, so that the last
+     * round's idle time is small, with at least 8 tiles of sources each
+     * (the prologue and the partial sums cost about one), or one where that
+     * leaves the chip idle (30 stations x 277 sources: 36 workgroups of one
+     * tile instead of 8 of four). */
+    int splits = (12 * 1024 + blocks - 1) / blocks;
+    const int max_splits = max(1, max(A.num_sources / (8 * G::TILE),
+            min((A.num_sources + G::TILE - 1) / G::TILE, 1024 / blocks)));
     splits = max(1, min(splits, min(max_splits, 256)));
     const size_t nb = (size_t) N * (N - 1) / 2;
-    if (fixed)
-    {
-        /* As many splits as the scratch array holds (one split writes vis
-         * directly and needs none). */
-        const size_t cap = XCORR_SCRATCH_BYTES / (nb * G::NR * sizeof(double));
-        splits = max(1, (int) min((size_t) splits, cap));
-    }
+    /* One split writes vis directly and needs no partial sums. */
+    splits = max(1, (int) min((size_t) splits,
+            XCORR_PARTIAL_BYTES / (nb * G::NR * sizeof(double))));
     int per = (A.num_sources + splits - 1) / splits;
     per = ((per + G::TILE - 1) / G::TILE) * G::TILE;
     splits = (A.num_sources + per - 1) / per;
@@ -459,14 +583,20 @@ hipError_t launch_t(XcorrArgs<FP> A, hipStream_t stream, double* fixed)
                 (size_t) splits * nb * G::NR * sizeof(double), stream, &err);
         if (err != hipSuccess) return err;
     }
-    dim3 grid(na, nbk, splits);
     hipLaunchKernelGGL((xcorr_direct_kernel<FP, MATRIX, GAUSS, BS, TS>),
-            grid, dim3(THREADS), 0, stream, A);
+            dim3((unsigned) blocks * (unsigned) splits), dim3(THREADS), 0,
+            stream, A, blocks);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess || splits == 1) return err;
-    hipLaunchKernelGGL((xcorr_reduce_kernel<FP, G::NR>),
-            dim3((unsigned) ((N + 255) / 256), (unsigned) (N - 1)), dim3(256),
-            0, stream, A);
+    const int reals = (N - 1) * G::NR;
+    if (splits >= 16)
+        hipLaunchKernelGGL((xcorr_reduce_kernel<FP, G::NR, 4>),
+                dim3((unsigned) ((reals + 63) / 64), (unsigned) (N - 1)),
+                dim3(256), 0, stream, A);
+    else
+        hipLaunchKernelGGL((xcorr_reduce_kernel<FP, G::NR, 1>),
+                dim3((unsigned) ((reals + 255) / 256), (unsigned) (N - 1)),
+                dim3(256), 0, stream, A);
     return hipGetLastError();
 }
 
@@ -476,8 +606,7 @@ hipError_t dispatch(const XcorrArgs<FP>& A, bool gauss, bool bs, bool ts,
 {
     /* No factor depends on the baseline: one matrix product. */
     if (!gauss && !bs && !ts)
-        return xcorr_product_launch<FP, MATRIX>(A, s, fixed,
-                XCORR_SCRATCH_BYTES);
+        return xcorr_product_launch<FP, MATRIX>(A, s, fixed);
 #define XC_CASE(G_, B_, T_) if (gauss == G_ && bs == B_ && ts == T_) \
         return launch_t<FP, MATRIX, G_, B_, T_>(A, s, fixed);
     XC_CASE(false, false, true)  XC_CASE(false, true, false)

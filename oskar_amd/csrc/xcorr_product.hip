@@ -676,7 +676,7 @@ namespace oskar_amd {
 
 template <typename FP, bool MATRIX>
 hipError_t xcorr_product_launch(XcorrArgs<FP> A, hipStream_t stream,
-        double* fixed, size_t fixed_bytes)
+        double* fixed)
 {
     using G = Geo<FP, MATRIX>;
     if (A.num_stations < 2 || A.num_sources <= 0) return hipSuccess;
@@ -687,13 +687,12 @@ hipError_t xcorr_product_launch(XcorrArgs<FP> A, hipStream_t stream,
      * (4096 matrix-core cycles, 1.75 us), k splits cost about stages / k for
      * the last workgroups to finish alone, and 0.026 k tiles for filling
      * each workgroup's pipeline (two stages on one of 256 CUs) and for its
-     * 64 KB of partial sums written and read at 4 TB/s.  The partial sums
-     * stay within 256 MB (the Infinity Cache).  197 stations x 30011
+     * 64 KB of partial sums written and read at 4 TB/s.  197 stations x 30011
      * sources in FP64: 71 splits against one round of 18. */
     const size_t split_bytes = (size_t) tiles * 4 * WAVE_VALUES *
             sizeof(double);
-    const size_t cap = fixed ? fixed_bytes : (size_t) 256 << 20;
-    const int most = max(1, (int) min((size_t) stages, cap / split_bytes));
+    const int most = max(1, (int) min((size_t) stages,
+            XCORR_PARTIAL_BYTES / split_bytes));
     int splits = (int) sqrt(stages / (0.026 * tiles));
     splits = max(1, min(splits, most));
     const int per = (stages + splits - 1) / splits;
@@ -724,12 +723,12 @@ hipError_t xcorr_product_launch(XcorrArgs<FP> A, hipStream_t stream,
 }
 
 template hipError_t xcorr_product_launch<double, true>(XcorrArgs<double>,
-        hipStream_t, double*, size_t);
+        hipStream_t, double*);
 template hipError_t xcorr_product_launch<double, false>(XcorrArgs<double>,
-        hipStream_t, double*, size_t);
+        hipStream_t, double*);
 template hipError_t xcorr_product_launch<float, true>(XcorrArgs<float>,
-        hipStream_t, double*, size_t);
+        hipStream_t, double*);
 template hipError_t xcorr_product_launch<float, false>(XcorrArgs<float>,
-        hipStream_t, double*, size_t);
+        hipStream_t, double*);
 
 } /* namespace oskar_amd */
