@@ -180,24 +180,20 @@ __global__ void dipole_kernel(int n, const FP* theta, const FP* phi_x,
     }
 }
 
-/* theta_phi_kernel and dipole_kernel in one pass, theta and phi kept in
- * registers: the pattern of directions [off_in, off_in + num), then, with
- * extra_point_at_pole, the pole (theta 0, phi = the deltas) at index num. */
+/* The pattern of directions [off_in, off_in + num) straight from their
+ * coordinates, then, with extra_point_at_pole, of the pole at index num. */
 template <typename FP, bool MATRIX>
 __global__ void dipole_enu_kernel(int off_in, int num, const FP* x,
-        const FP* y, const FP* z, int extra_point_at_pole, FP delta_phi1,
-        FP delta_phi2, FP kL, FP cos_kL, int swap_xy, int offset_out,
-        Cplx<FP>* pattern)
+        const FP* y, const FP* z, int extra_point_at_pole,
+        DipoleParams<FP> P, int offset_out, Cplx<FP>* pattern)
 {
     const size_t total = (size_t) num + (extra_point_at_pole ? 1 : 0);
     GRID_STRIDE(i, total)
     {
-        FP theta = (FP) 0, p1 = delta_phi1, p2 = delta_phi2;
-        if (i < (size_t) num)
-            theta_phi_point<FP>(x[i + off_in], y[i + off_in], z[i + off_in],
-                    delta_phi1, delta_phi2, &theta, &p1, &p2);
-        dipole_point<FP, MATRIX>(theta, p1, p2, kL, cos_kL, swap_xy,
-                pattern, i + offset_out);
+        const bool pole = i >= (size_t) num;
+        dipole_enu_point<FP, MATRIX>(pole ? (FP) 0 : x[i + off_in],
+                pole ? (FP) 0 : y[i + off_in], pole ? (FP) 1 : z[i + off_in],
+                P, pattern, i + offset_out);
     }
 }
 
@@ -549,9 +545,10 @@ extern "C" int oskar_amd_dipole_enu_launch(int precision, int matrix,
     const hipStream_t s = (hipStream_t) stream;
 #define DE(FP, M) hipLaunchKernelGGL((dipole_enu_kernel<FP, M>), \
         grid_for(total), dim3(THREADS), 0, s, offset_in, num, (const FP*) x, \
-        (const FP*) y, (const FP*) z, extra_point_at_pole, (FP) delta_phi1, \
-        (FP) delta_phi2, (FP) kL, (FP) cos_kL, swap_xy, offset_out, \
-        (Cplx<FP>*) pattern)
+        (const FP*) y, (const FP*) z, extra_point_at_pole, \
+        (DipoleParams<FP>{(FP) (kL * 0.15915494309189535), (FP) cos_kL, (FP) cos(delta_phi1), \
+        (FP) sin(delta_phi1), (FP) cos(delta_phi2), (FP) sin(delta_phi2), \
+        swap_xy}), offset_out, (Cplx<FP>*) pattern)
     if (precision == OSKAR_DOUBLE)
     {
         if (matrix) DE(double, true);

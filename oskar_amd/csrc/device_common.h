@@ -130,6 +130,95 @@ template <> struct Sinc<double>
     }
 };
 
+/* sin and cos of 2 pi t: t reduced exactly to [-1/2, 1/2], folded to
+ * g in [-1/4, 1/4] (the cosine changes sign), then polynomials in g^2 that
+ * interpolate sin(2 pi g) / g and cos(2 pi g) at Chebyshev nodes (formed in
+ * extended precision).  Largest and RMS error over 5e5 random arguments:
+ * 2.7e-16 and 5.5e-17 (sine), 2.2e-16 and 4.9e-17 (cosine); 29 instructions
+ * where the library's sincos took about 100. */
+__device__ __forceinline__ void sincos_rev(double t, double* s, double* c)
+{
+    const double r = t - rint(t);
+    const bool far = fabs(r) > 0.25;
+    const double g = far ? copysign(0.5, r) - r : r;
+    const double y = g * g;
+    double ps = 0.10087905121711918;
+    ps = fma(ps, y, -0.7177290771684038);
+    ps = fma(ps, y, 3.8199275897803275);
+    ps = fma(ps, y, -15.094641648143382);
+    ps = fma(ps, y, 42.05869392458247);
+    ps = fma(ps, y, -76.70585975281163);
+    ps = fma(ps, y, 81.60524927607352);
+    ps = fma(ps, y, -41.341702240399755);
+    ps = fma(ps, y, 6.283185307179586);
+    double pc = 0.2730462895403127;
+    pc = fma(pc, y, -1.7134850372266826);
+    pc = fma(pc, y, 7.903488575512233);
+    pc = fma(pc, y, -26.426255384546224);
+    pc = fma(pc, y, 60.24464134963378);
+    pc = fma(pc, y, -85.45681720652);
+    pc = fma(pc, y, 64.93939402266777);
+    pc = fma(pc, y, -19.739208802178716);
+    pc = fma(pc, y, 1.0);
+    *s = ps * g;
+    *c = far ? -pc : pc;
+}
+
+/* cos(2 pi t) likewise. */
+__device__ __forceinline__ double cos_rev(double t)
+{
+    double s, c;
+    sincos_rev(t, &s, &c);
+    return c;
+}
+/* FP32: largest and RMS error 1.3e-7 and 2.9e-8 (12 instructions). */
+__device__ __forceinline__ float cos_rev(float t)
+{
+    const float r = t - rintf(t);
+    const bool far = fabsf(r) > 0.25f;
+    const float g = far ? 0.5f - fabsf(r) : r;
+    const float y = g * g;
+    float p = -2.521816254e+1f;
+    p = fmaf(p, y, 6.017903900e+1f);
+    p = fmaf(p, y, -8.545536041e+1f);
+    p = fmaf(p, y, 6.493938446e+1f);
+    p = fmaf(p, y, -1.973920822e+1f);
+    p = fmaf(p, y, 1.0f);
+    return far ? -p : p;
+}
+
+/* 1 / sqrt(x) for normal x: the hardware estimate (1 ulp in FP32, about
+ * 2^-26 in FP64) and Newton steps. */
+__device__ __forceinline__ float inv_sqrt(float x)
+{
+    const float y = __builtin_amdgcn_rsqf(x);
+    return fmaf(0.5f * y, fmaf(-x * y, y, 1.0f), y);
+}
+__device__ __forceinline__ double inv_sqrt(double x)
+{
+    double y = __builtin_amdgcn_rsq(x);
+    y = fma(0.5 * y, fma(-x * y, y, 1.0), y);
+    return fma(0.5 * y, fma(-x * y, y, 1.0), y);
+}
+
+/* a / b for a normal b: the reciprocal's estimate and a Newton step (two in
+ * FP64), then the quotient's remainder. */
+__device__ __forceinline__ float quotient(float a, float b)
+{
+    float r = __builtin_amdgcn_rcpf(b);
+    r = fmaf(fmaf(-b, r, 1.0f), r, r);
+    const float q = a * r;
+    return fmaf(fmaf(-b, q, a), r, q);
+}
+__device__ __forceinline__ double quotient(double a, double b)
+{
+    double r = __builtin_amdgcn_rcp(b);
+    r = fma(fma(-b, r, 1.0), r, r);
+    r = fma(fma(-b, r, 1.0), r, r);
+    const double q = a * r;
+    return fma(fma(-b, q, a), r, q);
+}
+
 template <typename FP> __device__ __forceinline__ void sincos_v(FP x,
         FP* s, FP* c);
 template <> __device__ __forceinline__ void sincos_v<float>(float x,

@@ -25,7 +25,8 @@
  *    times 1/(2 pi) folded into the direction once per thread), reduces it
  *    to [-1/2, 1/2] and uses the hardware sine and cosine, which take
  *    revolutions; each term is four fused multiply-adds into the array
- *    factor.  Double precision uses radians and the full-accuracy sincos.
+ *    factor.  Double precision reduces the phase to a quarter revolution and
+ *    uses polynomials.
  */
 #include <hip/hip_runtime.h>
 #include <type_traits>
@@ -41,19 +42,17 @@ namespace {
 constexpr int THREADS = 256;
 constexpr int CHUNK = 256;
 
-/* exp(i t) of the phase in the unit the kernel carries it in: FP32 phases
- * are in revolutions for the hardware sine and cosine (which take
- * revolutions), reduced to [-1/2, 1/2] first unless DIRECT; FP64 phases
- * are in radians, with the full-accuracy sincos.  The hardware reduces a
- * phase of up to 256 revolutions exactly (the same errors against the FP64
- * DFT with and without the reduction at up to 250 revolutions, measured),
- * so DIRECT serves when |t| is bounded below that: two fewer instructions
- * per term. */
+/* exp(i 2 pi t) of a phase in revolutions.  FP32: the hardware sine and
+ * cosine, which take revolutions, of the phase reduced to [-1/2, 1/2]
+ * unless DIRECT: the hardware reduces a phase of up to 256 revolutions
+ * exactly (the same errors against the FP64 DFT with and without the
+ * reduction at up to 250 revolutions, measured), so DIRECT serves when |t|
+ * is bounded below that: two fewer instructions per term. */
 template <bool DIRECT, typename FP>
 __device__ __forceinline__ void phase_sincos(FP t, FP* s, FP* c)
 {
     if constexpr (sizeof(FP) == 8)
-        sincos(t, s, c);
+        sincos_rev(t, s, c);
     else
     {
         const float r = DIRECT ? t : t - __builtin_rintf(t);
@@ -62,12 +61,8 @@ __device__ __forceinline__ void phase_sincos(FP t, FP* s, FP* c)
     }
 }
 
-/* Factor from k (x_out x_in + ...) to the kernel's phase unit. */
-template <typename FP> __device__ __forceinline__ FP phase_unit();
-template <> __device__ __forceinline__ float phase_unit<float>()
-{ return 0.159154943091895336f; }           /* 1 / (2 pi) */
-template <> __device__ __forceinline__ double phase_unit<double>()
-{ return 1.0; }
+/* Factor from k (x_out x_in + ...) to revolutions, 1 / (2 pi). */
+constexpr double PHASE_UNIT = 0.15915494309189535;
 
 /* One element of the chunk staged in LDS: position and weight. */
 template <typename FP> struct Elem
@@ -189,7 +184,7 @@ void dftw_kernel(const int num_in, const FP wavenumber,
     FP xo = (FP) 0, yo = (FP) 0, zo = (FP) 0;
     if (active)
     {
-        const FP kk = wavenumber * phase_unit<FP>();
+        const FP kk = wavenumber * (FP) PHASE_UNIT;
         xo = kk * x_out[i_out + offset_coord_out];
         yo = kk * y_out[i_out + offset_coord_out];
         if (IS_3D) zo = kk * z_out[i_out + offset_coord_out];
@@ -320,120 +315,159 @@ void dftw_kernel(const int num_in, const FP wavenumber,
     }
 }
 
-/* The beam of a flat aperture-array station whose elements are all of one
- * dipole type with a common orientation, in one pass per direction: the
- * array factor (dftw_kernel's sum, in its order), times the direction's
- * dipole pattern (computed here with the pattern kernels' device
- * functions instead of read from a stored pattern), times norm_factor,
- * zero below the horizon (blank_kernel's rule).  With NORM the result is
- * divided as oskar_mem_normalise divides by the beam in the normalisation
- * direction (nx, ny, nz), which every workgroup forms itself: each thread
- * sums the array factor over a stride of the elements, a fixed-order tree
- * in LDS adds the 256 partial sums (so every workgroup gets the same
- * value), and thread 0 applies the pattern, the blank and the scale rule.
- * Only the order of that one sum differs from the separate kernels. */
-template <typename FP, bool MATRIX, bool IS_3D, bool NORM>
+/* An element of an aperture-array beam in LDS: position, and the weight as
+ * amplitude and phase in revolutions. */
+template <typename FP, bool IS_3D> struct AaElem;
+template <typename FP> struct alignas(4 * sizeof(FP)) AaElem<FP, false>
+{
+    FP x, y, phase, amp;
+    __device__ __forceinline__ FP at(FP xo, FP yo, FP) const
+    {
+        return fma(yo, y, fma(xo, x, phase));
+    }
+};
+template <typename FP> struct alignas(4 * sizeof(FP)) AaElem<FP, true>
+{
+    FP x, y, phase, amp, z, pad[3];
+    __device__ __forceinline__ FP at(FP xo, FP yo, FP zo) const
+    {
+        return fma(zo, z, fma(yo, y, fma(xo, x, phase)));
+    }
+};
+
+struct AaGroup { oskar_AaStation st[OSKAR_AA_GROUP]; };
+
+/* Beams of flat aperture-array stations whose elements are all of one
+ * dipole type with a common orientation, in one pass per direction:
+ * blockIdx.y = station of the group, D directions per thread (an element
+ * read from LDS serves them all).  The array factor (dftw_kernel's sum, in
+ * its order), times the direction's dipole pattern, times norm_factor, zero
+ * below the horizon (blank_kernel's rule).  DFT weights without errors are
+ * formed here, in FP64, from the measured positions and the pointing, once
+ * per workgroup; others are read.  With NORM the result is divided as
+ * oskar_mem_normalise divides by the beam in the normalisation direction,
+ * whose pattern the host gives (norm_power) and whose array factor every
+ * workgroup forms itself, each thread a stride of the elements, added in a
+ * fixed order, so every workgroup of a station gets the same value.
+ *
+ * Bound: vector instructions: 4 and a hardware sine and cosine (FP32) or
+ * 34 (FP64) per element and direction, and about 150 per direction for the
+ * pattern and the output.  60 stations of 96 dipoles x 16,385 directions in
+ * FP64: 1.8 ms as 60 launches of 65 workgroups with library sincos and
+ * angles, 0.14 ms as 4 launches.  One station of 256 dipoles x 1M
+ * directions in FP32: 78.3 -> 68.9 us (vector unit and transcendentals 80 %
+ * of the time). */
+template <typename FP, bool MATRIX, bool IS_3D, bool NORM, int D>
 __global__ __launch_bounds__(THREADS)
-void aa_fused_kernel(const int num_in, const FP wavenumber,
-        const Cplx<FP>* __restrict__ weights, const FP* __restrict__ x_in,
-        const FP* __restrict__ y_in, const FP* __restrict__ z_in,
-        const int num_out, const FP* __restrict__ x_out,
-        const FP* __restrict__ y_out, const FP* __restrict__ z_out,
-        const FP nx, const FP ny, const FP nz, const FP kL, const FP cos_kL,
-        const FP dphi_x, const FP dphi_y, const int swap_xy,
-        const FP norm_factor, Cplx<FP>* __restrict__ output)
+void aa_beam_kernel(AaGroup G, const double wavenumber, const int num_out,
+        const FP* __restrict__ x_out, const FP* __restrict__ y_out,
+        const FP* __restrict__ z_out, Cplx<FP>* __restrict__ output)
 {
     constexpr int NC = MATRIX ? 4 : 1;
-    __shared__ Elem<FP> c_e[CHUNK];
-    __shared__ Cplx<FP> red[THREADS];
-    __shared__ FP s_scal;
+    using E = AaElem<FP, IS_3D>;
+    __shared__ E c_e[CHUNK];
+    __shared__ FP red[2][THREADS / 64];
     __shared__ unsigned int c_ext;
+    static_assert(D == 1 || D == 2, "directions per thread");
+    const oskar_AaStation& S = G.st[blockIdx.y];
     const int tid = (int) threadIdx.x;
-    const FP kk = wavenumber * phase_unit<FP>();
+    const int num_in = S.num_elements;
+    const double rev = wavenumber * PHASE_UNIT;
+    const FP kk = (FP) rev;
 
-    /* The array factor plus w exp(i t) of one element, as in dftw_kernel
-     * (w in term_weight's form). */
-    auto add_term = [](Cplx<FP>& af, FP t, const Cplx<FP>& w, auto direct) {
-        FP s, c;
-        phase_sincos<decltype(direct)::value, FP>(t, &s, &c);
-        term_add<FP>(af, w, s, c);
-    };
-    /* The beam of one direction from its array factor: pattern x af,
-     * scaled, blanked (dftw_kernel's flush and output, blank_kernel). */
-    auto beam_of = [&](FP x, FP y, FP z, const Cplx<FP>& af, FP* v) {
-        Cplx<FP> d[NC];
-        FP theta, p1, p2;
-        theta_phi_point<FP>(x, y, z, dphi_x, dphi_y, &theta, &p1, &p2);
-        dipole_point<FP, MATRIX>(theta, p1, p2, kL, cos_kL, swap_xy, d, 0);
-#pragma unroll
-        for (int k = 0; k < NC; ++k)
+    auto element = [&](int g) {
+        E e;
+        e.x = ((const FP*) S.x)[g];
+        e.y = ((const FP*) S.y)[g];
+        if constexpr (IS_3D) e.z = ((const FP*) S.z)[g];
+        if (S.weights)
         {
-            Cplx<FP> o;
-            o.x = o.y = (FP) 0;
-            o.x += d[k].x * af.x - d[k].y * af.y;
-            o.y += d[k].y * af.x + d[k].x * af.y;
-            v[2 * k] = z < (FP) 0 ? (FP) 0 : o.x * norm_factor;
-            v[2 * k + 1] = z < (FP) 0 ? (FP) 0 : o.y * norm_factor;
+            const Cplx<FP> w = ((const Cplx<FP>*) S.weights)[g];
+            e.amp = sqrt(w.x * w.x + w.y * w.y);
+            e.phase = atan2(w.y, w.x) * (FP) PHASE_UNIT;
         }
+        else
+        {
+            double p = (double) ((const FP*) S.mx)[g] * S.beam_x +
+                    (double) ((const FP*) S.my)[g] * S.beam_y +
+                    (double) ((const FP*) S.mz)[g] * S.beam_z;
+            if (S.cable) p += (double) ((const FP*) S.cable)[g];
+            p *= -rev;
+            e.amp = (FP) 1;
+            e.phase = (FP) (p - rint(p));
+        }
+        return e;
     };
 
     FP scal = (FP) 1;
     if constexpr (NORM)
     {
-        const FP xn = kk * nx, yn = kk * ny;
-        const FP zn = IS_3D ? kk * nz : (FP) 0;
-        Cplx<FP> a;
-        a.x = a.y = (FP) 0;
-        for (int e = tid; e < num_in; e += THREADS)
+        const FP xn = kk * (FP) S.nx, yn = kk * (FP) S.ny;
+        const FP zn = kk * (FP) S.nz;
+        FP re = (FP) 0, im = (FP) 0;
+        for (int g = tid; g < num_in; g += THREADS)
         {
-            const Cplx<FP> w = term_weight<FP>(weights[e]);
-            const FP t = term_phase<FP, IS_3D>(xn, yn, zn, x_in[e], y_in[e],
-                    IS_3D ? z_in[e] : (FP) 0, w);
-            add_term(a, t, w, std::false_type());
+            const E e = element(g);
+            FP s, c;
+            phase_sincos<false, FP>(e.at(xn, yn, zn), &s, &c);
+            re = fma(e.amp, c, re);
+            im = fma(e.amp, s, im);
         }
-        red[tid] = a;
-        __syncthreads();
-        for (int o = THREADS / 2; o > 0; o >>= 1)
-        {
-            if (tid < o)
-            {
-                red[tid].x += red[tid + o].x;
-                red[tid].y += red[tid + o].y;
-            }
-            __syncthreads();
-        }
-        if (tid == 0)
-        {
-            FP v[2 * NC];
-            beam_of(nx, ny, nz, red[0], v);
-            FP amp = (FP) 0;
 #pragma unroll
-            for (int r = 0; r < 2 * NC; ++r) amp += v[r] * v[r];
-            if (MATRIX) amp /= (FP) 2;
-            s_scal = (FP) 1 / sqrt(amp);
+        for (int o = 32; o > 0; o >>= 1)
+        {
+            re += __shfl_xor(re, o);
+            im += __shfl_xor(im, o);
+        }
+        if ((tid & 63) == 0)
+        {
+            red[0][tid >> 6] = re;
+            red[1][tid >> 6] = im;
         }
         __syncthreads();
-        scal = s_scal;
+        re = (red[0][0] + red[0][1]) + (red[0][2] + red[0][3]);
+        im = (red[1][0] + red[1][1]) + (red[1][2] + red[1][3]);
+        const FP f = (FP) S.norm_factor;
+        const FP amp = (re * re + im * im) * (f * f) * (FP) S.norm_power;
+        scal = (FP) 1 / sqrt(amp);
     }
 
-    const int i_out = blockIdx.x * THREADS + tid;
-    const bool active = i_out < num_out;
-    FP xd = (FP) 0, yd = (FP) 0, zd = (FP) 0;
-    if (active)
+    FP xo[D], yo[D], zo[D];
+    Cplx<FP> af[D];
+    const int first = (int) blockIdx.x * (THREADS * D) + tid;
+#pragma unroll
+    for (int d = 0; d < D; ++d)
     {
-        xd = x_out[i_out];
-        yd = y_out[i_out];
-        zd = z_out[i_out];
+        const int i = min(first + d * THREADS, num_out - 1);
+        xo[d] = kk * x_out[i];
+        yo[d] = kk * y_out[i];
+        zo[d] = IS_3D ? kk * z_out[i] : (FP) 0;
+        af[d].x = af[d].y = (FP) 0;
     }
-    const FP xo = kk * xd, yo = kk * yd, zo = IS_3D ? kk * zd : (FP) 0;
-    Cplx<FP> af;
-    af.x = af.y = (FP) 0;
-    auto term = [&](const Elem<FP>& e, auto direct) {
-        add_term(af, term_phase<FP, IS_3D>(xo, yo, zo, e.x, e.y, e.z, e.w),
-                e.w, direct);
+    /* Directions d0 .. d1 - 1 of the thread over the staged elements. */
+    auto sum = [&](int chunk, auto direct, auto d0, auto d1) {
+        auto term = [&](const E& e) {
+#pragma unroll
+            for (int d = decltype(d0)::value; d < decltype(d1)::value; ++d)
+            {
+                FP s, c;
+                phase_sincos<decltype(direct)::value, FP>(
+                        e.at(xo[d], yo[d], zo[d]), &s, &c);
+                af[d].x = fma(e.amp, c, af[d].x);
+                af[d].y = fma(e.amp, s, af[d].y);
+            }
+        };
+        int i = 0;
+        for (; i + 4 <= chunk; i += 4)
+        {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) term(c_e[i + u]);
+        }
+        for (; i < chunk; ++i) term(c_e[i]);
     };
-    const std::true_type direct_t;
-    const std::false_type reduce_t;
+    const std::integral_constant<int, 0> d_0;
+    const std::integral_constant<int, 1> d_1;
+    const std::integral_constant<int, D> d_all;
     for (int j = 0; j < num_in; j += CHUNK)
     {
         const int chunk = min(CHUNK, num_in - j);
@@ -442,77 +476,84 @@ void aa_fused_kernel(const int num_in, const FP wavenumber,
         __syncthreads();
         for (int t = tid; t < chunk; t += THREADS)
         {
-            const int g = j + t;
-            Elem<FP> e;
-            e.x = x_in[g];
-            e.y = y_in[g];
-            e.z = IS_3D ? z_in[g] : (FP) 0;
-            e.pad = (FP) 0;
-            e.w = term_weight<FP>(weights[g]);
+            const E e = element(j + t);
             c_e[t] = e;
-            chunk_extent<FP>(&c_ext, e);
+            if constexpr (sizeof(FP) == 4)
+            {
+                FP a = fmaxf(fabsf(e.x), fabsf(e.y));
+                if constexpr (IS_3D) a = fmaxf(a, fabsf(e.z));
+                atomicMax(&c_ext, __float_as_uint(a));
+            }
         }
         __syncthreads();
-        int i = 0;
-        if (direct_phase<FP>(xo, yo, zo, c_ext))
-        {
-            for (; i + 4 <= chunk; i += 4)
-            {
+        /* Whether a direction's phases need the reduction depends on that
+         * direction only, so that its value does not depend on D. */
+        bool direct[D];
 #pragma unroll
-                for (int u = 0; u < 4; ++u) term(c_e[i + u], direct_t);
-            }
-            for (; i < chunk; ++i) term(c_e[i], direct_t);
+        for (int d = 0; d < D; ++d)
+            direct[d] = direct_phase<FP>(xo[d], yo[d], zo[d], c_ext);
+        if (direct[0] && direct[D - 1])
+            sum(chunk, std::true_type(), d_0, d_all);
+        else if (!direct[0] && !direct[D - 1])
+            sum(chunk, std::false_type(), d_0, d_all);
+        else if (direct[0])
+        {
+            sum(chunk, std::true_type(), d_0, d_1);
+            sum(chunk, std::false_type(), d_1, d_all);
         }
         else
         {
-            for (; i + 4 <= chunk; i += 4)
-            {
-#pragma unroll
-                for (int u = 0; u < 4; ++u) term(c_e[i + u], reduce_t);
-            }
-            for (; i < chunk; ++i) term(c_e[i], reduce_t);
+            sum(chunk, std::false_type(), d_0, d_1);
+            sum(chunk, std::true_type(), d_1, d_all);
         }
     }
-    if (!active) return;
-    FP v[2 * NC];
-    beam_of(xd, yd, zd, af, v);
-    Cplx<FP>* o = output + (size_t) i_out * NC;
+    const DipoleParams<FP> P = {(FP) (S.kL * PHASE_UNIT), (FP) S.cos_kL, (FP) S.cos_dx,
+            (FP) S.sin_dx, (FP) S.cos_dy, (FP) S.sin_dy, S.swap_xy};
 #pragma unroll
-    for (int k = 0; k < NC; ++k)
+    for (int d = 0; d < D; ++d)
     {
-        Cplx<FP> r;
-        r.x = v[2 * k];
-        r.y = v[2 * k + 1];
-        if constexpr (NORM)
+        const int i = first + d * THREADS;
+        if (i >= num_out) break;
+        const FP z = z_out[i];
+        Cplx<FP> e[NC];
+        dipole_enu_point<FP, MATRIX>(x_out[i], y_out[i], z, P, e, 0);
+        const FP f = (FP) S.norm_factor;
+        Cplx<FP>* o = output + (S.offset + (size_t) i) * NC;
+#pragma unroll
+        for (int k = 0; k < NC; ++k)
         {
-            r.x = r.x * scal;
-            r.y = r.y * scal;
+            Cplx<FP> v;
+            v.x = z < (FP) 0 ? (FP) 0 : e[k].x * af[d].x * f;
+            v.y = z < (FP) 0 ? (FP) 0 : e[k].x * af[d].y * f;
+            if constexpr (NORM)
+            {
+                v.x *= scal;
+                v.y *= scal;
+            }
+            o[k] = v;
         }
-        o[k] = r;
     }
 }
 
-template <typename FP, bool MATRIX, bool IS_3D>
-hipError_t aa_fused_t(int normalise, int num_in, double wavenumber,
-        const void* weights, const void* x_in, const void* y_in,
-        const void* z_in, int num_out, const void* x_out, const void* y_out,
-        const void* z_out, double nx, double ny, double nz, double kL,
-        double cos_kL, double dphi_x, double dphi_y, int swap_xy,
-        double norm_factor, void* output, hipStream_t stream)
+template <typename FP, bool MATRIX, bool IS_3D, bool NORM>
+hipError_t aa_beam_t(const AaGroup& G, int count, double wavenumber,
+        int num_out, const void* x_out, const void* y_out,
+        const void* z_out, void* output, hipStream_t stream)
 {
-    const dim3 grid((num_out + THREADS - 1) / THREADS);
-#define AF_ARGS num_in, (FP) wavenumber, (const Cplx<FP>*) weights,       \
-        (const FP*) x_in, (const FP*) y_in, (const FP*) z_in, num_out,      \
-        (const FP*) x_out, (const FP*) y_out, (const FP*) z_out, (FP) nx,   \
-        (FP) ny, (FP) nz, (FP) kL, (FP) cos_kL, (FP) dphi_x, (FP) dphi_y,   \
-        swap_xy, (FP) norm_factor, (Cplx<FP>*) output
-    if (normalise)
-        hipLaunchKernelGGL((aa_fused_kernel<FP, MATRIX, IS_3D, true>), grid,
-                dim3(THREADS), 0, stream, AF_ARGS);
-    else
-        hipLaunchKernelGGL((aa_fused_kernel<FP, MATRIX, IS_3D, false>), grid,
-                dim3(THREADS), 0, stream, AF_ARGS);
-#undef AF_ARGS
+    /* Two directions per thread where that still gives every CU four
+     * workgroups (an element's LDS reads and the workgroup's weights and
+     * normalisation serve both); one otherwise. */
+    const long long pairs = ((long long) num_out + 2 * THREADS - 1) /
+            (2 * THREADS);
+#define AA_LAUNCH(D) hipLaunchKernelGGL( \
+        (aa_beam_kernel<FP, MATRIX, IS_3D, NORM, D>), \
+        dim3((num_out + THREADS * D - 1) / (THREADS * D), count), \
+        dim3(THREADS), 0, stream, G, wavenumber, num_out, \
+        (const FP*) x_out, (const FP*) y_out, (const FP*) z_out, \
+        (Cplx<FP>*) output)
+    if (pairs * count >= 4 * 256) AA_LAUNCH(2);
+    else AA_LAUNCH(1);
+#undef AA_LAUNCH
     return hipGetLastError();
 }
 
@@ -570,28 +611,29 @@ extern "C" int oskar_amd_dftw_launch(int precision, int matrix, int is_3d,
             offset_out, output, norm_factor, (hipStream_t) stream);
 }
 
-extern "C" int oskar_amd_aa_fused_launch(int precision, int matrix,
-        int is_3d, int normalise, int num_in, double wavenumber,
-        const void* weights, const void* x_in, const void* y_in,
-        const void* z_in, int num_out, const void* x_out, const void* y_out,
-        const void* z_out, double nx, double ny, double nz, double kL,
-        double cos_kL, double dphi_x, double dphi_y, int swap_xy,
-        double norm_factor, void* output, void* stream)
+extern "C" int oskar_amd_aa_beam_launch(int precision, int matrix,
+        int is_3d, int normalise, const oskar_AaStation* stations, int count,
+        double wavenumber, int num_out, const void* x_out,
+        const void* y_out, const void* z_out, void* output, void* stream)
 {
-    if (num_out <= 0) return 0;
+    if (num_out <= 0 || count <= 0) return 0;
+    if (count > OSKAR_AA_GROUP) return (int) hipErrorInvalidValue;
     const hipStream_t s = (hipStream_t) stream;
-#define AF(FP, M, D) return (int) aa_fused_t<FP, M, D>(normalise, num_in, \
-        wavenumber, weights, x_in, y_in, z_in, num_out, x_out, y_out, z_out, \
-        nx, ny, nz, kL, cos_kL, dphi_x, dphi_y, swap_xy, norm_factor, output, \
-        s)
+    AaGroup G;
+    for (int i = 0; i < count; ++i) G.st[i] = stations[i];
+    for (int i = count; i < OSKAR_AA_GROUP; ++i) G.st[i] = stations[0];
+#define AB(FP, M, D, N) return (int) aa_beam_t<FP, M, D, N>(G, count, \
+        wavenumber, num_out, x_out, y_out, z_out, output, s)
+#define AF(FP, M, D) { if (normalise) AB(FP, M, D, true); AB(FP, M, D, false); }
     if (precision == OSKAR_DOUBLE)
     {
-        if (matrix) { if (is_3d) AF(double, true, true); AF(double, true, false); }
-        if (is_3d) AF(double, false, true);
-        AF(double, false, false);
+        if (matrix) { if (is_3d) AF(double, true, true) AF(double, true, false) }
+        if (is_3d) AF(double, false, true)
+        AF(double, false, false)
     }
-    if (matrix) { if (is_3d) AF(float, true, true); AF(float, true, false); }
-    if (is_3d) AF(float, false, true);
-    AF(float, false, false);
+    if (matrix) { if (is_3d) AF(float, true, true) AF(float, true, false) }
+    if (is_3d) AF(float, false, true)
+    AF(float, false, false)
 #undef AF
+#undef AB
 }

@@ -1,7 +1,7 @@
 /*
  * Device functions of the dipole element pattern, shared by the pattern
- * kernels (beam_util.hip) and the fused aperture-array beam (dftw.hip):
- * theta and phi of an ENU direction
+ * kernels (beam_util.hip) and the aperture-array beam (dftw.hip): theta and
+ * phi of an ENU direction
  * (oskar/convert/define_convert_enu_directions_to_theta_phi.h) and the
  * pattern of a pair of crossed dipoles
  * (oskar/telescope/station/element/define_evaluate_dipole_pattern.h).
@@ -82,6 +82,74 @@ __device__ __forceinline__ void dipole_point(FP theta, FP phi_x, FP phi_y,
                 y_th.x * y_th.x + y_ph.x * y_ph.x) / (FP) 2);
         pattern[o].x = amp;
         pattern[o].y = (FP) 0;
+    }
+}
+
+/* The dipole pattern of one ENU direction from its coordinates: the same
+ * as theta_phi_point then dipole_point, with the sines and cosines of theta
+ * and phi as quotients of the coordinates (phi = 0 or pi at the zenith, as
+ * atan2) and each feed's phi turned by its delta's sine and cosine.  What
+ * is left of the functions is the cosine of each dipole's projected length
+ * (the angles took two atan2, two fmod and three sincos per direction).
+ * kL_rev: kL / (2 pi). */
+template <typename FP> struct DipoleParams
+{
+    FP kL_rev, cos_kL, cos_dx, sin_dx, cos_dy, sin_dy;
+    int swap_xy;
+};
+
+template <typename FP, bool MATRIX>
+__device__ __forceinline__ void dipole_enu_point(FP x, FP y, FP z,
+        const DipoleParams<FP>& P, Cplx<FP>* pattern, size_t o)
+{
+    /* Directions next to the zenith, whose x^2 + y^2 would be lost, are
+     * scaled up for phi (theta is 0 there). */
+    constexpr FP TINY = sizeof(FP) == 4 ? (FP) 1e-30 : (FP) 1e-280;
+    constexpr FP UP = sizeof(FP) == 4 ? (FP) 0x1p60 : (FP) 0x1p500;
+    FP r2 = x * x + y * y;
+    const FP h2 = r2 + z * z;
+    const bool up = r2 < TINY;
+    const FP sx = up ? x * UP : x, sy = up ? y * UP : y;
+    r2 = sx * sx + sy * sy;
+    const bool zenith = !(r2 > (FP) 0);
+    const FP ir = inv_sqrt(r2), ih = inv_sqrt(h2);
+    const FP cos_theta = h2 > (FP) 0 ? z * ih : (FP) 1;
+    const FP sin_theta = up ? (FP) 0 : r2 * ir * ih;
+    const FP cos_phi = zenith ? copysign((FP) 1, x) : sx * ir;
+    const FP sin_phi = zenith ? (FP) 0 : sy * ir;
+    FP e[2][2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+    {
+        const FP cd = k ? P.cos_dy : P.cos_dx, sd = k ? P.sin_dy : P.sin_dx;
+        const FP c = cos_phi * cd - sin_phi * sd;
+        const FP s = sin_phi * cd + cos_phi * sd;
+        const FP q = c * sin_theta;
+        const FP denom = fma(-q, q, (FP) 1);
+        const FP t = denom == (FP) 0 ? (FP) 0 :
+                quotient(cos_rev(P.kL_rev * q) - P.cos_kL, denom);
+        e[k][0] = -c * cos_theta * t;
+        e[k][1] = s * t;
+    }
+    const int row = MATRIX && P.swap_xy ? 1 : 0;
+    if (MATRIX)
+    {
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+        {
+            Cplx<FP> v;
+            v.x = row ? e[1 - k / 2][k % 2] : e[k / 2][k % 2];
+            v.y = (FP) 0;
+            pattern[4 * o + k] = v;
+        }
+    }
+    else
+    {
+        Cplx<FP> v;
+        v.x = sqrt((e[0][0] * e[0][0] + e[0][1] * e[0][1] +
+                e[1][0] * e[1][0] + e[1][1] * e[1][1]) / (FP) 2);
+        v.y = (FP) 0;
+        pattern[o] = v;
     }
 }
 

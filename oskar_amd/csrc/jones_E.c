@@ -3,12 +3,80 @@
  * Jones array (oskar/interferometer/src/oskar_evaluate_jones_E.c:88-192):
  * one oskar_station_beam() per station model, or, with station beam
  * duplication, one per distinct model of the type map and a device copy for
- * every later station of that model.
+ * every later station of that model.  Flat stations of one dipole type with
+ * plain weights are evaluated up to 16 to a launch, by the kernel that
+ * oskar_station_beam() uses for one.
  */
+#include <math.h>
 #include <stdlib.h>
 
 #include "private.h"
 #include "oskar_evaluate_jones_E.h"
+
+/* Beams waiting to be evaluated by one launch: members of the same kind,
+ * over the same directions. */
+typedef struct Group
+{
+    oskar_AaStation member[OSKAR_AA_GROUP];
+    int count, is_3d, normalise, num_points;
+    const oskar_Mem* const* dirs;
+    double frequency_hz;
+    oskar_Mem* beam;
+} Group;
+
+static void group_flush(Group* g, int* status)
+{
+    const int n = g->count;
+    g->count = 0;
+    if (n == 0 || *status) return;
+    *status = oskar_amd_hip_status(oskar_amd_aa_beam_launch(
+            oskar_mem_precision(g->beam), oskar_mem_is_matrix(g->beam),
+            g->is_3d, g->normalise, g->member, n,
+            2.0 * M_PI * g->frequency_hz / 299792458.0, g->num_points,
+            oskar_mem_void_const(g->dirs[0]),
+            oskar_mem_void_const(g->dirs[1]),
+            oskar_mem_void_const(g->dirs[2]), oskar_mem_void(g->beam),
+            oskar_amd_current_stream()));
+}
+
+/* The beam of one station model into row offset_out of the Jones array:
+ * added to the group if it can be evaluated with others, else evaluated
+ * now (rows are independent, so the order does not matter). */
+static void station_row(Group* g, oskar_Station* station,
+        oskar_StationWork* work, int coord_type, int num_points,
+        const oskar_Mem* const source_coords[3], double ref_lon_rad,
+        double ref_lat_rad, const oskar_Telescope* tel, int time_index,
+        double time_start_mjd_utc, double time_mjd_utc, double frequency_hz,
+        int offset_out, oskar_Mem* out, int* status)
+{
+    int is_3d = 0, normalise = 0;
+    oskar_AaStation member;
+    const int norm_type = oskar_telescope_phase_centre_coord_type(tel);
+    const double norm_lon = oskar_telescope_phase_centre_longitude_rad(tel);
+    const double norm_lat = oskar_telescope_phase_centre_latitude_rad(tel);
+    if (*status) return;
+    if (station && oskar_amd_station_beam_member(station, work, coord_type,
+            num_points, source_coords, norm_type, norm_lon, norm_lat,
+            time_index, time_mjd_utc, frequency_hz, offset_out, out,
+            &member, &is_3d, &normalise))
+    {
+        if (g->count == OSKAR_AA_GROUP || (g->count > 0 &&
+                (is_3d != g->is_3d || normalise != g->normalise)))
+            group_flush(g, status);
+        g->is_3d = is_3d;
+        g->normalise = normalise;
+        g->num_points = num_points;
+        g->dirs = source_coords;
+        g->frequency_hz = frequency_hz;
+        g->beam = out;
+        g->member[g->count++] = member;
+        return;
+    }
+    oskar_station_beam(station, work, coord_type, num_points, source_coords,
+            ref_lon_rad, ref_lat_rad, norm_type, norm_lon, norm_lat,
+            time_index, time_start_mjd_utc, time_mjd_utc, frequency_hz,
+            offset_out, out, status);
+}
 
 void oskar_evaluate_jones_E(oskar_Jones* E, int coord_type, int num_points,
         const oskar_Mem* const source_coords[3], double ref_lon_rad,
@@ -36,9 +104,8 @@ void oskar_evaluate_jones_E(oskar_Jones* E, int coord_type, int num_points,
         return;
     }
     oskar_Mem* out = oskar_jones_mem(E);
-    const int norm_type = oskar_telescope_phase_centre_coord_type(tel);
-    const double norm_lon = oskar_telescope_phase_centre_longitude_rad(tel);
-    const double norm_lat = oskar_telescope_phase_centre_latitude_rad(tel);
+    Group group;
+    group.count = 0;
     if (!oskar_telescope_allow_station_beam_duplication(tel))
     {
         if (oskar_telescope_num_station_models(tel) < num_stations)
@@ -47,11 +114,12 @@ void oskar_evaluate_jones_E(oskar_Jones* E, int coord_type, int num_points,
             return;
         }
         for (i = 0; i < num_stations && !*status; ++i)
-            oskar_station_beam(oskar_telescope_station(tel, i), work,
+            station_row(&group, oskar_telescope_station(tel, i), work,
                     coord_type, num_points, source_coords, ref_lon_rad,
-                    ref_lat_rad, norm_type, norm_lon, norm_lat, time_index,
-                    time_start_mjd_utc, time_mjd_utc, frequency_hz,
-                    i * num_sources, out, status);
+                    ref_lat_rad, tel, time_index, time_start_mjd_utc,
+                    time_mjd_utc, frequency_hz, i * num_sources, out,
+                    status);
+        group_flush(&group, status);
         return;
     }
     {
@@ -80,21 +148,25 @@ void oskar_evaluate_jones_E(oskar_Jones* E, int coord_type, int num_points,
             for (j = 0; j < num_done; ++j)
                 if (model_done[j] == model) { row = model_row[j]; break; }
             if (row >= 0)
+            {
+                group_flush(&group, status);
                 oskar_mem_copy_contents(out, out,
                         (size_t) i * (size_t) num_sources,
                         (size_t) row * (size_t) num_sources,
                         (size_t) num_sources, status);
+            }
             else
             {
-                oskar_station_beam(oskar_telescope_station(tel, model), work,
-                        coord_type, num_points, source_coords, ref_lon_rad,
-                        ref_lat_rad, norm_type, norm_lon, norm_lat,
-                        time_index, time_start_mjd_utc, time_mjd_utc,
-                        frequency_hz, i * num_sources, out, status);
+                station_row(&group, oskar_telescope_station(tel, model),
+                        work, coord_type, num_points, source_coords,
+                        ref_lon_rad, ref_lat_rad, tel, time_index,
+                        time_start_mjd_utc, time_mjd_utc, frequency_hz,
+                        i * num_sources, out, status);
                 model_done[num_done] = model;
                 model_row[num_done++] = i;
             }
         }
+        group_flush(&group, status);
         free(model_done);
         free(model_row);
     }

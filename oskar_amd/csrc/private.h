@@ -238,20 +238,51 @@ void oskar_amd_station_beam_aa_unblanked(oskar_Station* s,
         const oskar_Mem* y, const oskar_Mem* z, int time_index,
         double gast_rad, double frequency_hz, oskar_Mem* beam, int* status);
 
-/* The beam of a flat aperture-array station whose elements are all of one
- * dipole type with a common orientation and common polarisation beams, in
- * one kernel per call (dftw.hip aa_fused_kernel): array factor x dipole
- * pattern, blanked below the horizon and, with normalise, divided as
- * oskar_mem_normalise divides by the beam in the direction (nx, ny, nz).
- * covers() says whether a station and beam type are of that kind; the
- * beam goes to beam from offset_out. */
-int oskar_amd_station_beam_aa_fused_covers(const oskar_Station* s,
+/* One station of a group of aperture-array beams (dftw.hip
+ * aa_beam_kernel): flat stations whose elements are all of one dipole type
+ * with a common orientation and common polarisation beams.  x, y, z: true
+ * element positions; weights, or NULL for DFT weights formed from the
+ * measured positions (mx, my, mz), cable lengths (NULL = none) and the
+ * pointing (beam_x, beam_y, beam_z).  norm_power: the power of the dipole
+ * pattern in the normalisation direction (nx, ny, nz), zero below the
+ * horizon.  offset: first element of the output. */
+typedef struct oskar_AaStation
+{
+    const void *x, *y, *z, *mx, *my, *mz, *cable, *weights;
+    double beam_x, beam_y, beam_z, nx, ny, nz, norm_power, norm_factor;
+    double kL, cos_kL, cos_dx, sin_dx, cos_dy, sin_dy;
+    size_t offset;
+    int num_elements, swap_xy;
+} oskar_AaStation;
+#define OSKAR_AA_GROUP 16          /* stations per launch (kernel arguments) */
+
+/* Whether a station and beam type are of that kind. */
+int oskar_amd_aa_station_covers(const oskar_Station* s,
         const oskar_Mem* beam);
-void oskar_amd_station_beam_aa_fused(oskar_Station* s,
-        oskar_StationWork* work, int num_points, const oskar_Mem* x,
-        const oskar_Mem* y, const oskar_Mem* z, int normalise, double nx,
-        double ny, double nz, int time_index, double gast_rad,
-        double frequency_hz, int offset_out, oskar_Mem* beam, int* status);
+/* Whether its weights are plain DFT weights (formed by the beam kernel). */
+int oskar_amd_aa_station_plain(const oskar_Station* s);
+/* Fills *out for one station (covers() holds); stations with element errors
+ * or apodisation have their weights formed in the work array first. */
+void oskar_amd_aa_station_fill(oskar_Station* s, oskar_StationWork* work,
+        const oskar_Mem* beam, int normalise, double nx, double ny,
+        double nz, int time_index, double gast_rad, double frequency_hz,
+        size_t offset, oskar_AaStation* out, int* status);
+/* A beam as one member of a group, if oskar_station_beam() would evaluate it
+ * by the group kernel with plain weights and the directions as they are:
+ * returns 1 with *out, *is_3d and *normalise filled, else 0 with nothing
+ * done (evaluate it by oskar_station_beam()). */
+int oskar_amd_station_beam_member(oskar_Station* station,
+        oskar_StationWork* work, int source_coord_type, int num_points,
+        const oskar_Mem* const source_coords[3], int norm_coord_type,
+        double norm_lon_rad, double norm_lat_rad, int time_index,
+        double time_mjd_utc, double frequency_hz, int offset_out,
+        const oskar_Mem* beam, oskar_AaStation* out, int* is_3d,
+        int* normalise);
+/* dftw.hip: the beams of `count` stations (at most OSKAR_AA_GROUP). */
+int oskar_amd_aa_beam_launch(int precision, int matrix, int is_3d,
+        int normalise, const oskar_AaStation* stations, int count,
+        double wavenumber, int num_out, const void* x_out,
+        const void* y_out, const void* z_out, void* output, void* stream);
 
 /* ---- piecewise chunk I/O (binary.c) --------------------------------------
  * A chunk written in pieces: begin writes the tag (data_size must equal the
@@ -378,17 +409,7 @@ int oskar_amd_dipole_launch(int precision, int matrix, int num_points,
         const void* theta, const void* phi_x, const void* phi_y, double kL,
         double cos_kL, int swap_xy, int offset_out, void* pattern,
         void* stream);
-/* dftw.hip: the fused aperture-array beam (see
- * oskar_amd_station_beam_aa_fused); output already offset. */
-int oskar_amd_aa_fused_launch(int precision, int matrix, int is_3d,
-        int normalise, int num_in, double wavenumber, const void* weights,
-        const void* x_in, const void* y_in, const void* z_in, int num_out,
-        const void* x_out, const void* y_out, const void* z_out, double nx,
-        double ny, double nz, double kL, double cos_kL, double dphi_x,
-        double dphi_y, int swap_xy, double norm_factor, void* output,
-        void* stream);
-/* The dipole pattern straight from ENU directions (theta_phi then dipole,
- * theta and phi never stored): directions [offset_in, offset_in + num),
+/* The dipole pattern straight from ENU directions: directions [offset_in, offset_in + num),
  * plus the pole at index num with extra_point_at_pole. */
 int oskar_amd_dipole_enu_launch(int precision, int matrix, int offset_in,
         int num, const void* x, const void* y, const void* z,

@@ -1596,7 +1596,7 @@ static void aa_beam(oskar_Station* s, oskar_StationWork* work,
                 beam, status);
 }
 
-int oskar_amd_station_beam_aa_fused_covers(const oskar_Station* s,
+int oskar_amd_aa_station_covers(const oskar_Station* s,
         const oskar_Mem* beam)
 {
     int i = 0;
@@ -1624,71 +1624,105 @@ int oskar_amd_station_beam_aa_fused_covers(const oskar_Station* s,
     return 1;
 }
 
-void oskar_amd_station_beam_aa_fused(oskar_Station* s,
-        oskar_StationWork* work, int num_points, const oskar_Mem* x,
-        const oskar_Mem* y, const oskar_Mem* z, int normalise, double nx,
-        double ny, double nz, int time_index, double gast_rad,
-        double frequency_hz, int offset_out, oskar_Mem* beam, int* status)
+int oskar_amd_aa_station_plain(const oskar_Station* s)
 {
-    double beam_x = 0.0, beam_y = 0.0, beam_z = 0.0;
+    return !s->apply_element_errors && !s->apply_element_weight;
+}
+
+/* Power of the crossed dipoles in one direction: the sum of squares of the
+ * pattern, over 2 (both for a matrix, as oskar_mem_normalise takes it, and
+ * for a scalar amplitude squared). */
+static double dipole_power(const oskar_AaStation* a, double x, double y,
+        double z)
+{
+    double sum = 0.0;
+    int k = 0;
+    const double r = sqrt(x * x + y * y), h = sqrt(x * x + y * y + z * z);
+    const double ct = h > 0.0 ? z / h : 1.0, st = h > 0.0 ? r / h : 0.0;
+    const double cp = r > 0.0 ? x / r : copysign(1.0, x);
+    const double sp = r > 0.0 ? y / r : 0.0;
+    if (z < 0.0) return 0.0;
+    for (k = 0; k < 2; ++k)
+    {
+        const double cd = k ? a->cos_dy : a->cos_dx;
+        const double sd = k ? a->sin_dy : a->sin_dx;
+        const double c = cp * cd - sp * sd, s = sp * cd + cp * sd;
+        const double q = c * st, denom = fma(-q, q, 1.0);
+        const double t = denom == 0.0 ? 0.0 :
+                (cos(a->kL * q) - a->cos_kL) / denom;
+        sum += (c * ct * t) * (c * ct * t) + (s * t) * (s * t);
+    }
+    return 0.5 * sum;
+}
+
+void oskar_amd_aa_station_fill(oskar_Station* s, oskar_StationWork* work,
+        const oskar_Mem* beam, int normalise, double nx, double ny,
+        double nz, int time_index, double gast_rad, double frequency_hz,
+        size_t offset, oskar_AaStation* out, int* status)
+{
     int i = 0;
     if (*status) return;
-    if (!oskar_amd_station_beam_aa_fused_covers(s, beam))
+    if (!oskar_amd_aa_station_covers(s, beam))
     {
         *status = OSKAR_ERR_FUNCTION_NOT_AVAILABLE;
         return;
     }
-    for (i = 0; i < 3; ++i)
+    memset(out, 0, sizeof(*out));
+    oskar_station_beam_horizon_direction(s, gast_rad, &out->beam_x,
+            &out->beam_y, &out->beam_z, status);
+    if (!oskar_amd_aa_station_plain(s))
     {
-        const oskar_Mem* d = i == 0 ? x : (i == 1 ? y : z);
-        if (oskar_mem_type(d) != s->precision)
-        {
-            *status = OSKAR_ERR_TYPE_MISMATCH;
-            return;
-        }
-        if (!check_gpu(d, status)) return;
-        if (oskar_mem_length(d) < (size_t) num_points)
-        {
-            *status = OSKAR_ERR_DIMENSION_MISMATCH;
-            return;
-        }
+        station_weights(s, 0, work, 2.0 * M_PI * frequency_hz / C_0,
+                out->beam_x, out->beam_y, out->beam_z, time_index, status);
+        if (*status) return;
+        out->weights = oskar_mem_void_const(work->weights);
     }
-    const double wavenumber = 2.0 * M_PI * frequency_hz / C_0;
-    oskar_station_beam_horizon_direction(s, gast_rad, &beam_x, &beam_y,
-            &beam_z, status);
-    oskar_mem_ensure(beam, (size_t) offset_out + (size_t) num_points, status);
-    station_weights(s, 0, work, wavenumber, beam_x, beam_y, beam_z,
-            time_index, status);
-    if (*status || num_points == 0) return;
+    else
     {
-        /* The element pattern's parameters as element_evaluate forms them
-         * for oskar_convert_enu_directions_to_theta_phi and
-         * oskar_evaluate_dipole_pattern. */
-        const oskar_Element* model = s->element[0];
-        double dipole_length_m = model->dipole_length;
-        if (model->dipole_length_units == OSKAR_WAVELENGTHS)
-            dipole_length_m *= (C_0 / frequency_hz);
-        const double kL = dipole_length_m * (M_PI * frequency_hz / C_0);
-        const double orientation_x =
-                oskar_station_element_euler_index_rad(s, 0, 0, 0) + M_PI / 2;
-        const double orientation_y =
-                oskar_station_element_euler_index_rad(s, 1, 0, 0);
-        const size_t es = oskar_mem_element_size(oskar_mem_type(beam));
-        *status = oskar_amd_hip_status(oskar_amd_aa_fused_launch(
-                s->precision, oskar_mem_is_matrix(beam), s->array_is_3d,
-                normalise, s->num_elements, wavenumber,
-                oskar_mem_void_const(work->weights),
-                oskar_mem_void_const(feed_mem(s, 0, F_TRUE)),
-                oskar_mem_void_const(feed_mem(s, 0, F_TRUE + 1)),
-                oskar_mem_void_const(feed_mem(s, 0, F_TRUE + 2)),
-                num_points, oskar_mem_void_const(x), oskar_mem_void_const(y),
-                oskar_mem_void_const(z), nx, ny, nz, kL, cos(kL),
-                (M_PI / 2) - orientation_x, (M_PI / 2) - orientation_y,
-                s->swap_xy,
-                s->normalise_array_pattern ? 1.0 / s->num_elements : 1.0,
-                (char*) oskar_mem_void(beam) + (size_t) offset_out * es,
-                oskar_amd_current_stream()));
+        /* The checks of oskar_evaluate_element_weights_dft, whose work the
+         * beam kernel does here. */
+        for (i = 0; i < 4 && !*status; ++i)
+            if (oskar_mem_type(feed_mem(s, 0, i < 3 ? F_MEAS + i : F_CABLE))
+                    != s->precision) *status = OSKAR_ERR_TYPE_MISMATCH;
+        for (i = 0; i < 4 && !*status; ++i)
+            if (oskar_mem_location(feed_mem(s, 0, i < 3 ? F_MEAS + i :
+                    F_CABLE)) != OSKAR_GPU)
+                *status = OSKAR_ERR_LOCATION_MISMATCH;
     }
+    if (*status) return;
+    /* The element pattern's parameters as element_evaluate forms them for
+     * oskar_convert_enu_directions_to_theta_phi and
+     * oskar_evaluate_dipole_pattern. */
+    const oskar_Element* model = s->element[0];
+    double dipole_length_m = model->dipole_length;
+    if (model->dipole_length_units == OSKAR_WAVELENGTHS)
+        dipole_length_m *= (C_0 / frequency_hz);
+    const double dphi_x = (M_PI / 2) -
+            (oskar_station_element_euler_index_rad(s, 0, 0, 0) + M_PI / 2);
+    const double dphi_y = (M_PI / 2) -
+            oskar_station_element_euler_index_rad(s, 1, 0, 0);
+    out->kL = dipole_length_m * (M_PI * frequency_hz / C_0);
+    out->cos_kL = cos(out->kL);
+    out->cos_dx = cos(dphi_x);
+    out->sin_dx = sin(dphi_x);
+    out->cos_dy = cos(dphi_y);
+    out->sin_dy = sin(dphi_y);
+    out->x = oskar_mem_void_const(feed_mem(s, 0, F_TRUE));
+    out->y = oskar_mem_void_const(feed_mem(s, 0, F_TRUE + 1));
+    out->z = oskar_mem_void_const(feed_mem(s, 0, F_TRUE + 2));
+    out->mx = oskar_mem_void_const(feed_mem(s, 0, F_MEAS));
+    out->my = oskar_mem_void_const(feed_mem(s, 0, F_MEAS + 1));
+    out->mz = oskar_mem_void_const(feed_mem(s, 0, F_MEAS + 2));
+    out->cable = oskar_mem_void_const(feed_mem(s, 0, F_CABLE));
+    out->nx = nx;
+    out->ny = ny;
+    out->nz = nz;
+    out->norm_power = normalise ? dipole_power(out, nx, ny, nz) : 0.0;
+    out->norm_factor = s->normalise_array_pattern ?
+            1.0 / s->num_elements : 1.0;
+    out->offset = offset;
+    out->num_elements = s->num_elements;
+    out->swap_xy = s->swap_xy;
 }
 
 /* Points per pass through a hierarchical station: each depth holds one

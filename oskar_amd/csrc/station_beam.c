@@ -29,6 +29,7 @@
 #define DEG_TO_RAD 0.017453292519943295769
 #define HOUR_TO_RAD 0.26179938779914943654
 #define SEC_TO_RAD 7.2722052166430399038e-5   /* 2 pi / 86400 */
+#define WAVENUMBER(F) (2.0 * M_PI * (F) / 299792458.0)
 
 double oskar_convert_mjd_to_gmst(double mjd)
 {
@@ -226,13 +227,14 @@ void oskar_station_beam(oskar_Station* station, oskar_StationWork* work,
                 oskar_mem_length(source_coords[i]) >= (size_t) n;
     if (*status) return;
     if (type == OSKAR_STATION_TYPE_AA &&
-            oskar_amd_station_beam_aa_fused_covers(station, beam))
+            oskar_amd_aa_station_covers(station, beam))
     {
         /* A flat station of one dipole type: one kernel forms the array
          * factor, the element pattern, the blank and the normalisation and
          * writes beam (directions read where they are when they are ENU
          * on the device, with no normalisation point appended). */
         const oskar_Mem* d[3];
+        oskar_AaStation a;
         for (i = 0; i < 3; ++i) d[i] = source_coords[i];
         if (!enu_on_device)
         {
@@ -241,9 +243,36 @@ void oskar_station_beam(oskar_Station* station, oskar_StationWork* work,
                     lst_rad, lat_rad, work->enu, status);
             for (i = 0; i < 3; ++i) d[i] = work->enu[i];
         }
-        oskar_amd_station_beam_aa_fused(station, work, num_points, d[0],
-                d[1], d[2], normalise, nx, ny, nz, time_index, gast_rad,
-                frequency_hz, offset_out, beam, status);
+        if (*status) return;
+        for (i = 0; i < 3; ++i)
+        {
+            if (oskar_mem_type(d[i]) != oskar_station_precision(station))
+            {
+                *status = OSKAR_ERR_TYPE_MISMATCH;
+                return;
+            }
+            if (oskar_mem_location(d[i]) != OSKAR_GPU)
+            {
+                *status = OSKAR_ERR_BAD_LOCATION;
+                return;
+            }
+            if (oskar_mem_length(d[i]) < (size_t) num_points)
+            {
+                *status = OSKAR_ERR_DIMENSION_MISMATCH;
+                return;
+            }
+        }
+        oskar_amd_aa_station_fill(station, work, beam, normalise, nx, ny, nz,
+                time_index, gast_rad, frequency_hz, (size_t) offset_out, &a,
+                status);
+        if (*status) return;
+        *status = oskar_amd_hip_status(oskar_amd_aa_beam_launch(
+                oskar_mem_precision(beam), oskar_mem_is_matrix(beam),
+                oskar_station_array_is_3d(station), normalise, &a, 1,
+                WAVENUMBER(frequency_hz), num_points,
+                oskar_mem_void_const(d[0]), oskar_mem_void_const(d[1]),
+                oskar_mem_void_const(d[2]), oskar_mem_void(beam),
+                oskar_amd_current_stream()));
         return;
     }
     if (enu_on_device)
@@ -315,4 +344,51 @@ void oskar_station_beam(oskar_Station* station, oskar_StationWork* work,
                 (char*) oskar_mem_void(beam) + (size_t) offset_out * es,
                 oskar_amd_current_stream()));
     }
+}
+
+int oskar_amd_station_beam_member(oskar_Station* station,
+        oskar_StationWork* work, int source_coord_type, int num_points,
+        const oskar_Mem* const source_coords[3], int norm_coord_type,
+        double norm_lon_rad, double norm_lat_rad, int time_index,
+        double time_mjd_utc, double frequency_hz, int offset_out,
+        const oskar_Mem* beam, oskar_AaStation* out, int* is_3d,
+        int* normalise)
+{
+    double bx = 0, by = 0, bz = 0, nx = 0, ny = 0, nz = 0;
+    int i = 0, status = 0;
+    if (source_coord_type != OSKAR_COORDS_ENU_DIR || num_points <= 0 ||
+            offset_out < 0 || oskar_mem_location(beam) != OSKAR_GPU ||
+            oskar_station_mem_location(station) != OSKAR_GPU ||
+            !oskar_mem_is_complex(beam) ||
+            oskar_mem_precision(beam) != oskar_station_precision(station) ||
+            oskar_station_precision(station) != work->precision ||
+            oskar_station_type(station) != OSKAR_STATION_TYPE_AA ||
+            !oskar_amd_aa_station_covers(station, beam) ||
+            !oskar_amd_aa_station_plain(station) ||
+            oskar_mem_length(beam) < (size_t) offset_out +
+            (size_t) num_points)
+        return 0;
+    for (i = 0; i < 3; ++i)
+        if (oskar_mem_location(source_coords[i]) != OSKAR_GPU ||
+                oskar_mem_type(source_coords[i]) !=
+                oskar_station_precision(station) ||
+                oskar_mem_length(source_coords[i]) < (size_t) num_points)
+            return 0;
+    const double gast_rad = oskar_convert_mjd_to_gast_fast(time_mjd_utc);
+    const double lat_rad = oskar_station_lat_rad(station);
+    const double lst_rad = gast_rad + oskar_station_lon_rad(station);
+    one_direction_to_enu(oskar_station_beam_coord_type(station),
+            oskar_station_beam_lon_rad(station),
+            oskar_station_beam_lat_rad(station), lst_rad, lat_rad,
+            &bx, &by, &bz, &status);
+    if (status || atan2(bz, sqrt(bx * bx + by * by)) < 0.0) return 0;
+    *normalise = oskar_station_normalise_final_beam(station);
+    *is_3d = oskar_station_array_is_3d(station);
+    if (*normalise)
+        one_direction_to_enu(norm_coord_type, norm_lon_rad, norm_lat_rad,
+                lst_rad, lat_rad, &nx, &ny, &nz, &status);
+    oskar_amd_aa_station_fill(station, work, beam, *normalise, nx, ny, nz,
+            time_index, gast_rad, frequency_hz, (size_t) offset_out, out,
+            &status);
+    return status == 0;
 }
