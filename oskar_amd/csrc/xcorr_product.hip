@@ -322,7 +322,9 @@ template <typename FP> struct Sums
     }
 };
 
-/* FP64 sums over stages of the FP32 accumulators (FP64 ones run on). */
+/* FP64 sums over stages of the accumulators (FP32: each stage; FP64: up
+ * to four stages, so that rounding grows with the square root of
+ * the stages rather than of all products). */
 template <typename FP> struct Totals
 {
     double re[2][2][4], im[2][2][4];
@@ -553,13 +555,19 @@ void xcorr_product_kernel(XcorrArgs<FP> A, int tiles)
          * stage is whole: the rest is left to the loop below. */
         Sums<FP> other;
         other.clear();
-        for (; s + 3 * G::TILE <= s_end; s += 2 * G::TILE)
+        for (int pair = 0; s + 3 * G::TILE <= s_end; s += 2 * G::TILE)
         {
             full_stage<FP, MATRIX>(A, d, lds[0], lds[1], s + 2 * G::TILE,
                     s_end, lane, wp, wq, sums, other, tot);
             __syncthreads();
             full_stage<FP, MATRIX>(A, d, lds[1], lds[0], s + 3 * G::TILE,
                     s_end, lane, wp, wq, SINGLE ? other : sums, sums, tot);
+            if (!SINGLE && (++pair & 1) == 0)
+            {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) tot.add(sums, i);
+                sums.clear();
+            }
             __syncthreads();
         }
         if constexpr (SINGLE)
@@ -575,12 +583,9 @@ void xcorr_product_kernel(XcorrArgs<FP> A, int tiles)
         if (role.active)
             part_stage<FP, MATRIX>(lds[buf], lane, wp, wq, role.first,
                     role.step, skip, sums);
-        if constexpr (SINGLE)
-        {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) tot.add(sums, i);
-            sums.clear();
-        }
+        for (int i = 0; i < 16; ++i) tot.add(sums, i);
+        sums.clear();
         /* The other buffer was last read before the last barrier. */
         buf ^= 1;
         if (s + G::TILE < s_end)
@@ -598,8 +603,7 @@ void xcorr_product_kernel(XcorrArgs<FP> A, int tiles)
     for (int i = 0; i < 16; ++i)
     {
         const int r = i / 8, c = (i / 4) % 2, v = i % 4;
-        const double vr = SINGLE ? tot.re[r][c][v] : (double) sums.re[r][c][v];
-        const double vi = SINGLE ? tot.im[r][c][v] : (double) sums.im[r][c][v];
+        const double vr = tot.re[r][c][v], vi = tot.im[r][c][v];
         if (part)
         {
             part[(i * 2 + 0) * 64] = vr;
