@@ -537,7 +537,7 @@ extern "C" int oskar_amd_theta_phi_launch(int precision, int offset_in,
 extern "C" int oskar_amd_dipole_enu_launch(int precision, int matrix,
         int offset_in, int num, const void* x, const void* y, const void* z,
         int extra_point_at_pole, double delta_phi1, double delta_phi2,
-        double kL, double cos_kL, int swap_xy, int offset_out, void* pattern,
+        double kL, int swap_xy, int offset_out, void* pattern,
         void* stream)
 {
     const int total = num + (extra_point_at_pole ? 1 : 0);
@@ -546,7 +546,7 @@ extern "C" int oskar_amd_dipole_enu_launch(int precision, int matrix,
 #define DE(FP, M) hipLaunchKernelGGL((dipole_enu_kernel<FP, M>), \
         grid_for(total), dim3(THREADS), 0, s, offset_in, num, (const FP*) x, \
         (const FP*) y, (const FP*) z, extra_point_at_pole, \
-        (DipoleParams<FP>{(FP) (kL * 0.15915494309189535), (FP) cos_kL, (FP) cos(delta_phi1), \
+        (DipoleParams<FP>{(FP) kL, (FP) cos(delta_phi1), \
         (FP) sin(delta_phi1), (FP) cos(delta_phi2), (FP) sin(delta_phi2), \
         swap_xy}), offset_out, (Cplx<FP>*) pattern)
     if (precision == OSKAR_DOUBLE)

@@ -130,61 +130,64 @@ template <> struct Sinc<double>
     }
 };
 
-/* sin and cos of 2 pi t: t reduced exactly to [-1/2, 1/2], folded to
- * g in [-1/4, 1/4] (the cosine changes sign), then polynomials in g^2 that
- * interpolate sin(2 pi g) / g and cos(2 pi g) at Chebyshev nodes (formed in
- * extended precision).  Largest and RMS error over 5e5 random arguments:
- * 2.7e-16 and 5.5e-17 (sine), 2.2e-16 and 4.9e-17 (cosine); 29 instructions
- * where the library's sincos took about 100. */
-__device__ __forceinline__ void sincos_rev(double t, double* s, double* c)
+/* sin and cos of x: r = x - k pi in [-pi/2, pi/2] (k from the low bits of a
+ * sum with 1.5 2^52, two-part pi), polynomials in r^2 that interpolate
+ * sin(r) / r and cos(r) at Chebyshev nodes (formed in extended precision),
+ * both negated for odd k.  Largest and RMS error over 5e5 random r: 2.4e-16
+ * and 4.4e-17 (sine), 1.8e-16 and 3.9e-17 (cosine); 26 instructions where
+ * the library's sincos took about 100.  The k is exact for |x| up to 2^51
+ * (whose rounding is then half a radian). */
+__device__ __forceinline__ void sincos_fold(double x, double* s, double* c)
 {
-    const double r = t - rint(t);
-    const bool far = fabs(r) > 0.25;
-    const double g = far ? copysign(0.5, r) - r : r;
-    const double y = g * g;
-    double ps = 0.10087905121711918;
-    ps = fma(ps, y, -0.7177290771684038);
-    ps = fma(ps, y, 3.8199275897803275);
-    ps = fma(ps, y, -15.094641648143382);
-    ps = fma(ps, y, 42.05869392458247);
-    ps = fma(ps, y, -76.70585975281163);
-    ps = fma(ps, y, 81.60524927607352);
-    ps = fma(ps, y, -41.341702240399755);
-    ps = fma(ps, y, 6.283185307179586);
-    double pc = 0.2730462895403127;
-    pc = fma(pc, y, -1.7134850372266826);
-    pc = fma(pc, y, 7.903488575512233);
-    pc = fma(pc, y, -26.426255384546224);
-    pc = fma(pc, y, 60.24464134963378);
-    pc = fma(pc, y, -85.45681720652);
-    pc = fma(pc, y, 64.93939402266777);
-    pc = fma(pc, y, -19.739208802178716);
+    const double m = fma(x, 0.31830988618379067, 6755399441055744.0);
+    const double k = m - 6755399441055744.0;
+    double r = fma(-k, 3.141592653589793, x);
+    r = fma(-k, 1.2246467991473532e-16, r);
+    const int sign = __double2loint(m) << 31;
+    const double y = r * r;
+    double ps = 2.731901991295671e-15;
+    ps = fma(ps, y, -7.644016021446303e-13);
+    ps = fma(ps, y, 1.605897917453392e-10);
+    ps = fma(ps, y, -2.505210765661666e-08);
+    ps = fma(ps, y, 2.7557319219632427e-06);
+    ps = fma(ps, y, -0.00019841269841258002);
+    ps = fma(ps, y, 0.008333333333333325);
+    ps = fma(ps, y, -0.16666666666666666);
+    ps = fma(ps, y, 1.0);
+    double pc = 4.627703831606997e-14;
+    pc = fma(pc, y, -1.146469250716007e-11);
+    pc = fma(pc, y, 2.0876630965308777e-09);
+    pc = fma(pc, y, -2.7557317769149775e-07);
+    pc = fma(pc, y, 2.4801587292463866e-05);
+    pc = fma(pc, y, -0.0013888888888860791);
+    pc = fma(pc, y, 0.04166666666666634);
+    pc = fma(pc, y, -0.5);
     pc = fma(pc, y, 1.0);
-    *s = ps * g;
-    *c = far ? -pc : pc;
+    ps *= r;
+    *s = __hiloint2double(__double2hiint(ps) ^ sign, __double2loint(ps));
+    *c = __hiloint2double(__double2hiint(pc) ^ sign, __double2loint(pc));
 }
 
-/* cos(2 pi t) likewise. */
-__device__ __forceinline__ double cos_rev(double t)
+/* sin(x), relative error below 2e-7 (FP32: in revolutions, folded to a
+ * quarter) or 4e-16 next to zero. */
+__device__ __forceinline__ double sin_fold(double x)
 {
     double s, c;
-    sincos_rev(t, &s, &c);
-    return c;
+    sincos_fold(x, &s, &c);
+    return s;
 }
-/* FP32: largest and RMS error 1.3e-7 and 2.9e-8 (12 instructions). */
-__device__ __forceinline__ float cos_rev(float t)
+__device__ __forceinline__ float sin_fold(float x)
 {
+    const float t = x * 0.159154943f;
     const float r = t - rintf(t);
-    const bool far = fabsf(r) > 0.25f;
-    const float g = far ? 0.5f - fabsf(r) : r;
+    const float g = fabsf(r) > 0.25f ? copysignf(0.5f, r) - r : r;
     const float y = g * g;
-    float p = -2.521816254e+1f;
-    p = fmaf(p, y, 6.017903900e+1f);
-    p = fmaf(p, y, -8.545536041e+1f);
-    p = fmaf(p, y, 6.493938446e+1f);
-    p = fmaf(p, y, -1.973920822e+1f);
-    p = fmaf(p, y, 1.0f);
-    return far ? -p : p;
+    float p = 3.975982666e+1f;
+    p = fmaf(p, y, -7.658116913e+1f);
+    p = fmaf(p, y, 8.160247803e+1f);
+    p = fmaf(p, y, -4.134168243e+1f);
+    p = fmaf(p, y, 6.283185482f);
+    return p * g;
 }
 
 /* 1 / sqrt(x) for normal x: the hardware estimate (1 ulp in FP32, about

@@ -42,17 +42,18 @@ namespace {
 constexpr int THREADS = 256;
 constexpr int CHUNK = 256;
 
-/* exp(i 2 pi t) of a phase in revolutions.  FP32: the hardware sine and
- * cosine, which take revolutions, of the phase reduced to [-1/2, 1/2]
- * unless DIRECT: the hardware reduces a phase of up to 256 revolutions
- * exactly (the same errors against the FP64 DFT with and without the
- * reduction at up to 250 revolutions, measured), so DIRECT serves when |t|
- * is bounded below that: two fewer instructions per term. */
+/* exp(i t) of the phase in the unit the kernel carries it in: FP64 phases
+ * are in radians; FP32 phases are in revolutions for the hardware sine and
+ * cosine (which take revolutions), reduced to [-1/2, 1/2] first unless
+ * DIRECT.  The hardware reduces a phase of up to 256 revolutions exactly
+ * (the same errors against the FP64 DFT with and without the reduction at
+ * up to 250 revolutions, measured), so DIRECT serves when |t| is bounded
+ * below that: two fewer instructions per term. */
 template <bool DIRECT, typename FP>
 __device__ __forceinline__ void phase_sincos(FP t, FP* s, FP* c)
 {
     if constexpr (sizeof(FP) == 8)
-        sincos_rev(t, s, c);
+        sincos_fold(t, s, c);
     else
     {
         const float r = DIRECT ? t : t - __builtin_rintf(t);
@@ -61,8 +62,9 @@ __device__ __forceinline__ void phase_sincos(FP t, FP* s, FP* c)
     }
 }
 
-/* Factor from k (x_out x_in + ...) to revolutions, 1 / (2 pi). */
-constexpr double PHASE_UNIT = 0.15915494309189535;
+/* Factor from k (x_out x_in + ...) to the kernel's phase unit. */
+template <typename FP> constexpr double PHASE_UNIT =
+        sizeof(FP) == 8 ? 1.0 : 0.15915494309189535;    /* 1 / (2 pi) */
 
 /* One element of the chunk staged in LDS: position and weight. */
 template <typename FP> struct Elem
@@ -184,7 +186,7 @@ void dftw_kernel(const int num_in, const FP wavenumber,
     FP xo = (FP) 0, yo = (FP) 0, zo = (FP) 0;
     if (active)
     {
-        const FP kk = wavenumber * (FP) PHASE_UNIT;
+        const FP kk = wavenumber * (FP) PHASE_UNIT<FP>;
         xo = kk * x_out[i_out + offset_coord_out];
         yo = kk * y_out[i_out + offset_coord_out];
         if (IS_3D) zo = kk * z_out[i_out + offset_coord_out];
@@ -315,23 +317,26 @@ void dftw_kernel(const int num_in, const FP wavenumber,
     }
 }
 
-/* An element of an aperture-array beam in LDS: position, and the weight as
- * amplitude and phase in revolutions. */
+/* An element of an aperture-array beam in LDS: position, and the weight in
+ * term_weight's form. */
 template <typename FP, bool IS_3D> struct AaElem;
 template <typename FP> struct alignas(4 * sizeof(FP)) AaElem<FP, false>
 {
-    FP x, y, phase, amp;
+    FP x, y;
+    Cplx<FP> w;
     __device__ __forceinline__ FP at(FP xo, FP yo, FP) const
     {
-        return fma(yo, y, fma(xo, x, phase));
+        return term_phase<FP, false>(xo, yo, (FP) 0, x, y, (FP) 0, w);
     }
 };
 template <typename FP> struct alignas(4 * sizeof(FP)) AaElem<FP, true>
 {
-    FP x, y, phase, amp, z, pad[3];
+    FP x, y;
+    Cplx<FP> w;
+    FP z, pad[3];
     __device__ __forceinline__ FP at(FP xo, FP yo, FP zo) const
     {
-        return fma(zo, z, fma(yo, y, fma(xo, x, phase)));
+        return term_phase<FP, true>(xo, yo, zo, x, y, z, w);
     }
 };
 
@@ -351,7 +356,7 @@ struct AaGroup { oskar_AaStation st[OSKAR_AA_GROUP]; };
  * fixed order, so every workgroup of a station gets the same value.
  *
  * Bound: vector instructions: 4 and a hardware sine and cosine (FP32) or
- * 34 (FP64) per element and direction, and about 150 per direction for the
+ * 32 (FP64) per element and direction, and about 150 per direction for the
  * pattern and the output.  60 stations of 96 dipoles x 16,385 directions in
  * FP64: 1.8 ms as 60 launches of 65 workgroups with library sincos and
  * angles, 0.14 ms as 4 launches.  One station of 256 dipoles x 1M
@@ -372,8 +377,8 @@ void aa_beam_kernel(AaGroup G, const double wavenumber, const int num_out,
     const oskar_AaStation& S = G.st[blockIdx.y];
     const int tid = (int) threadIdx.x;
     const int num_in = S.num_elements;
-    const double rev = wavenumber * PHASE_UNIT;
-    const FP kk = (FP) rev;
+    const double unit = wavenumber * PHASE_UNIT<FP>;
+    const FP kk = (FP) unit;
 
     auto element = [&](int g) {
         E e;
@@ -381,20 +386,22 @@ void aa_beam_kernel(AaGroup G, const double wavenumber, const int num_out,
         e.y = ((const FP*) S.y)[g];
         if constexpr (IS_3D) e.z = ((const FP*) S.z)[g];
         if (S.weights)
-        {
-            const Cplx<FP> w = ((const Cplx<FP>*) S.weights)[g];
-            e.amp = sqrt(w.x * w.x + w.y * w.y);
-            e.phase = atan2(w.y, w.x) * (FP) PHASE_UNIT;
-        }
+            e.w = term_weight<FP>(((const Cplx<FP>*) S.weights)[g]);
         else
         {
             double p = (double) ((const FP*) S.mx)[g] * S.beam_x +
                     (double) ((const FP*) S.my)[g] * S.beam_y +
                     (double) ((const FP*) S.mz)[g] * S.beam_z;
             if (S.cable) p += (double) ((const FP*) S.cable)[g];
-            p *= -rev;
-            e.amp = (FP) 1;
-            e.phase = (FP) (p - rint(p));
+            p *= -unit;
+            if constexpr (sizeof(FP) == 4)
+            {
+                /* Whole revolutions taken off before the rounding. */
+                e.w.x = 1.0f;
+                e.w.y = (float) (p - rint(p));
+            }
+            else
+                sincos_fold(p, &e.w.y, &e.w.x);
         }
         return e;
     };
@@ -404,15 +411,16 @@ void aa_beam_kernel(AaGroup G, const double wavenumber, const int num_out,
     {
         const FP xn = kk * (FP) S.nx, yn = kk * (FP) S.ny;
         const FP zn = kk * (FP) S.nz;
-        FP re = (FP) 0, im = (FP) 0;
+        Cplx<FP> a;
+        a.x = a.y = (FP) 0;
         for (int g = tid; g < num_in; g += THREADS)
         {
             const E e = element(g);
             FP s, c;
             phase_sincos<false, FP>(e.at(xn, yn, zn), &s, &c);
-            re = fma(e.amp, c, re);
-            im = fma(e.amp, s, im);
+            term_add<FP>(a, e.w, s, c);
         }
+        FP re = a.x, im = a.y;
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1)
         {
@@ -453,8 +461,7 @@ void aa_beam_kernel(AaGroup G, const double wavenumber, const int num_out,
                 FP s, c;
                 phase_sincos<decltype(direct)::value, FP>(
                         e.at(xo[d], yo[d], zo[d]), &s, &c);
-                af[d].x = fma(e.amp, c, af[d].x);
-                af[d].y = fma(e.amp, s, af[d].y);
+                term_add<FP>(af[d], e.w, s, c);
             }
         };
         int i = 0;
@@ -507,7 +514,7 @@ void aa_beam_kernel(AaGroup G, const double wavenumber, const int num_out,
             sum(chunk, std::true_type(), d_1, d_all);
         }
     }
-    const DipoleParams<FP> P = {(FP) (S.kL * PHASE_UNIT), (FP) S.cos_kL, (FP) S.cos_dx,
+    const DipoleParams<FP> P = {(FP) S.kL, (FP) S.cos_dx,
             (FP) S.sin_dx, (FP) S.cos_dy, (FP) S.sin_dy, S.swap_xy};
 #pragma unroll
     for (int d = 0; d < D; ++d)

@@ -88,13 +88,11 @@ __device__ __forceinline__ void dipole_point(FP theta, FP phi_x, FP phi_y,
 /* The dipole pattern of one ENU direction from its coordinates: the same
  * as theta_phi_point then dipole_point, with the sines and cosines of theta
  * and phi as quotients of the coordinates (phi = 0 or pi at the zenith, as
- * atan2) and each feed's phi turned by its delta's sine and cosine.  What
- * is left of the functions is the cosine of each dipole's projected length
- * (the angles took two atan2, two fmod and three sincos per direction).
- * kL_rev: kL / (2 pi). */
+ * atan2) and each feed's phi turned by its delta's sine and cosine (the
+ * angles took two atan2, two fmod and three sincos per direction). */
 template <typename FP> struct DipoleParams
 {
-    FP kL_rev, cos_kL, cos_dx, sin_dx, cos_dy, sin_dy;
+    FP kL, cos_dx, sin_dx, cos_dy, sin_dy;
     int swap_xy;
 };
 
@@ -109,14 +107,14 @@ __device__ __forceinline__ void dipole_enu_point(FP x, FP y, FP z,
     FP r2 = x * x + y * y;
     const FP h2 = r2 + z * z;
     const bool up = r2 < TINY;
-    const FP sx = up ? x * UP : x, sy = up ? y * UP : y;
-    r2 = sx * sx + sy * sy;
+    const FP ux = up ? x * UP : x, uy = up ? y * UP : y;
+    r2 = ux * ux + uy * uy;
     const bool zenith = !(r2 > (FP) 0);
     const FP ir = inv_sqrt(r2), ih = inv_sqrt(h2);
     const FP cos_theta = h2 > (FP) 0 ? z * ih : (FP) 1;
     const FP sin_theta = up ? (FP) 0 : r2 * ir * ih;
-    const FP cos_phi = zenith ? copysign((FP) 1, x) : sx * ir;
-    const FP sin_phi = zenith ? (FP) 0 : sy * ir;
+    const FP cos_phi = zenith ? copysign((FP) 1, x) : ux * ir;
+    const FP sin_phi = zenith ? (FP) 0 : uy * ir;
     FP e[2][2];
 #pragma unroll
     for (int k = 0; k < 2; ++k)
@@ -124,10 +122,18 @@ __device__ __forceinline__ void dipole_enu_point(FP x, FP y, FP z,
         const FP cd = k ? P.cos_dy : P.cos_dx, sd = k ? P.sin_dy : P.sin_dx;
         const FP c = cos_phi * cd - sin_phi * sd;
         const FP s = sin_phi * cd + cos_phi * sd;
-        const FP q = c * sin_theta;
-        const FP denom = fma(-q, q, (FP) 1);
+        /* t = (cos(kL q) - cos(kL)) / (1 - q^2), q = cos(phi) sin(theta),
+         * with no difference of nearly equal values: 1 - q^2 as the sum of
+         * the other coordinates' squares, and the numerator as 2 sin(kL (1 +
+         * |q|) / 2) sin(kL (1 - |q|) / 2). */
+        const FP q = fabs(c) * sin_theta, sy = s * sin_theta;
+        const FP denom = fma(sy, sy, cos_theta * cos_theta);
+        const FP half = (FP) 0.5 * P.kL;
+        const FP up_q = (FP) 1 + q;
+        const FP num = sin_fold(half * up_q) *
+                sin_fold(half * quotient(denom, up_q));
         const FP t = denom == (FP) 0 ? (FP) 0 :
-                quotient(cos_rev(P.kL_rev * q) - P.cos_kL, denom);
+                (FP) 2 * quotient(num, denom);
         e[k][0] = -c * cos_theta * t;
         e[k][1] = s * t;
     }

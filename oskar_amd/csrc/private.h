@@ -250,7 +250,7 @@ typedef struct oskar_AaStation
 {
     const void *x, *y, *z, *mx, *my, *mz, *cable, *weights;
     double beam_x, beam_y, beam_z, nx, ny, nz, norm_power, norm_factor;
-    double kL, cos_kL, cos_dx, sin_dx, cos_dy, sin_dy;
+    double kL, cos_dx, sin_dx, cos_dy, sin_dy;
     size_t offset;
     int num_elements, swap_xy;
 } oskar_AaStation;
@@ -414,7 +414,7 @@ int oskar_amd_dipole_launch(int precision, int matrix, int num_points,
 int oskar_amd_dipole_enu_launch(int precision, int matrix, int offset_in,
         int num, const void* x, const void* y, const void* z,
         int extra_point_at_pole, double delta_phi1, double delta_phi2,
-        double kL, double cos_kL, int swap_xy, int offset_out, void* pattern,
+        double kL, int swap_xy, int offset_out, void* pattern,
         void* stream);
 int oskar_amd_blank_below_horizon_launch(int precision, int matrix,
         int offset_mask, int num, const void* mask, int offset_out,

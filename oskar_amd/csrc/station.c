@@ -1341,7 +1341,7 @@ static void element_evaluate(const oskar_Element* model, int normalise,
                 oskar_mem_void_const(x), oskar_mem_void_const(y),
                 oskar_mem_void_const(z), normalise,
                 (M_PI / 2) - orientation_x, (M_PI / 2) - orientation_y, kL,
-                cos(kL), swap_xy, offset_out, oskar_mem_void(output),
+                swap_xy, offset_out, oskar_mem_void(output),
                 oskar_amd_current_stream()));
     }
     else *status = OSKAR_ERR_FUNCTION_NOT_AVAILABLE;
@@ -1647,9 +1647,11 @@ static double dipole_power(const oskar_AaStation* a, double x, double y,
         const double cd = k ? a->cos_dy : a->cos_dx;
         const double sd = k ? a->sin_dy : a->sin_dx;
         const double c = cp * cd - sp * sd, s = sp * cd + cp * sd;
-        const double q = c * st, denom = fma(-q, q, 1.0);
+        /* As dipole_enu_point. */
+        const double q = fabs(c) * st, denom = s * st * s * st + ct * ct;
         const double t = denom == 0.0 ? 0.0 :
-                (cos(a->kL * q) - a->cos_kL) / denom;
+                2.0 * sin(0.5 * a->kL * (1.0 + q)) *
+                sin(0.5 * a->kL * denom / (1.0 + q)) / denom;
         sum += (c * ct * t) * (c * ct * t) + (s * t) * (s * t);
     }
     return 0.5 * sum;
@@ -1702,7 +1704,6 @@ void oskar_amd_aa_station_fill(oskar_Station* s, oskar_StationWork* work,
     const double dphi_y = (M_PI / 2) -
             oskar_station_element_euler_index_rad(s, 1, 0, 0);
     out->kL = dipole_length_m * (M_PI * frequency_hz / C_0);
-    out->cos_kL = cos(out->kL);
     out->cos_dx = cos(dphi_x);
     out->sin_dx = sin(dphi_x);
     out->cos_dy = cos(dphi_y);
