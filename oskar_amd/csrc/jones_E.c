@@ -18,7 +18,7 @@
 typedef struct Group
 {
     oskar_AaStation member[OSKAR_AA_GROUP];
-    int count, is_3d, normalise, num_points;
+    int count, size, is_3d, normalise, num_points;
     const oskar_Mem* const* dirs;
     double frequency_hz;
     oskar_Mem* beam;
@@ -37,6 +37,27 @@ static void group_flush(Group* g, int* status)
             oskar_mem_void_const(g->dirs[1]),
             oskar_mem_void_const(g->dirs[2]), oskar_mem_void(g->beam),
             oskar_amd_current_stream()));
+}
+
+/* Members of a launch: as many (up to OSKAR_AA_GROUP) as leave the least of
+ * the last round of workgroups idle, a round being four on each of 256 CUs
+ * (16 stations x 65 workgroups ran as two rounds, 37 us; 15 as one). */
+static int group_size(int num_points)
+{
+    const long long blocks = ((long long) num_points + 255) / 256;
+    int m = 0, best = 1;
+    double most = 0.0;
+    for (m = 1; m <= OSKAR_AA_GROUP; ++m)
+    {
+        const long long rounds = (m * blocks + 1023) / 1024;
+        const double full = (double) (m * blocks) / (1024.0 * rounds);
+        if (full >= most)
+        {
+            most = full;
+            best = m;
+        }
+    }
+    return best;
 }
 
 /* The beam of one station model into row offset_out of the Jones array:
@@ -60,7 +81,7 @@ static void station_row(Group* g, oskar_Station* station,
             time_index, time_mjd_utc, frequency_hz, offset_out, out,
             &member, &is_3d, &normalise))
     {
-        if (g->count == OSKAR_AA_GROUP || (g->count > 0 &&
+        if (g->count == g->size || (g->count > 0 &&
                 (is_3d != g->is_3d || normalise != g->normalise)))
             group_flush(g, status);
         g->is_3d = is_3d;
@@ -106,6 +127,7 @@ void oskar_evaluate_jones_E(oskar_Jones* E, int coord_type, int num_points,
     oskar_Mem* out = oskar_jones_mem(E);
     Group group;
     group.count = 0;
+    group.size = group_size(num_points);
     if (!oskar_telescope_allow_station_beam_duplication(tel))
     {
         if (oskar_telescope_num_station_models(tel) < num_stations)

@@ -20,10 +20,10 @@
  *  - tiles of 2048 sources per 256-thread workgroup, read in rows of 256
  *    (thread t takes source base + 256 j + t, so every load is coalesced);
  *    a 0/1 mask is scanned with wave ballots and population counts;
- *  - block counts -> one workgroup scans them into block offsets and
- *    writes the total after the last index -> each block scans its tile
- *    again, writes the indices of all its sources and scatters its kept
- *    rows;
+ *  - block counts -> (of many tiles: one workgroup scans them into block
+ *    offsets) -> workgroups that share a tile scan it again, write the
+ *    indices of all its sources and copy its kept rows by columns; the
+ *    total goes after the last index;
  *  - the general prefix sum (any int input) gives each thread 8 consecutive
  *    values (two 16-byte loads), scans them serially and the thread totals
  *    across the workgroup.
@@ -31,6 +31,8 @@
  */
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <algorithm>
 
 #include "private.h"
 
@@ -276,8 +278,16 @@ __device__ __forceinline__ void copy_row(int i, int r, int cap_in,
 }
 
 /* Fused clip, last pass: indices of every source of the tile (exclusive
- * scan of the 0/1 mask in source order) and the kept rows scattered. */
-template <typename FP>
+ * scan of the 0/1 mask in source order) and the kept rows.  The tile's kept
+ * sources are listed in LDS, then whole columns are copied through the list
+ * (8 loads in flight per thread, stores of consecutive rows), and the
+ * valid-column counts as 16-byte pieces of consecutive rows.  Workgroups
+ * (x, y) of a tile share its columns and pieces by y.
+ * offsets: the tiles' counts, whose sum before the tile the workgroup forms
+ * itself (and the last tile the total), or with SCANNED their prefix sums.
+ * Bound: HBM.  1M sources, 18 columns, half kept: 57 us with a thread per
+ * row (a load and a store at a time, 489 workgroups). */
+template <typename FP, bool SCANNED>
 __global__ __launch_bounds__(THREADS)
 void clip_scatter_kernel(int num, const int* __restrict__ mask,
         const int* __restrict__ offsets, int* __restrict__ indices,
@@ -285,39 +295,85 @@ void clip_scatter_kernel(int num, const int* __restrict__ mask,
         FP* __restrict__ tout, const int* __restrict__ vin,
         int* __restrict__ vout)
 {
-    __shared__ int pre[ROWS * WAVES];
-    const int base = (int) blockIdx.x * TILE;
-    const int lane = lane_id(), wave = (int) threadIdx.x >> 6;
+    __shared__ int pre[ROWS * WAVES + 1];
+    __shared__ int list[TILE];
+    __shared__ int part[WAVES];
+    const int tile = (int) blockIdx.x, base = tile * TILE;
+    const int tid = (int) threadIdx.x;
+    const int lane = lane_id(), wave = tid >> 6;
     const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     uint64_t bal[ROWS];
 #pragma unroll
     for (int j = 0; j < ROWS; ++j)
     {
-        const int i = base + j * THREADS + (int) threadIdx.x;
+        const int i = base + j * THREADS + tid;
         const int bit = (i < num) ? (mask[i] != 0) : 0;
         bal[j] = __ballot(bit);
         if (lane == 0) pre[j * WAVES + wave] = __popcll(bal[j]);
     }
-    __syncthreads();
-    /* Exclusive scan of the (row, wave) counts in source order. */
-    if (threadIdx.x < 64)
+    if constexpr (!SCANNED)
     {
-        const int v = (lane < ROWS * WAVES) ? pre[lane] : 0;
-        const int ex = wave_scan_incl(v) - v;
-        if (lane < ROWS * WAVES) pre[lane] = ex;
+        int sum = 0;
+        for (int k = tid; k < tile; k += THREADS) sum += offsets[k];
+        sum = wave_scan_incl(sum);
+        if (lane == 63) part[wave] = sum;
     }
     __syncthreads();
-    const int off = offsets[blockIdx.x];
+    /* Exclusive scan of the (row, wave) counts in source order. */
+    if (tid < 64)
+    {
+        const int v = (lane < ROWS * WAVES) ? pre[lane] : 0;
+        const int in = wave_scan_incl(v);
+        if (lane < ROWS * WAVES) pre[lane] = in - v;
+        if (lane == ROWS * WAVES - 1) pre[lane + 1] = in;
+    }
+    __syncthreads();
+    const int kept = pre[ROWS * WAVES];
+    int off;
+    if constexpr (SCANNED) off = offsets[tile];
+    else
+    {
+        off = (part[0] + part[1]) + (part[2] + part[3]);
+        if (tile == (int) gridDim.x - 1 && blockIdx.y == 0 && tid == 0)
+            indices[num] = off + kept;
+    }
 #pragma unroll
     for (int j = 0; j < ROWS; ++j)
     {
-        const int i = base + j * THREADS + (int) threadIdx.x;
+        const int i = base + j * THREADS + tid;
         if (i >= num) continue;
-        const int r = off + pre[j * WAVES + wave] + __popcll(bal[j] & below);
-        indices[i] = r;
-        if ((bal[j] >> lane) & 1ull)
-            copy_row<FP>(i, r, cap_in, cap_out, num_columns, tin, tout, vin,
-                    vout);
+        const int r = pre[j * WAVES + wave] + __popcll(bal[j] & below);
+        if (blockIdx.y == 0) indices[i] = off + r;
+        if ((bal[j] >> lane) & 1ull) list[r] = i;
+    }
+    __syncthreads();
+    for (int c = (int) blockIdx.y; c < num_columns; c += (int) gridDim.y)
+    {
+        const FP* src = tin + (size_t) c * cap_in;
+        FP* dst = tout + (size_t) c * cap_out + off;
+        FP v[ROWS];
+#pragma unroll
+        for (int j = 0; j < ROWS; ++j)
+        {
+            const int k = j * THREADS + tid;
+            if (k < kept) v[j] = src[list[k]];
+        }
+#pragma unroll
+        for (int j = 0; j < ROWS; ++j)
+        {
+            const int k = j * THREADS + tid;
+            if (k < kept) dst[k] = v[j];
+        }
+    }
+    constexpr int Q = NFIX / 4;
+    const int4* src = reinterpret_cast<const int4*>(vin);
+    int4* dst = reinterpret_cast<int4*>(vout) + (size_t) Q * off;
+    const int step = THREADS * (int) gridDim.y;
+#pragma unroll 4
+    for (int k = THREADS * (int) blockIdx.y + tid; k < Q * kept; k += step)
+    {
+        const int row = k / Q;
+        dst[k] = src[(size_t) Q * list[row] + (k - Q * row)];
     }
 }
 
@@ -397,14 +453,28 @@ hipError_t clip_t(int num_in, const void* l, const void* m, const void* n,
         err = hipGetLastError();
         if (err != hipSuccess) return err;
     }
-    hipLaunchKernelGGL(scan_offsets_kernel, dim3(1), dim3(1024), 0, s, nb,
-            counts, indices + num_in);
-    err = hipGetLastError();
-    if (err != hipSuccess || nb == 0) return err;
-    hipLaunchKernelGGL((clip_scatter_kernel<FP>), dim3(nb), dim3(THREADS), 0,
-            s, num_in, (const int*) mask, (const int*) counts, indices,
-            cap_in, cap_out, num_columns, (const FP*) tin, (FP*) tout, vin,
-            vout);
+    /* Up to 2048 tiles (4M sources) each workgroup of the last pass adds the
+     * counts before its own (8 per thread), which takes no longer than
+     * starting a kernel to scan them (2 us and its launch). */
+    const bool scan = nb > 2048 || nb == 0;
+    if (scan)
+    {
+        hipLaunchKernelGGL(scan_offsets_kernel, dim3(1), dim3(1024), 0, s,
+                nb, counts, indices + num_in);
+        err = hipGetLastError();
+        if (err != hipSuccess || nb == 0) return err;
+    }
+    /* About 2048 workgroups (8 per CU), the columns of a tile shared by at
+     * most one each. */
+    const int share = std::max(1, std::min(num_columns, 2048 / nb));
+    const dim3 grid(nb, share);
+#define CLIP_SCATTER(SCANNED) hipLaunchKernelGGL( \
+        (clip_scatter_kernel<FP, SCANNED>), grid, dim3(THREADS), 0, s, \
+        num_in, (const int*) mask, (const int*) counts, indices, cap_in, \
+        cap_out, num_columns, (const FP*) tin, (FP*) tout, vin, vout)
+    if (scan) CLIP_SCATTER(true);
+    else CLIP_SCATTER(false);
+#undef CLIP_SCATTER
     return hipGetLastError();
 }
 
