@@ -275,9 +275,13 @@ template <typename FP> struct Operands
 {
     FP x[2], y[2], w[2];
 
+    /* LDS elements.  Volatile: the reads stay single ones, whose 16-bit
+     * offsets hold the k-step (paired reads reach only 256 elements, and
+     * need an address of their own per k-step). */
+    typedef const volatile __attribute__((address_space(3))) FP* Lds;
+
     /* xp, yp, xq: this lane's element of the wave's first blocks. */
-    __device__ __forceinline__ void read(const FP* xp, const FP* yp,
-            const FP* xq)
+    __device__ __forceinline__ void read(Lds xp, Lds yp, Lds xq)
     {
 #pragma unroll
         for (int r = 0; r < 2; ++r)
@@ -301,6 +305,22 @@ template <typename FP> struct Sums
 #pragma unroll
             for (int v = 0; v < 4; ++v)
                 re[b / 2][b % 2][v] = im[b / 2][b % 2][v] = (FP) 0;
+    }
+
+    /* The first k-step of a sum: nothing to add to. */
+    __device__ __forceinline__ void multiply_first(const Operands<FP>& o,
+            unsigned int sign)
+    {
+        const FP y0 = flip<FP>(o.y[0], sign), y1 = flip<FP>(o.y[1], sign);
+        const typename Acc<FP>::type z = {(FP) 0, (FP) 0, (FP) 0, (FP) 0};
+        re[0][0] = mfma(o.x[0], o.w[0], z);
+        re[1][0] = mfma(o.x[1], o.w[0], z);
+        re[1][1] = mfma(o.x[1], o.w[1], z);
+        im[0][0] = mfma(y0, o.w[0], z);
+        im[1][0] = mfma(y1, o.w[0], z);
+        im[1][1] = mfma(y1, o.w[1], z);
+        re[0][1] = mfma(o.x[0], o.w[1], z);
+        im[0][1] = mfma(y0, o.w[1], z);
     }
 
     /* skip (wave-uniform): block (0, 1) holds no baseline. */
@@ -365,7 +385,8 @@ __device__ __forceinline__ void full_stage(const XcorrArgs<FP>& A,
     const int ox = opaque(wp * 2 * (4 * BLK) + lane);
     const int oy = opaque(wp * 2 * (4 * BLK) + (lane ^ 16));
     const int oq = opaque(G::SIDE + wq * 2 * (4 * BLK) + lane);
-    const FP *xp = cur + ox, *yp = cur + oy, *xq = cur + oq;
+    typedef typename Operands<FP>::Lds Lds;
+    const Lds xp = (Lds) cur + ox, yp = (Lds) cur + oy, xq = (Lds) cur + oq;
     constexpr int EVERY = G::KT / G::EPT;
     Operands<FP> o[2];
     o[0].read(xp, yp, xq);
@@ -381,8 +402,8 @@ __device__ __forceinline__ void full_stage(const XcorrArgs<FP>& A,
         if (kt % EVERY == 2) d.load_entry(kt / EVERY, s_after, s_end);
         if (kt == G::KT - 1) d.load_flux(A, s_after, s_end);
         if constexpr (SINGLE) tot.add(old, kt);
-        if (SINGLE && kt == 0) sums.clear();
-        sums.multiply(o[kt & 1], sign, false);
+        if (SINGLE && kt == 0) sums.multiply_first(o[0], sign);
+        else sums.multiply(o[kt & 1], sign, false);
         __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
 #pragma unroll
         for (int i = 0; i < 8; ++i)
@@ -404,9 +425,10 @@ __device__ __forceinline__ void part_stage(const FP* cur, int lane, int wp,
     using G = Geo<FP, MATRIX>;
     const unsigned int sign = (lane & 16) ? 0x80000000u : 0u;
     const int at = first * G::KSTRIDE;
-    const FP* xp = cur + wp * 2 * (4 * BLK) + lane + at;
-    const FP* yp = cur + wp * 2 * (4 * BLK) + (lane ^ 16) + at;
-    const FP* xq = cur + G::SIDE + wq * 2 * (4 * BLK) + lane + at;
+    typedef typename Operands<FP>::Lds Lds;
+    Lds xp = (Lds) cur + wp * 2 * (4 * BLK) + lane + at;
+    Lds yp = (Lds) cur + wp * 2 * (4 * BLK) + (lane ^ 16) + at;
+    Lds xq = (Lds) cur + G::SIDE + wq * 2 * (4 * BLK) + lane + at;
     const int inc = step * G::KSTRIDE;
     Operands<FP> o[2];
     o[0].read(xp, yp, xq);
