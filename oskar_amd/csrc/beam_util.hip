@@ -414,51 +414,79 @@ __global__ void join_kernel(size_t n, Cplx<FP>* out, const Cplx<FP>* a,
     }
 }
 
-/* The join on whole 2x2 matrices loaded and stored as aligned blocks
- * (two 16-byte accesses per FP32 matrix, four per FP64), one element per
- * thread and iteration; arithmetic as join_kernel, term for term.  Used
- * when every pointer is aligned to a matrix. */
+/* The joins on aligned blocks, arithmetic as join_kernel, term for term;
+ * used when every pointer to matrices is aligned to a matrix.  Two
+ * matrices: whole ones (two 16-byte accesses per FP32 matrix, four per
+ * FP64), one element per thread and iteration. */
 template <typename FP> struct alignas(4 * sizeof(Cplx<FP>)) JonesMat
 {
     Cplx<FP> v[4];
 };
 
-template <typename FP, bool AM, bool BM>
+template <typename FP>
 __global__ __launch_bounds__(THREADS)
-void join_vec_kernel(size_t n, JonesMat<FP>* out, const void* a, const void* b)
+void join_vec_kernel(size_t n, JonesMat<FP>* out, const JonesMat<FP>* a,
+        const JonesMat<FP>* b)
 {
     GRID_STRIDE(i, n)
     {
         JonesMat<FP> r;
-        if (AM && BM)
-        {
-            const JonesMat<FP> A = ((const JonesMat<FP>*) a)[i];
-            const JonesMat<FP> B = ((const JonesMat<FP>*) b)[i];
-            Cplx<FP> t0 = cmul_rn(A.v[0], B.v[0]);
-            Cplx<FP> t1 = cmul_rn(A.v[1], B.v[2]);
-            r.v[0].x = t0.x + t1.x; r.v[0].y = t0.y + t1.y;
-            t0 = cmul_rn(A.v[0], B.v[1]); t1 = cmul_rn(A.v[1], B.v[3]);
-            r.v[1].x = t0.x + t1.x; r.v[1].y = t0.y + t1.y;
-            t0 = cmul_rn(A.v[2], B.v[0]); t1 = cmul_rn(A.v[3], B.v[2]);
-            r.v[2].x = t0.x + t1.x; r.v[2].y = t0.y + t1.y;
-            t0 = cmul_rn(A.v[2], B.v[1]); t1 = cmul_rn(A.v[3], B.v[3]);
-            r.v[3].x = t0.x + t1.x; r.v[3].y = t0.y + t1.y;
-        }
-        else if (AM)
-        {
-            const JonesMat<FP> A = ((const JonesMat<FP>*) a)[i];
-            const Cplx<FP> sc = ((const Cplx<FP>*) b)[i];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) r.v[k] = cmul_rn(A.v[k], sc);
-        }
-        else
-        {
-            const Cplx<FP> sc = ((const Cplx<FP>*) a)[i];
-            const JonesMat<FP> B = ((const JonesMat<FP>*) b)[i];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) r.v[k] = cmul_rn(sc, B.v[k]);
-        }
+        const JonesMat<FP> A = a[i];
+        const JonesMat<FP> B = b[i];
+        Cplx<FP> t0 = cmul_rn(A.v[0], B.v[0]);
+        Cplx<FP> t1 = cmul_rn(A.v[1], B.v[2]);
+        r.v[0].x = t0.x + t1.x; r.v[0].y = t0.y + t1.y;
+        t0 = cmul_rn(A.v[0], B.v[1]); t1 = cmul_rn(A.v[1], B.v[3]);
+        r.v[1].x = t0.x + t1.x; r.v[1].y = t0.y + t1.y;
+        t0 = cmul_rn(A.v[2], B.v[0]); t1 = cmul_rn(A.v[3], B.v[2]);
+        r.v[2].x = t0.x + t1.x; r.v[2].y = t0.y + t1.y;
+        t0 = cmul_rn(A.v[2], B.v[1]); t1 = cmul_rn(A.v[3], B.v[3]);
+        r.v[3].x = t0.x + t1.x; r.v[3].y = t0.y + t1.y;
         out[i] = r;
+    }
+}
+
+/* Matrices times scalars (A_MATRIX: matrix * scalar, else scalar * matrix,
+ * operands in join_kernel's order): 16 bytes of a matrix per thread and
+ * iteration, so that a wave's accesses are consecutive, JOIN_EACH in
+ * flight.  Bound: HBM bandwidth.  60 x 16,385 FP64 matrices: 27.5 us as
+ * one matrix per thread (16-byte accesses 64 bytes apart), 21.3 us. */
+constexpr int JOIN_EACH = 4;
+
+template <typename FP> struct alignas(16) JonesPart
+{
+    Cplx<FP> v[16 / sizeof(Cplx<FP>)];
+};
+
+template <typename FP, bool A_MATRIX>
+__global__ __launch_bounds__(THREADS)
+void join_scalar_kernel(size_t n, JonesPart<FP>* out,
+        const JonesPart<FP>* matrix, const Cplx<FP>* scalar)
+{
+    constexpr int NV = 16 / sizeof(Cplx<FP>), PARTS = 4 / NV;
+    const size_t parts = n * PARTS;
+    const size_t first = (size_t) blockIdx.x * (THREADS * JOIN_EACH) +
+            threadIdx.x;
+    JonesPart<FP> m[JOIN_EACH];
+    Cplx<FP> s[JOIN_EACH];
+#pragma unroll
+    for (int e = 0; e < JOIN_EACH; ++e)
+    {
+        const size_t i = first + e * THREADS;
+        const size_t c = i < parts ? i : parts - 1;
+        m[e] = matrix[c];
+        s[e] = scalar[c / PARTS];
+    }
+#pragma unroll
+    for (int e = 0; e < JOIN_EACH; ++e)
+    {
+        const size_t i = first + e * THREADS;
+        JonesPart<FP> r;
+#pragma unroll
+        for (int k = 0; k < NV; ++k)
+            r.v[k] = A_MATRIX ? cmul_rn(m[e].v[k], s[e]) :
+                    cmul_rn(s[e], m[e].v[k]);
+        if (i < parts) out[i] = r;
     }
 }
 
@@ -787,29 +815,38 @@ extern "C" int oskar_amd_jones_join_launch(int precision, int a_matrix,
     const bool aligned = ((size_t) out % mat == 0) &&
             (!a_matrix || (size_t) a % mat == 0) &&
             (!b_matrix || (size_t) b % mat == 0);
-#define JOIN(FP, AM, BM)                                                     \
-    if ((AM || BM) && aligned)                                               \
-        hipLaunchKernelGGL((join_vec_kernel<FP, AM, BM>), grid_for(n),       \
-                dim3(THREADS), 0, s, n, (JonesMat<FP>*) out, a, b);              \
-    else                                                                     \
-        hipLaunchKernelGGL((join_kernel<FP, AM, BM>), grid_for(n),           \
-                dim3(THREADS), 0, s, n, (Cplx<FP>*) out,                     \
-                (const Cplx<FP>*) a, (const Cplx<FP>*) b)
-    if (precision == OSKAR_DOUBLE)
-    {
-        if (a_matrix && b_matrix) JOIN(double, true, true);
-        else if (a_matrix) JOIN(double, true, false);
-        else if (b_matrix) JOIN(double, false, true);
-        else JOIN(double, false, false);
-    }
-    else
-    {
-        if (a_matrix && b_matrix) JOIN(float, true, true);
-        else if (a_matrix) JOIN(float, true, false);
-        else if (b_matrix) JOIN(float, false, true);
-        else JOIN(float, false, false);
-    }
+    const size_t each = (size_t) THREADS * JOIN_EACH;
+#define GENERAL(FP, AM, BM) hipLaunchKernelGGL((join_kernel<FP, AM, BM>), \
+        grid_for(n), dim3(THREADS), 0, s, n, (Cplx<FP>*) out, \
+        (const Cplx<FP>*) a, (const Cplx<FP>*) b)
+#define SCALAR(FP, AM, MATRIX, SC) hipLaunchKernelGGL( \
+        (join_scalar_kernel<FP, AM>), dim3((unsigned) ((n * (sizeof(FP) / 2) \
+        + each - 1) / each)), dim3(THREADS), 0, s, n, (JonesPart<FP>*) out, \
+        (const JonesPart<FP>*) MATRIX, (const Cplx<FP>*) SC)
+#define JOIN(FP) \
+    if (a_matrix && b_matrix) \
+    { \
+        if (aligned) hipLaunchKernelGGL(join_vec_kernel<FP>, grid_for(n), \
+                dim3(THREADS), 0, s, n, (JonesMat<FP>*) out, \
+                (const JonesMat<FP>*) a, (const JonesMat<FP>*) b); \
+        else GENERAL(FP, true, true); \
+    } \
+    else if (a_matrix) \
+    { \
+        if (aligned) SCALAR(FP, true, a, b); \
+        else GENERAL(FP, true, false); \
+    } \
+    else if (b_matrix) \
+    { \
+        if (aligned) SCALAR(FP, false, b, a); \
+        else GENERAL(FP, false, true); \
+    } \
+    else GENERAL(FP, false, false)
+    if (precision == OSKAR_DOUBLE) { JOIN(double); }
+    else { JOIN(float); }
 #undef JOIN
+#undef SCALAR
+#undef GENERAL
     return (int) hipGetLastError();
 }
 
@@ -817,25 +854,25 @@ namespace {
 
 /* K[a][s] (define_evaluate_jones_K.h:56-75, CPU evaluation order).  A
  * thread holds one source's direction and filter value and walks a group of
- * K_GROUP stations (wave-uniform station values), so the source inputs are
+ * stations (wave-uniform station values), so the source inputs are
  * read once per group and each store of a wave covers 64 consecutive
  * sources of one station row. */
-constexpr int K_GROUP = 16;
+constexpr int K_GROUP = 16;         /* most stations of a group */
 
 template <typename FP>
 __global__ __launch_bounds__(256)
 void jones_K_kernel(int num_sources, const FP* l, const FP* m, const FP* n,
-        int num_stations, const FP* u, const FP* v, const FP* w,
+        int group, int num_stations, const FP* u, const FP* v, const FP* w,
         FP wavenumber, const FP* filter, FP fmin, FP fmax, int ignore_w,
         Cplx<FP>* jones)
 {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    const int a0 = blockIdx.y * K_GROUP;
+    const int a0 = blockIdx.y * group;
     if (s >= num_sources) return;
     const FP f = filter[s];
     const bool keep = f > fmin && f <= fmax;
     const FP ls = l[s], ms = m[s], ns1 = n[s] - (FP) 1;
-    const int a1 = min(a0 + K_GROUP, num_stations);
+    const int a1 = min(a0 + group, num_stations);
     for (int a = a0; a < a1; ++a)
     {
         Cplx<FP> k;
@@ -860,20 +897,27 @@ extern "C" int oskar_amd_jones_K_launch(int precision, int num_sources,
         void* jones, void* stream)
 {
     if (num_sources <= 0 || num_stations <= 0) return 0;
-    const dim3 grid((num_sources + 255) / 256,
-            (num_stations + K_GROUP - 1) / K_GROUP);
+    /* Smaller groups while there are fewer than three workgroups for each of
+     * 256 CUs (60 stations, 16,385 sources, FP64: 12.3 us as 260 workgroups
+     * of 16 stations, 7.1 us as 975 of 4). */
+    const int blocks = (num_sources + 255) / 256;
+    int group = K_GROUP;
+    while (group > 1 && (long long) blocks *
+            ((num_stations + group - 1) / group) < 768)
+        group /= 2;
+    const dim3 grid(blocks, (num_stations + group - 1) / group);
     const hipStream_t s = (hipStream_t) stream;
     if (precision == OSKAR_DOUBLE)
         hipLaunchKernelGGL(jones_K_kernel<double>, grid, dim3(256), 0, s,
                 num_sources, (const double*) l, (const double*) m,
-                (const double*) n, num_stations, (const double*) u,
+                (const double*) n, group, num_stations, (const double*) u,
                 (const double*) v, (const double*) w, wavenumber,
                 (const double*) filter, fmin, fmax, ignore_w,
                 (Cplx<double>*) jones);
     else
         hipLaunchKernelGGL(jones_K_kernel<float>, grid, dim3(256), 0, s,
                 num_sources, (const float*) l, (const float*) m,
-                (const float*) n, num_stations, (const float*) u,
+                (const float*) n, group, num_stations, (const float*) u,
                 (const float*) v, (const float*) w, (float) wavenumber,
                 (const float*) filter, (float) fmin, (float) fmax, ignore_w,
                 (Cplx<float>*) jones);
