@@ -41,10 +41,11 @@
  * Bound: vector instructions.  FP32 matrices with all factors take 92 per
  * evaluation, 40 of them the contraction (163 with library sines, divisions
  * and both sinc branches), and the vector unit is busy throughout: 512
- * stations x 20,000 sources 10.97 -> 5.84 ms.  FP64 with both smearings
+ * stations x 20,000 sources 10.97 -> 5.73 ms.  FP64 with both smearings
  * takes 82 (565), vector unit 64 % busy at three waves per SIMD: 255 x
  * 10,007 sources 4.69 -> 1.19 ms.  Scalars with bandwidth smearing in FP32,
- * 351 x 50,001: 2.54 -> 1.41 ms.
+ * 351 x 50,001: 2.51 -> 1.35 ms (1.43 with the flux in an LDS
+ * read of its own: LDS was active 71 % of the time).
  */
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -185,7 +186,7 @@ void xcorr_direct_kernel(XcorrArgs<FP> A, int blocks)
     __shared__ V sJa[TILE][VPE][BLOCK_A + 1];
     __shared__ V sJb[TILE][VPE][BLOCK_B + 1];
     __shared__ Quad<FP> sFlux[TILE];      /* I, Q, U, V */
-    __shared__ Quad<FP> sDir[TILE];       /* l, m, n - 1 */
+    __shared__ Quad<FP> sDir[TILE];       /* l, m, n - 1, I */
     __shared__ Quad<FP> sExt[TILE];       /* a, b, c */
 
     const int N = A.num_stations;
@@ -298,7 +299,7 @@ void xcorr_direct_kernel(XcorrArgs<FP> A, int blocks)
                     (MATRIX && in) ? A.V[g] : z};
             if (BS || TS)
                 sDir[s] = Quad<FP>{in ? A.l[g] : z, in ? A.m[g] : z,
-                        in ? A.n[g] - (FP) 1 : z, z};
+                        in ? A.n[g] - (FP) 1 : z, in ? A.I[g] : z};
             if (GAUSS)
             {
                 /* .w: whether the source is extended. */
@@ -351,7 +352,8 @@ void xcorr_direct_kernel(XcorrArgs<FP> A, int blocks)
 #pragma unroll UNROLL
         for (int s = 0; s < TILE; ++s)
         {
-            const Quad<FP> fl = sFlux[s];
+            /* Scalars: the flux, with the direction where that is read. */
+            FP flux = (BS || TS) ? (FP) 0 : sFlux[s].x;
             FP sm[2] = {(FP) 1, (FP) 1};
             if (GAUSS)
             {
@@ -367,6 +369,7 @@ void xcorr_direct_kernel(XcorrArgs<FP> A, int blocks)
             if (BS || TS)
             {
                 const Quad<FP> d = sDir[s];
+                flux = d.w;
                 smear_factors<FP, BS, TS>(bt, d.x, d.y, d.z, sm);
             }
             /* The values of this thread's stations. */
@@ -419,14 +422,13 @@ void xcorr_direct_kernel(XcorrArgs<FP> A, int blocks)
             }
             else
             {
-                const FP Ii = fl.x;
 #pragma unroll
                 for (int k = 0; k < 2; ++k)
                 {
                     FP jb[2];
                     get(&sJb[s][0][lb + 8 * k], BLOCK_B + 1, jb);
                     /* J_first * conj(J_second) * (smear * I) */
-                    const FP w = sm[k] * Ii;
+                    const FP w = sm[k] * flux;
                     const FP re = ja[0] * jb[0] + ja[1] * jb[1];
                     const FP im = ja[1] * jb[0] - ja[0] * jb[1];
                     t[k][0] += re * w;
