@@ -367,14 +367,15 @@ int oskar_amd_sky_copy_launch(int precision, int num_in, int capacity_in,
         int capacity_out, const int* mask, const int* indices,
         int num_columns, const void* table_in, void* table_out,
         const int* valid_in, int* valid_out, void* stream);
-/* Fused clip: mask over all models, block counts, block offsets, then the
- * block scan writes indices (total at [num_in]) and scatters the rows. */
+/* Fused clip: mask over all models with the tiles' counts, then indices
+ * (total at [num_in], and in the pinned word host_total unless that is NULL
+ * or num_in is 0) and the kept rows. */
 int oskar_amd_horizon_clip_launch(int precision, int num_in,
         const void* l, const void* m, const void* n,
         const oskar_HorizonModels* models, int* mask, int* indices,
         int capacity_in, int capacity_out, int num_columns,
         const void* table_in, void* table_out, const int* valid_in,
-        int* valid_out, void* stream);
+        int* valid_out, int* host_total, void* stream);
 
 /* dftw.hip */
 int oskar_amd_dftw_launch(int precision, int matrix, int is_3d,

@@ -50,3 +50,12 @@ def test_none_and_all(hip, models):
     assert sky_out.attr(Sky.NUM_SOURCES) == keep.size
     for t, values in cols:
         assert np.array_equal(sky_out.get_column(t), values[keep])
+
+
+def test_number_kept_over_many_calls(hip):
+    """More calls than pinned words for the number kept, of different sizes
+    and numbers: each call returns its own."""
+    for k in range(70):
+        sky_in, sky_out, cols, want, got_mask, got_idx = clip_case(
+            "f", 100 + 37 * k, [(0.3, -0.5)], 0.1 * k, k)
+        assert sky_out.attr(Sky.NUM_SOURCES) == int(want.sum())
