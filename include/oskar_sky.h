@@ -177,9 +177,10 @@ void oskar_sky_copy_source_data(const oskar_Sky* in,
  * ha0 = (gast + longitude) - RA0, dec0 = the sky's reference Dec, per
  * model), in their input order; the work's horizon mask and source indices
  * hold the mask and its prefix sum afterwards.  out is resized if its
- * capacity is below the input's source count.  The clip runs as three
- * kernels (mask and per-block counts; block offsets; block scan, index
- * write and row scatter) and one 4-byte read of the total. */
+ * capacity is below the input's source count.  The clip runs as two
+ * kernels (mask and per-tile counts; index write and row scatter), with a
+ * third for the tile offsets past 4M sources, and waits for them: the last
+ * writes the total to host memory. */
 OSKAR_EXPORT
 void oskar_sky_horizon_clip(oskar_Sky* out, const oskar_Sky* in,
         const oskar_Telescope* telescope, double gast_rad,
