@@ -29,8 +29,12 @@
  * of a station's matrix, consecutive threads on consecutive addresses,
  * prefetched in registers one stage ahead), forms the row of M for the
  * first side and writes the four contraction steps as [k-step][16-row
- * block][4][16], which an MFMA operand reads as 64 consecutive values.  Y
- * is the same block read with Re and Im exchanged and one sign flipped.
+ * block][4][16], which an MFMA operand reads as 64 consecutive values.
+ * K-steps come in pairs, one of real and one of imaginary parts, so that
+ * the operands of Y are those of X with the two k-steps exchanged and the
+ * sign of one taken by the instruction (FP64) or flipped (FP32): a third
+ * fewer LDS reads and half or none of the flips of k-steps that hold both
+ * parts (7.54 -> 7.36 ms and 0.87 -> 0.85 ms at the sizes below).
  *
  * Bound and measurements: the FP32 and FP64 MFMAs run on the multipliers of
  * the vector unit (no vector instruction issues beside them: matrix and
@@ -39,9 +43,10 @@
  * whole rows of the Jones array per wave instruction (8-byte loads 64 bytes
  * apart cost 13.8 ms instead of 8.1 in FP32).  The per-baseline kernel it
  * replaces read 48 bytes of LDS per evaluation and took, for 512 stations
- * x 100,000 sources in FP32, 24.9 ms (now 7.54 ms, matrix pipe 75 % and vector unit 14 % busy; 7.96
- * with LDS addresses formed per k-step) and, for 197 stations x 30,011
- * sources in FP64, 1.77 ms (now 0.87 ms: 69 % and 11 %).
+ * x 100,000 sources in FP32, 24.9 ms (now 7.36 ms; at 7.54 ms matrix pipe 75 % and vector unit 14 %
+ * busy; 7.96 ms with LDS addresses formed per k-step) and, for 197 stations
+ * x 30,011 sources in FP64, 1.77 ms (now 0.85 ms; at 0.87 ms 69 % and
+ * 11 %).
  *
  * The source range is split over workgroups; partial sums go to an FP64
  * workspace in accumulator order (coalesced) and a second kernel adds the
@@ -63,6 +68,8 @@ constexpr int NT = 256;
 constexpr int ROWS = 64;             /* rows per workgroup side */
 constexpr int BLK = 16;              /* rows of an MFMA operand */
 constexpr int WAVE_VALUES = 2048;    /* FP64 accumulators of a wave */
+/* One k-step of one side: 4 row blocks x 4 x 16 values, and padding. */
+constexpr int KSTRIDE = 4 * 4 * BLK + 2;
 
 typedef double d4v __attribute__((ext_vector_type(4)));
 typedef float f4v __attribute__((ext_vector_type(4)));
@@ -79,6 +86,18 @@ __device__ __forceinline__ f4v mfma(float a, float b, f4v c)
 {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
+/* c - a b as mfma_minus(minus(a), b, c): FP64 instructions negate an
+ * operand themselves (the blgp field's low bit: the first). */
+__device__ __forceinline__ double minus(double a) { return a; }
+__device__ __forceinline__ d4v mfma_minus(double a, double b, d4v c)
+{
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 1);
+}
+__device__ __forceinline__ float minus(float a) { return -a; }
+__device__ __forceinline__ f4v mfma_minus(float a, float b, f4v c)
+{
+    return mfma(a, b, c);
+}
 
 /* Row of accumulator register v in lane group g = lane / 16 (the column is
  * lane % 16). */
@@ -93,15 +112,20 @@ template <typename FP, bool MATRIX> struct Geo
     static constexpr int RPS = MATRIX ? 2 : 1;     /* rows per station */
     static constexpr int SPK = MATRIX ? 1 : 2;     /* sources per k-step */
     static constexpr int KT = sizeof(FP) == 8 ? 8 : 16; /* k-steps, stage */
+    static constexpr int PAIRS = KT / 2;
     static constexpr int TILE = KT * SPK;          /* sources per stage */
     static constexpr int BST = ROWS / RPS;         /* stations, workgroup */
     static constexpr int WST = BST / 2;            /* stations, wave */
     static constexpr int EPT = ROWS * KT / NT;     /* entries per thread */
     static constexpr int RPE = NT / KT;            /* rows between entries */
-    /* One k-step of one side: 4 row blocks x 4 x 16 values.  The padding
-     * puts the threads of one store (RPS neighbouring rows of KT k-steps)
-     * in different banks. */
-    static constexpr int KSTRIDE = 4 * 4 * BLK + 2;
+    /* The four contraction steps of an entry (two complex numbers) and
+     * those of its neighbour make a pair of k-steps: the real parts of all
+     * four numbers, then the imaginary parts.  Steps of a k-step between
+     * the two entries, and between the numbers of one, so that the threads
+     * of one store (neighbouring rows of KT entries) meet different banks,
+     * with the padding of KSTRIDE. */
+    static constexpr int ENTRY = sizeof(FP) == 8 ? BLK : 2 * BLK;
+    static constexpr int NUMBER = 3 * BLK - ENTRY;
     static constexpr int SIDE = KT * KSTRIDE;
     static_assert(RPE % BLK == 0, "entries of a thread: whole row blocks");
 };
@@ -152,7 +176,8 @@ template <typename FP, bool MATRIX> struct Stager
         const int i = tid % G::RPS;
         kt = (tid / G::RPS) % G::KT;
         row0 = (tid / (G::RPS * G::KT)) * G::RPS + i;
-        slot = kt * G::KSTRIDE + (row0 / BLK) * (4 * BLK) + row0 % BLK;
+        slot = (kt & ~1) * KSTRIDE + (kt & 1) * G::ENTRY +
+                (row0 / BLK) * (4 * BLK) + row0 % BLK;
 #pragma unroll
         for (int e = 0; e < G::EPT; ++e)
         {
@@ -229,8 +254,9 @@ template <typename FP, bool MATRIX> struct Stager
         for (int k = 0; k < 4; ++k)
         {
             const bool use = !EDGE || in[MATRIX ? 0 : k / 2];
-            side_p[o + k * BLK] = use ? M[k] : (FP) 0;
-            side_q[o + k * BLK] = use ? q[e][k] : (FP) 0;
+            const int at = o + (k & 1) * KSTRIDE + (k >> 1) * G::NUMBER;
+            side_p[at] = use ? M[k] : (FP) 0;
+            side_q[at] = use ? q[e][k] : (FP) 0;
         }
     }
 
@@ -250,54 +276,42 @@ template <typename FP, bool MATRIX> struct Stager
     }
 };
 
-template <typename FP> __device__ __forceinline__ FP flip(FP x,
-        unsigned int sign);
-template <> __device__ __forceinline__ float flip<float>(float x,
-        unsigned int sign)
-{
-    return __uint_as_float(__float_as_uint(x) ^ sign);
-}
-template <> __device__ __forceinline__ double flip<double>(double x,
-        unsigned int sign)
-{
-    return __hiloint2double(__double2hiint(x) ^ (int) sign,
-            __double2loint(x));
-}
-
 __device__ __forceinline__ int opaque(int x)
 {
     asm volatile("" : "+v"(x));
     return x;
 }
 
-/* Operands of one k-step in a wave: X and Y of its two row blocks on the
- * first side, X of its two on the second. */
+/* Operands of a pair of k-steps in a wave: real (0) and imaginary (1) parts
+ * of its two row blocks on each side. */
 template <typename FP> struct Operands
 {
-    FP x[2], y[2], w[2];
+    FP x[2][2], w[2][2];
 
     /* LDS elements.  Volatile: the reads stay single ones, whose 16-bit
      * offsets hold the k-step (paired reads reach only 256 elements, and
      * need an address of their own per k-step). */
     typedef const volatile __attribute__((address_space(3))) FP* Lds;
 
-    /* xp, yp, xq: this lane's element of the wave's first blocks. */
-    __device__ __forceinline__ void read(Lds xp, Lds yp, Lds xq)
+    /* xp, wp: this lane's element of the wave's first blocks. */
+    __device__ __forceinline__ void read(Lds xp, Lds wp)
     {
 #pragma unroll
-        for (int r = 0; r < 2; ++r)
-        {
-            x[r] = xp[r * (4 * BLK)];
-            y[r] = yp[r * (4 * BLK)];
-            w[r] = xq[r * (4 * BLK)];
-        }
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int r = 0; r < 2; ++r)
+            {
+                x[c][r] = xp[c * KSTRIDE + r * (4 * BLK)];
+                w[c][r] = wp[c * KSTRIDE + r * (4 * BLK)];
+            }
     }
 };
 
 /* A wave's FP accumulators of Re and Im. */
 template <typename FP> struct Sums
 {
-    typename Acc<FP>::type re[2][2], im[2][2];
+    typedef typename Acc<FP>::type A;
+    A re[2][2], im[2][2];
 
     __device__ __forceinline__ void clear()
     {
@@ -308,37 +322,38 @@ template <typename FP> struct Sums
                 re[b / 2][b % 2][v] = im[b / 2][b % 2][v] = (FP) 0;
     }
 
-    /* The first k-step of a sum: nothing to add to. */
-    __device__ __forceinline__ void multiply_first(const Operands<FP>& o,
-            unsigned int sign)
-    {
-        const FP y0 = flip<FP>(o.y[0], sign), y1 = flip<FP>(o.y[1], sign);
-        const typename Acc<FP>::type z = {(FP) 0, (FP) 0, (FP) 0, (FP) 0};
-        re[0][0] = mfma(o.x[0], o.w[0], z);
-        re[1][0] = mfma(o.x[1], o.w[0], z);
-        re[1][1] = mfma(o.x[1], o.w[1], z);
-        im[0][0] = mfma(y0, o.w[0], z);
-        im[1][0] = mfma(y1, o.w[0], z);
-        im[1][1] = mfma(y1, o.w[1], z);
-        re[0][1] = mfma(o.x[0], o.w[1], z);
-        im[0][1] = mfma(y0, o.w[1], z);
-    }
-
-    /* skip (wave-uniform): block (0, 1) holds no baseline. */
+    /* Re += x_re w_re + x_im w_im, Im += x_im w_re - x_re w_im.
+     * skip (wave-uniform): block (0, 1) holds no baseline.  FIRST: the sums
+     * start here. */
+    template <bool FIRST>
     __device__ __forceinline__ void multiply(const Operands<FP>& o,
-            unsigned int sign, bool skip)
+            bool skip)
     {
-        const FP y0 = flip<FP>(o.y[0], sign), y1 = flip<FP>(o.y[1], sign);
-        re[0][0] = mfma(o.x[0], o.w[0], re[0][0]);
-        re[1][0] = mfma(o.x[1], o.w[0], re[1][0]);
-        re[1][1] = mfma(o.x[1], o.w[1], re[1][1]);
-        im[0][0] = mfma(y0, o.w[0], im[0][0]);
-        im[1][0] = mfma(y1, o.w[0], im[1][0]);
-        im[1][1] = mfma(y1, o.w[1], im[1][1]);
+        const A z = {(FP) 0, (FP) 0, (FP) 0, (FP) 0};
+        const FP n[2] = {minus(o.x[0][0]), minus(o.x[0][1])};
+#pragma unroll
+        for (int b = 0; b < 3; ++b)
+        {
+            const int r = b > 0, c = b > 1;    /* (0,0), (1,0), (1,1) */
+            re[r][c] = mfma(o.x[0][r], o.w[0][c], FIRST ? z : re[r][c]);
+            im[r][c] = mfma(o.x[1][r], o.w[0][c], FIRST ? z : im[r][c]);
+        }
         if (!skip)
         {
-            re[0][1] = mfma(o.x[0], o.w[1], re[0][1]);
-            im[0][1] = mfma(y0, o.w[1], im[0][1]);
+            re[0][1] = mfma(o.x[0][0], o.w[0][1], FIRST ? z : re[0][1]);
+            im[0][1] = mfma(o.x[1][0], o.w[0][1], FIRST ? z : im[0][1]);
+        }
+#pragma unroll
+        for (int b = 0; b < 3; ++b)
+        {
+            const int r = b > 0, c = b > 1;
+            re[r][c] = mfma(o.x[1][r], o.w[1][c], re[r][c]);
+            im[r][c] = mfma_minus(n[r], o.w[1][c], im[r][c]);
+        }
+        if (!skip)
+        {
+            re[0][1] = mfma(o.x[1][0], o.w[1][1], re[0][1]);
+            im[0][1] = mfma_minus(n[0], o.w[1][1], im[0][1]);
         }
     }
 };
@@ -380,34 +395,36 @@ __device__ __forceinline__ void full_stage(const XcorrArgs<FP>& A,
 {
     using G = Geo<FP, MATRIX>;
     constexpr bool SINGLE = sizeof(FP) == 4;
-    const unsigned int sign = (lane & 16) ? 0x80000000u : 0u;
     /* Opaque, so that the addresses of the k-steps are formed where they
      * are used instead of being held in registers across stages. */
-    const int ox = opaque(wp * 2 * (4 * BLK) + lane);
-    const int oy = opaque(wp * 2 * (4 * BLK) + (lane ^ 16));
-    const int oq = opaque(G::SIDE + wq * 2 * (4 * BLK) + lane);
     typedef typename Operands<FP>::Lds Lds;
-    const Lds xp = (Lds) cur + ox, yp = (Lds) cur + oy, xq = (Lds) cur + oq;
-    constexpr int EVERY = G::KT / G::EPT;
+    const Lds xp = (Lds) cur + opaque(wp * 2 * (4 * BLK) + lane);
+    const Lds xq = (Lds) cur + opaque(G::SIDE + wq * 2 * (4 * BLK) + lane);
+    constexpr int EVERY = G::PAIRS / G::EPT;
+    static_assert(EVERY == 2, "an entry's store, then its next load");
     Operands<FP> o[2];
-    o[0].read(xp, yp, xq);
+    o[0].read(xp, xq);
 #pragma unroll
-    for (int kt = 0; kt < G::KT; ++kt)
+    for (int m = 0; m < G::PAIRS; ++m)
     {
-        if (kt + 1 < G::KT)
-            o[(kt + 1) & 1].read(xp + (kt + 1) * G::KSTRIDE,
-                    yp + (kt + 1) * G::KSTRIDE, xq + (kt + 1) * G::KSTRIDE);
-        if (kt % EVERY == 1)
-            d.template store_entry<false>(kt / EVERY, nxt,
-                    nxt + G::SIDE);
-        if (kt % EVERY == 2) d.load_entry(kt / EVERY, s_after, s_end);
-        if (kt == G::KT - 1) d.load_flux(A, s_after, s_end);
-        if constexpr (SINGLE) tot.add(old, kt);
-        if (SINGLE && kt == 0) sums.multiply_first(o[0], sign);
-        else sums.multiply(o[kt & 1], sign, false);
-        __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
+        if (m + 1 < G::PAIRS)
+            o[(m + 1) & 1].read(xp + 2 * (m + 1) * KSTRIDE,
+                    xq + 2 * (m + 1) * KSTRIDE);
+        if (m % EVERY == 0)
+            d.template store_entry<false>(m / EVERY, nxt, nxt + G::SIDE);
+        else
+            d.load_entry(m / EVERY, s_after, s_end);
+        if (m == G::PAIRS - 1) d.load_flux(A, s_after, s_end);
+        if constexpr (SINGLE)
+        {
+            tot.add(old, 2 * m);
+            tot.add(old, 2 * m + 1);
+        }
+        if (SINGLE && m == 0) sums.template multiply<true>(o[0], false);
+        else sums.template multiply<false>(o[m & 1], false);
+        __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
+        for (int i = 0; i < 16; ++i)
         {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
             __builtin_amdgcn_sched_group_barrier(0x002, SINGLE ? 6 : 8, 0);
@@ -418,36 +435,33 @@ __device__ __forceinline__ void full_stage(const XcorrArgs<FP>& A,
     }
 }
 
-/* The products of one stage for k-steps first, first + step, ... */
+/* The products of one stage for pairs first, first + step, ... of k-steps. */
 template <typename FP, bool MATRIX>
 __device__ __forceinline__ void part_stage(const FP* cur, int lane, int wp,
         int wq, int first, int step, bool skip, Sums<FP>& sums)
 {
     using G = Geo<FP, MATRIX>;
-    const unsigned int sign = (lane & 16) ? 0x80000000u : 0u;
-    const int at = first * G::KSTRIDE;
+    const int at = first * 2 * KSTRIDE + lane;
     typedef typename Operands<FP>::Lds Lds;
-    Lds xp = (Lds) cur + wp * 2 * (4 * BLK) + lane + at;
-    Lds yp = (Lds) cur + wp * 2 * (4 * BLK) + (lane ^ 16) + at;
-    Lds xq = (Lds) cur + G::SIDE + wq * 2 * (4 * BLK) + lane + at;
-    const int inc = step * G::KSTRIDE;
+    Lds xp = (Lds) cur + wp * 2 * (4 * BLK) + at;
+    Lds xq = (Lds) cur + G::SIDE + wq * 2 * (4 * BLK) + at;
+    const int inc = step * 2 * KSTRIDE;
     Operands<FP> o[2];
-    o[0].read(xp, yp, xq);
-    /* Two k-steps per iteration, each reading the next one's operands
-     * ahead of its MFMAs (the last read repeats the last k-step). */
-    for (int kt = first; kt < G::KT; kt += 2 * step)
+    o[0].read(xp, xq);
+    /* Two pairs per iteration, each reading the next one's operands ahead
+     * of its MFMAs (the last read repeats the last pair). */
+    for (int m = first; m < G::PAIRS; m += 2 * step)
     {
 #pragma unroll
         for (int h = 0; h < 2; ++h)
         {
-            if (kt + h * step >= G::KT) break;
-            const int up = kt + (h + 1) * step < G::KT ? inc : 0;
+            if (m + h * step >= G::PAIRS) break;
+            const int up = m + (h + 1) * step < G::PAIRS ? inc : 0;
             xp += up;
-            yp += up;
             xq += up;
-            o[h ^ 1].read(xp, yp, xq);
+            o[h ^ 1].read(xp, xq);
             __builtin_amdgcn_sched_barrier(0);
-            sums.multiply(o[h], sign, skip);
+            sums.template multiply<false>(o[h], skip);
             __builtin_amdgcn_sched_barrier(0);
         }
     }
