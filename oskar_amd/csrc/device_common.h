@@ -28,23 +28,30 @@ template <> __device__ __forceinline__ double pi_v<double>()
  *   |x| <= SMALL  polynomial in x^2, exactly 1 at 0;
  *   |x| <= MID    polynomial in x^2 - 8 (centred, so that its terms stay
  *                 below 1);
- *   otherwise     sin(r) / x with r = x - k pi (two-part pi, reduced twice
+ *   |x| <= WIDE   sin(r) / x with r = x - k pi (two-part pi, k from the low
+ *                 bits of a sum) and sin(r) = r sinc(r), which is the result
+ *                 itself for k = 0;
+ *   otherwise     the same with r = x - k pi (two-part pi, reduced twice
  *                 so that a rounded k does no harm) in [-pi/2, pi/2] and
  *                 sin(r) = r sinc(r); zero past LARGE, where |sinc| is
  *                 below the precision's roundoff.
  * The polynomials interpolate sin(x)/x at Chebyshev nodes (formed in
  * extended precision).  Largest and RMS error over 4e5 random arguments, in
  * units of 1e-8 (FP32) and 1e-17 (FP64): small 7.9 and 2.0, 14 and 3.6; mid
- * 11 and 2.3, 21 and 4.3; a correctly rounded sin(x) / x has 8.8 and 2.7,
- * 16 and 5.0.  They take 5 and 8 instructions (FP32), 9 and 12 (FP64); a
+ * 11 and 2.3, 21 and 4.3; wide 11 and 1.6, 20 and 3.1 over |x| <= 4 and less
+ * beyond; a correctly rounded sin(x) / x has 8.8 and 2.7, 16 and 5.0.  They
+ * take 5, 8 and 20 instructions (FP32), 9, 12 and 30 (FP64); a
  * library sine and division, taken beside a series for small x by the lanes
  * of a wave, took about 35 and 250.
  */
 template <typename FP> struct Sinc;
+__device__ __forceinline__ float quotient(float a, float b);
+__device__ __forceinline__ double quotient(double a, double b);
 
 template <> struct Sinc<float>
 {
-    static constexpr float SMALL = 1.6f, MID = 4.0f, LARGE = 3e7f;
+    static constexpr float SMALL = 1.6f, MID = 4.0f, WIDE = 1e5f;
+    static constexpr float LARGE = 3e7f;
 
     static __device__ __forceinline__ float small(float x)
     {
@@ -67,6 +74,17 @@ template <> struct Sinc<float>
         p = fmaf(p, y, -6.626768410e-2f);
         return fmaf(p, y, 1.089198068e-1f);
     }
+    static __device__ __forceinline__ float wide(float x)
+    {
+        const float m = fmaf(x, 0.318309886f, 12582912.0f);   /* 1.5 2^23 */
+        const float k = m - 12582912.0f;
+        float r = fmaf(-k, 3.14159274f, x);
+        r = fmaf(-k, -8.74227766e-8f, r);
+        const float p = small(r);
+        const float s = __uint_as_float(__float_as_uint(r * p) ^
+                (__float_as_uint(m) << 31));
+        return k == 0.0f ? p : quotient(s, x);
+    }
     static __device__ __forceinline__ float large(float x)
     {
         float k = rintf(x * 0.318309886f);
@@ -84,7 +102,8 @@ template <> struct Sinc<float>
 
 template <> struct Sinc<double>
 {
-    static constexpr double SMALL = 1.6, MID = 4.0, LARGE = 1e15;
+    static constexpr double SMALL = 1.6, MID = 4.0, WIDE = 1e10;
+    static constexpr double LARGE = 1e15;
 
     static __device__ __forceinline__ double small(double x)
     {
@@ -114,6 +133,17 @@ template <> struct Sinc<double>
         p = fma(p, y, 0.004510723318526139);
         p = fma(p, y, -0.06626768357401747);
         return fma(p, y, 0.10891980905843206);
+    }
+    static __device__ __forceinline__ double wide(double x)
+    {
+        const double m = fma(x, 0.31830988618379067, 6755399441055744.0);
+        const double k = m - 6755399441055744.0;
+        double r = fma(-k, 3.141592653589793, x);
+        r = fma(-k, 1.2246467991473532e-16, r);
+        const double p = small(r), s = r * p;
+        const double q = quotient(__hiloint2double(__double2hiint(s) ^
+                (__double2loint(m) << 31), __double2loint(s)), x);
+        return k == 0.0 ? p : q;
     }
     static __device__ __forceinline__ double large(double x)
     {

@@ -38,10 +38,11 @@
  *    workspace and a second kernel adds them to vis in a fixed order.  No
  *    atomics are used, so results are identical from run to run.
  *
- * Bound: vector instructions.  FP32 matrices with all factors take 92 per
+ * Bound: vector instructions.  FP32 matrices with all factors take 82 per
  * evaluation, 40 of them the contraction (163 with library sines, divisions
- * and both sinc branches), and the vector unit is busy throughout: 512
- * stations x 20,000 sources 10.97 -> 5.73 ms.  FP64 with both smearings
+ * and both sinc branches, 92 with the sinc's last form past MID), and the
+ * vector unit is busy throughout: 512 stations x 20,000 sources 10.86 ->
+ * 5.21 ms (5.73 without the form up to WIDE).  FP64 with both smearings
  * takes 82 (565), vector unit 64 % busy at three waves per SIMD: 255 x
  * 10,007 sources 4.69 -> 1.19 ms.  Scalars with bandwidth smearing in FP32,
  * 351 x 50,001: 2.51 -> 1.35 ms (1.43 with the flux in an LDS
@@ -119,6 +120,8 @@ __device__ __forceinline__ void smear_factors(
         apply([](FP x) { return S::small(x); });
     else if (!__any(most > S::MID))
         apply([](FP x) { return S::mid(x); });
+    else if (!__any(most > S::WIDE))
+        apply([](FP x) { return S::wide(x); });
     else
         apply([](FP x) { return S::large(x); });
 }

@@ -43,10 +43,10 @@
  * whole rows of the Jones array per wave instruction (8-byte loads 64 bytes
  * apart cost 13.8 ms instead of 8.1 in FP32).  The per-baseline kernel it
  * replaces read 48 bytes of LDS per evaluation and took, for 512 stations
- * x 100,000 sources in FP32, 24.9 ms (now 7.36 ms; at 7.54 ms matrix pipe 75 % and vector unit 14 %
- * busy; 7.96 ms with LDS addresses formed per k-step) and, for 197 stations
- * x 30,011 sources in FP64, 1.77 ms (now 0.85 ms; at 0.87 ms 69 % and
- * 11 %).
+ * x 100,000 sources in FP32, 24.9 ms (now 7.36 ms, matrix pipe 76 % and
+ * vector unit 13 % busy; 7.96 ms with LDS addresses formed per k-step)
+ * and, for 197 stations x 30,011 sources in FP64, 1.77 ms (now 0.85 ms,
+ * 71 % and 10 %).
  *
  * The source range is split over workgroups; partial sums go to an FP64
  * workspace in accumulator order (coalesced) and a second kernel adds the

@@ -43,7 +43,8 @@ def one_source(rng, ns, reach, matrix):
 @pytest.mark.parametrize("prec", ["f", "d"])
 @pytest.mark.parametrize("matrix", [0, 1])
 @pytest.mark.parametrize("reach", [0.0, 1e-3, 1.0, 1.599, 1.601, 3.999,
-                                   4.001, 12.0, 300.0, 1e5, 1e12])
+                                   4.001, 12.0, 300.0, 1e5, 1.1e5, 2e10,
+                                   1e12])
 def test_sinc(hip, prec, matrix, reach):
     ns = 70
     g = rounded(one_source(np.random.default_rng(3), ns, reach, matrix), prec)
