@@ -139,6 +139,8 @@ template <typename FP, bool MATRIX> struct Geometry
     static constexpr int TILE = MATRIX ? 16 : 64;
     static constexpr int VPE = MATRIX ? (sizeof(FP) == 4 ? 2 : 4) : 1;
     static constexpr int VR = NR / VPE;
+    /* Fewest sources of a split (the inner loop's granularity). */
+    static constexpr int LEAST = sizeof(FP) == 8 ? 4 : TILE;
     /* Station rows of a tile moved by one wave instruction. */
     static constexpr int RPI = 64 / (TILE * VPE);
     static_assert(RPI * TILE * VPE == 64, "whole station rows per wave");
@@ -352,8 +354,11 @@ void xcorr_direct_kernel(XcorrArgs<FP> A, int blocks)
          * matrix form (more registers would leave three waves per SIMD)
          * and in FP64. */
         constexpr int UNROLL = (sizeof(FP) == 4 && !MATRIX) ? 2 : 1;
+        /* Past ns: zeros (FP32 runs over them: with a count that varies the
+         * matrix kernels pass 128 VGPRs). */
+        const int count = G::LEAST < TILE ? ns : TILE;
 #pragma unroll UNROLL
-        for (int s = 0; s < TILE; ++s)
+        for (int s = 0; s < count; ++s)
         {
             /* Scalars: the flux, with the direction where that is read. */
             FP flux = (BS || TS) ? (FP) 0 : sFlux[s].x;
@@ -564,18 +569,20 @@ hipError_t launch_t(XcorrArgs<FP> A, hipStream_t stream, double* fixed)
     /* Splits: about 12 rounds of four workgroups per CU, so that the last
      * round's idle time is small, with at least 8 tiles of sources each
      * (the prologue and the partial sums cost about one), or one where that
-     * leaves the chip idle (30 stations x 277 sources: 36 workgroups of one
-     * tile instead of 8 of four). */
+     * leaves the chip idle, and down to LEAST sources each while there is less
+     * than a round (30 stations x 277 sources in FP64: 8 workgroups of four
+     * tiles 80 us, 36 of one 21.6 us, 140 of 4 sources 17.7 us). */
     int splits = (12 * 1024 + blocks - 1) / blocks;
     const int max_splits = max(1, max(A.num_sources / (8 * G::TILE),
-            min((A.num_sources + G::TILE - 1) / G::TILE, 1024 / blocks)));
+            min((A.num_sources + G::LEAST - 1) / G::LEAST, 1024 / blocks)));
     splits = max(1, min(splits, min(max_splits, 256)));
     const size_t nb = (size_t) N * (N - 1) / 2;
     /* One split writes vis directly and needs no partial sums. */
     splits = max(1, (int) min((size_t) splits,
             XCORR_PARTIAL_BYTES / (nb * G::NR * sizeof(double))));
     int per = (A.num_sources + splits - 1) / splits;
-    per = ((per + G::TILE - 1) / G::TILE) * G::TILE;
+    const int unit = per < G::TILE ? G::LEAST : G::TILE;
+    per = ((per + unit - 1) / unit) * unit;
     splits = (A.num_sources + per - 1) / per;
     A.src_per_split = per;
     A.num_splits = splits;

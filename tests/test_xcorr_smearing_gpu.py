@@ -93,3 +93,30 @@ def test_gaussian_and_point_sources_together(hip, prec, matrix):
     j = np.abs(g["jones_m" if matrix else "jones_s"]).max()
     scale = (4 if matrix else 1) * 2 * j * j * 4.0 * nsrc
     assert np.max(np.abs(both - apart)) <= 16 * nr * u * scale
+
+
+@pytest.mark.parametrize("prec", ["f", "d"])
+@pytest.mark.parametrize("matrix", [0, 1])
+@pytest.mark.parametrize("nsrc", [1, 3, 4, 5, 17, 65, 277])
+def test_few_sources(hip, prec, matrix, nsrc):
+    """Splits of fewer sources than a tile: the sum of each source on its
+    own, to the rounding of a sum of nsrc terms."""
+    ns = 30
+    from test_xcorr_gpu import random_sky
+    g = rounded(random_sky(np.random.default_rng(nsrc), ns, nsrc,
+                           spread=3000.0), prec)
+    nr = 8 if matrix else 2
+    got = gpu_cross_correlate(prec, 0, 1, matrix, g, 1, 1)
+    apart = np.zeros(got.size)
+    for s in range(nsrc):
+        h = dict(g)
+        for k in ("I", "Q", "U", "V", "l", "m", "n", "a", "b", "c"):
+            h[k] = g[k][s:s + 1]
+        h["jones_m"] = g["jones_m"].reshape(ns, nsrc, 8)[:, s].ravel()
+        h["jones_s"] = g["jones_s"].reshape(ns, nsrc, 2)[:, s].ravel()
+        apart += gpu_cross_correlate(prec, 0, 1, matrix, h, 1,
+                                     1).astype(np.float64)
+    u = 2.0 ** (-53 if prec == "d" else -24)
+    j = np.abs(g["jones_m" if matrix else "jones_s"]).max()
+    scale = (4 if matrix else 1) * 2 * j * j * 4.0 * nsrc
+    assert np.max(np.abs(got - apart)) <= 16 * nr * u * scale
