@@ -28,7 +28,8 @@ struct XcorrArgs
     const void* jones;
     const FP *I, *Q, *U, *V, *l, *m, *n, *a, *b, *c;
     const FP *st_u, *st_v, *st_w, *st_x, *st_y;
-    FP uv_min, uv_max, inv_wl, frac_bw, time_int, gha0, dec0;
+    FP uv_min, uv_max, inv_wl, frac_bw, time_int;
+    FP sin_ha, cos_ha, sin_dec, cos_dec;    /* of the phase centre */
     void* vis;
     double* partial;
 };
@@ -55,17 +56,14 @@ struct BaselineTerms
         du = dv = dw = (FP) 0;
         if (TS)
         {
-            FP sin_ha, cos_ha, sin_dec, cos_dec;
-            sincos_v<FP>(A.gha0, &sin_ha, &cos_ha);
-            sincos_v<FP>(A.dec0, &sin_dec, &cos_dec);
             FP temp = pi_v<FP>() * A.inv_wl;
             const FP xx = (A.st_x[sp] - A.st_x[sq]) * temp;
             const FP yy = (A.st_y[sp] - A.st_y[sq]) * temp;
             const FP rot = ((FP) OMEGA_EARTH) * A.time_int;
-            temp = (xx * sin_ha + yy * cos_ha) * rot;
-            du = (xx * cos_ha - yy * sin_ha) * rot;
-            dv = temp * sin_dec;
-            dw = -temp * cos_dec;
+            temp = (xx * A.sin_ha + yy * A.cos_ha) * rot;
+            du = (xx * A.cos_ha - yy * A.sin_ha) * rot;
+            dv = temp * A.sin_dec;
+            dw = -temp * A.cos_dec;
         }
     }
 };

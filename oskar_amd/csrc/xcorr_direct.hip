@@ -49,6 +49,7 @@
  * read of its own: LDS was active 71 % of the time).
  */
 #include <hip/hip_runtime.h>
+#include <math.h>
 #include <stdint.h>
 
 #include <mutex>
@@ -657,8 +658,12 @@ hipError_t build_and_launch(int matrix, const oskar_XcorrParams* p,
     A.inv_wl = (FP) p->inv_wavelength;
     A.frac_bw = (FP) p->frac_bandwidth;
     A.time_int = (FP) p->time_int_sec;
-    A.gha0 = (FP) p->gha0_rad;
-    A.dec0 = (FP) p->dec0_rad;
+    const double ha = (double) (FP) p->gha0_rad;
+    const double dec = (double) (FP) p->dec0_rad;
+    A.sin_ha = (FP) sin(ha);
+    A.cos_ha = (FP) cos(ha);
+    A.sin_dec = (FP) sin(dec);
+    A.cos_dec = (FP) cos(dec);
     A.vis = vis;
     A.partial = nullptr;
     if (A.num_stations < 2) return hipSuccess;
