@@ -100,19 +100,24 @@ template <typename FP, bool MATRIX>
 __device__ __forceinline__ void dipole_enu_point(FP x, FP y, FP z,
         const DipoleParams<FP>& P, Cplx<FP>* pattern, size_t o)
 {
-    /* Directions next to the zenith, whose x^2 + y^2 would be lost, are
-     * scaled up for phi (theta is 0 there). */
+    /* inv_sqrt and quotient take normal numbers.  Directions next to the
+     * zenith, whose x^2 + y^2 is below TINY, are scaled up for phi (theta is
+     * 0 there), so far that the least subnormal has a normal square; vectors
+     * that are that short altogether are scaled as a whole. */
     constexpr FP TINY = sizeof(FP) == 4 ? (FP) 1e-30 : (FP) 1e-280;
-    constexpr FP UP = sizeof(FP) == 4 ? (FP) 0x1p60 : (FP) 0x1p500;
+    constexpr FP UP = sizeof(FP) == 4 ? (FP) 0x1p100 : (FP) 0x1p800;
     FP r2 = x * x + y * y;
-    const FP h2 = r2 + z * z;
-    const bool up = r2 < TINY;
+    FP h2 = r2 + z * z;
+    const bool up = r2 < TINY, is_short = h2 < TINY;
     const FP ux = up ? x * UP : x, uy = up ? y * UP : y;
+    const FP uz = is_short ? z * UP : z;
     r2 = ux * ux + uy * uy;
+    if (is_short) h2 = r2 + uz * uz;
     const bool zenith = !(r2 > (FP) 0);
     const FP ir = inv_sqrt(r2), ih = inv_sqrt(h2);
-    const FP cos_theta = h2 > (FP) 0 ? z * ih : (FP) 1;
-    const FP sin_theta = up ? (FP) 0 : r2 * ir * ih;
+    const FP cos_theta = h2 > (FP) 0 ? uz * ih : (FP) 1;
+    const FP sin_theta = r2 == (FP) 0 || up != is_short ? (FP) 0 :
+            r2 * ir * ih;
     const FP cos_phi = zenith ? copysign((FP) 1, x) : ux * ir;
     const FP sin_phi = zenith ? (FP) 0 : uy * ir;
     FP e[2][2];
@@ -132,8 +137,9 @@ __device__ __forceinline__ void dipole_enu_point(FP x, FP y, FP z,
         const FP up_q = (FP) 1 + q;
         const FP num = sin_fold(half * up_q) *
                 sin_fold(half * quotient(denom, up_q));
-        const FP t = denom == (FP) 0 ? (FP) 0 :
-                (FP) 2 * quotient(num, denom);
+        /* Along the dipole's axis (denom = sin^2 of the angle to it), where
+         * t stays finite and the field goes to zero: zero. */
+        const FP t = denom < TINY ? (FP) 0 : (FP) 2 * quotient(num, denom);
         e[k][0] = -c * cos_theta * t;
         e[k][1] = s * t;
     }
