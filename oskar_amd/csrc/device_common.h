@@ -198,8 +198,13 @@ __device__ __forceinline__ void sincos_fold(double x, double* s, double* c)
     *c = __hiloint2double(__double2hiint(pc) ^ sign, __double2loint(pc));
 }
 
-/* sin(x), relative error below 2e-7 (FP32: in revolutions, folded to a
- * quarter) or 4e-16 next to zero. */
+/* sin(x): r = x - k pi in [-pi/2, pi/2] (k from the low bits of a sum with
+ * 1.5 2^23 in FP32, two-part pi), r sinc(r) negated for odd k.  FP32:
+ * relative error below 1.5e-7 for |x| up to 2 pi (4.4e-7 up to 32, next to
+ * the multiples of pi too), absolute below 1.7e-7 up to 1e6, against all
+ * floats next to the multiples and 4e6 random ones; a reduction in rounded
+ * revolutions erred by 1.0 of the value next to 2 pi and by 2.8e-6 at 32.
+ * FP64: sincos_fold's sine. */
 __device__ __forceinline__ double sin_fold(double x)
 {
     double s, c;
@@ -208,16 +213,12 @@ __device__ __forceinline__ double sin_fold(double x)
 }
 __device__ __forceinline__ float sin_fold(float x)
 {
-    const float t = x * 0.159154943f;
-    const float r = t - rintf(t);
-    const float g = fabsf(r) > 0.25f ? copysignf(0.5f, r) - r : r;
-    const float y = g * g;
-    float p = 3.975982666e+1f;
-    p = fmaf(p, y, -7.658116913e+1f);
-    p = fmaf(p, y, 8.160247803e+1f);
-    p = fmaf(p, y, -4.134168243e+1f);
-    p = fmaf(p, y, 6.283185482f);
-    return p * g;
+    const float m = fmaf(x, 0.318309886f, 12582912.0f);
+    const float k = m - 12582912.0f;
+    float r = fmaf(-k, 3.14159274f, x);
+    r = fmaf(-k, -8.74227766e-8f, r);
+    return __uint_as_float(__float_as_uint(r * Sinc<float>::small(r)) ^
+            (__float_as_uint(m) << 31));
 }
 
 /* 1 / sqrt(x) for normal x: the hardware estimate (1 ulp in FP32, about

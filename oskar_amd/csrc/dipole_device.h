@@ -130,7 +130,9 @@ __device__ __forceinline__ void dipole_enu_point(FP x, FP y, FP z,
         /* t = (cos(kL q) - cos(kL)) / (1 - q^2), q = cos(phi) sin(theta),
          * with no difference of nearly equal values: 1 - q^2 as the sum of
          * the other coordinates' squares, and the numerator as 2 sin(kL (1 +
-         * |q|) / 2) sin(kL (1 - |q|) / 2). */
+         * |q|) / 2) sin(kL (1 - |q|) / 2).  The first angle is rounded, so
+         * next to the nulls of dipoles of kL = pi and more, where its sine is
+         * near zero, the error is that of the angle, not of the value. */
         const FP q = fabs(c) * sin_theta, sy = s * sin_theta;
         const FP denom = fma(sy, sy, cos_theta * cos_theta);
         const FP half = (FP) 0.5 * P.kL;

@@ -124,3 +124,35 @@ def test_not_a_number_stays(hip, prec):
     got = gpu_beam(prec, (0.0,), x, y, z)
     assert np.all(np.isfinite(got[0]))
     assert not np.any(np.isfinite(got[1:]).all(-1))
+
+
+@pytest.mark.parametrize("prec", ["f", "d"])
+@pytest.mark.parametrize("length", [0.1, 0.5, 1.0, 1.5, 2.0, 9.5])
+def test_long_dipoles(hip, prec, length):
+    """Dipoles of other lengths than half a wave, up to many sines of the
+    pattern.  With denom = 1 - q^2 and q within 6 u, the angles a = kL (1 + q)
+    / 2 and b = kL denom / (2 (1 + q)) are within 5 kL u and 4 kL u, so
+    t = 2 sin(a) sin(b) / denom lies within
+    2 u (5 kL |sin b| + 4 |sin a| min(kL, b)) / denom + 16 u |t|,
+    |sin b| <= min(1, b); the sines' own 2.5 u are among the 16."""
+    rng = np.random.default_rng(8)
+    n, kL = 20000, np.pi * length
+    dt = np.float64 if prec == "d" else np.float32
+    z, p = rng.uniform(0, 1, n), rng.uniform(0, 2 * np.pi, n)
+    r = np.sqrt(1 - z * z)
+    x, y, z = (a.astype(dt) for a in (r * np.cos(p), r * np.sin(p), z))
+    got = gpu_beam(prec, (0.0,), x, y, z, length)
+    want = pattern(x, y, z, 0.0, kL)
+    u = 2.0 ** (-53 if prec == "d" else -24)
+    v = np.stack([x, y, z]).astype(np.float64)
+    v /= np.linalg.norm(v, axis=0)
+    for k in (0, 1):
+        q = np.abs(v[k])
+        denom = v[1 - k] ** 2 + v[2] ** 2
+        a, b = kL / 2 * (1 + q), kL / 2 * denom / (1 + q)
+        t = 2 * np.abs(np.sin(a) * np.sin(b)) / denom
+        tol = 2 * u * (5 * kL * np.minimum(1, b) + 4 * np.abs(np.sin(a)) *
+                       np.minimum(kL, b)) / denom + 16 * u * t
+        err = np.abs(got[:, 2 * k:2 * k + 2] - want[:, 2 * k:2 * k + 2])
+        assert np.all(err.max(-1) <= tol + 1e-300), (k, np.max(
+            err.max(-1) / tol))
