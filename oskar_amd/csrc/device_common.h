@@ -165,8 +165,8 @@ template <> struct Sinc<double>
  * sin(r) / r and cos(r) at Chebyshev nodes (formed in extended precision),
  * both negated for odd k.  Largest and RMS error over 5e5 random r: 2.4e-16
  * and 4.4e-17 (sine), 1.8e-16 and 3.9e-17 (cosine); 26 instructions where
- * the library's sincos took about 100.  The k is exact for |x| up to 2^51
- * (whose rounding is then half a radian). */
+ * the library's sincos took about 100.  For |x| up to 2^50 (whose rounding
+ * is an eighth of a radian); far_phase takes larger ones there. */
 __device__ __forceinline__ void sincos_fold(double x, double* s, double* c)
 {
     const double m = fma(x, 0.31830988618379067, 6755399441055744.0);
@@ -196,6 +196,19 @@ __device__ __forceinline__ void sincos_fold(double x, double* s, double* c)
     ps *= r;
     *s = __hiloint2double(__double2hiint(ps) ^ sign, __double2loint(ps));
     *c = __hiloint2double(__double2hiint(pc) ^ sign, __double2loint(pc));
+}
+
+/* x less whole revolutions, for sincos_fold: within 2^-105 |x| of the angle
+ * for |x| up to 2^100, 0 beyond (where the library's sincos reduces with as
+ * many bits of pi as it takes, in registers that the beam's kernels need: 96
+ * -> 177 with it).  An infinite x gives no number. */
+__device__ __forceinline__ double far_phase(double x)
+{
+    if (fabs(x) < 0x1p50) return x;
+    const double k = rint(x * 0.15915494309189535);
+    double r = fma(-k, 6.283185307179586, x);
+    r = fma(-k, 2.4492935982947064e-16, r);
+    return fabs(r) < 0x1p50 ? r : 0.0 * r;
 }
 
 /* sin(x): r = x - k pi in [-pi/2, pi/2] (k from the low bits of a sum with

@@ -42,18 +42,22 @@ namespace {
 constexpr int THREADS = 256;
 constexpr int CHUNK = 256;
 
-/* exp(i t) of the phase in the unit the kernel carries it in: FP64 phases
- * are in radians; FP32 phases are in revolutions for the hardware sine and
- * cosine (which take revolutions), reduced to [-1/2, 1/2] first unless
- * DIRECT.  The hardware reduces a phase of up to 256 revolutions exactly
- * (the same errors against the FP64 DFT with and without the reduction at
- * up to 250 revolutions, measured), so DIRECT serves when |t| is bounded
- * below that: two fewer instructions per term. */
+/* exp(i t) of the phase in the unit the kernel carries it in.  FP32 phases
+ * are in revolutions for the hardware sine and cosine (which take
+ * revolutions), reduced to [-1/2, 1/2] first unless DIRECT.  The hardware
+ * reduces a phase of up to 256 revolutions exactly (the same errors against
+ * the FP64 DFT with and without the reduction at up to 250 revolutions,
+ * measured), so DIRECT serves when |t| is bounded below that: two fewer
+ * instructions per term.  FP64 phases are in radians; DIRECT serves while
+ * |t| is within the reduction of sincos_fold, past which its polynomials
+ * leave their range without bound. */
 template <bool DIRECT, typename FP>
 __device__ __forceinline__ void phase_sincos(FP t, FP* s, FP* c)
 {
     if constexpr (sizeof(FP) == 8)
-        sincos_fold(t, s, c);
+    {
+        sincos_fold(DIRECT ? t : far_phase(t), s, c);
+    }
     else
     {
         const float r = DIRECT ? t : t - __builtin_rintf(t);
@@ -74,30 +78,30 @@ template <typename FP> struct Elem
 };
 
 /* Largest |coordinate| of the chunk's elements, gathered in LDS as float
- * bits (non-negative floats order as unsigned integers). */
+ * bits (non-negative floats order as unsigned integers); FP64: only whether
+ * any is 2^25 or more (or no number), a store that no array makes. */
 template <typename FP>
-__device__ __forceinline__ void chunk_extent(unsigned int* bits,
-        const Elem<FP>& e)
+__device__ __forceinline__ void chunk_extent(unsigned int* bits, FP x, FP y,
+        FP z)
 {
-    if constexpr (sizeof(FP) == 4)
-    {
-        const float a = fmaxf(fabsf(e.x), fmaxf(fabsf(e.y), fabsf(e.z)));
-        atomicMax(bits, __float_as_uint(a));
-    }
+    const FP a = fmax(fabs(x), fmax(fabs(y), fabs(z)));
+    if constexpr (sizeof(FP) == 4) atomicMax(bits, __float_as_uint(a));
+    else if (!(a < (FP) 0x1p25)) *bits = 1u;
 }
 
-/* Whether every phase of a thread's direction (xo, yo, zo, in revolutions
- * per metre) over elements of extent at most ext stays within the
- * hardware's exact reduction: |t| <= (|xo| + |yo| + |zo|) ext + 1/2 (the
- * weight's phase) < 255. */
+/* Whether every phase of a thread's direction (xo, yo, zo, in phase units
+ * per metre) over the chunk's elements takes phase_sincos's DIRECT form.
+ * FP32: |t| <= (|xo| + |yo| + |zo|) ext + 1/2 (the weight's phase) < 255
+ * revolutions; FP64: |t| < 2^50 radians. */
 template <typename FP>
 __device__ __forceinline__ bool direct_phase(FP xo, FP yo, FP zo,
-        unsigned int ext_bits)
+        unsigned int bits)
 {
-    if constexpr (sizeof(FP) == 8) return false;
+    const FP sum = fabs(xo) + fabs(yo) + fabs(zo);
+    if constexpr (sizeof(FP) == 4)
+        return sum * __uint_as_float(bits) < 254.0f;
     else
-        return (fabsf(xo) + fabsf(yo) + fabsf(zo)) *
-                __uint_as_float(ext_bits) < 254.0f;
+        return sum < (FP) 0x1p25 && bits == 0u;
 }
 
 /* An element's weight in the form the terms use.  FP32: amplitude and
@@ -246,7 +250,7 @@ void dftw_kernel(const int num_in, const FP wavenumber,
             e.pad = (FP) 0;
             e.w = term_weight<FP>(weights[g]);
             c_e[t] = e;
-            chunk_extent<FP>(&c_ext, e);
+            chunk_extent<FP>(&c_ext, e.x, e.y, e.z);
             const int idx = data_idx ? data_idx[g] : g;
             c_idx[t] = idx;
             /* Any element whose data row differs from the chunk's first
@@ -401,7 +405,7 @@ void aa_beam_kernel(AaGroup G, const double wavenumber, const int num_out,
                 e.w.y = (float) (p - rint(p));
             }
             else
-                sincos_fold(p, &e.w.y, &e.w.x);
+                sincos_fold(far_phase(p), &e.w.y, &e.w.x);
         }
         return e;
     };
@@ -465,11 +469,16 @@ void aa_beam_kernel(AaGroup G, const double wavenumber, const int num_out,
             }
         };
         int i = 0;
-        for (; i + 4 <= chunk; i += 4)
+        /* FP64's other form is for phases that no array reaches. */
+        if (sizeof(FP) == 4 || decltype(direct)::value)
         {
+            for (; i + 4 <= chunk; i += 4)
+            {
 #pragma unroll
-            for (int u = 0; u < 4; ++u) term(c_e[i + u]);
+                for (int u = 0; u < 4; ++u) term(c_e[i + u]);
+            }
         }
+#pragma unroll 1
         for (; i < chunk; ++i) term(c_e[i]);
     };
     const std::integral_constant<int, 0> d_0;
@@ -485,23 +494,21 @@ void aa_beam_kernel(AaGroup G, const double wavenumber, const int num_out,
         {
             const E e = element(j + t);
             c_e[t] = e;
-            if constexpr (sizeof(FP) == 4)
-            {
-                FP a = fmaxf(fabsf(e.x), fabsf(e.y));
-                if constexpr (IS_3D) a = fmaxf(a, fabsf(e.z));
-                atomicMax(&c_ext, __float_as_uint(a));
-            }
+            FP z = (FP) 0;
+            if constexpr (IS_3D) z = e.z;
+            chunk_extent<FP>(&c_ext, e.x, e.y, z);
         }
         __syncthreads();
         /* Whether a direction's phases need the reduction depends on that
-         * direction only, so that its value does not depend on D. */
+         * direction only, so that its value does not depend on D (FP64 phases
+         * in DIRECT's range have the same value in both forms). */
         bool direct[D];
 #pragma unroll
         for (int d = 0; d < D; ++d)
             direct[d] = direct_phase<FP>(xo[d], yo[d], zo[d], c_ext);
         if (direct[0] && direct[D - 1])
             sum(chunk, std::true_type(), d_0, d_all);
-        else if (!direct[0] && !direct[D - 1])
+        else if (sizeof(FP) == 8 || (!direct[0] && !direct[D - 1]))
             sum(chunk, std::false_type(), d_0, d_all);
         else if (direct[0])
         {
