@@ -34,6 +34,9 @@
 #include <stdint.h>
 
 #include "private.h"
+#include "workspace.h"
+
+using namespace oskar_amd;
 
 namespace {
 
@@ -218,29 +221,6 @@ void acorr_finish_kernel(int num_stations, int num_chunks, int offset_out,
     vis[((size_t) offset_out + st) * NR + r] += (FP) sum;
 }
 
-/* Per-device FP64 partial-sum buffer, grown on demand and kept for the life
- * of the process.  Growing frees the old buffer (hipFree waits for the
- * device), so earlier launches that still read it have finished. */
-void* acorr_workspace(size_t bytes, hipError_t* err)
-{
-    static void* ptr[64];
-    static size_t size[64];
-    int dev = 0;
-    *err = hipGetDevice(&dev);
-    if (*err != hipSuccess) return nullptr;
-    if (dev < 0 || dev >= 64) { *err = hipErrorInvalidDevice; return nullptr; }
-    if (size[dev] < bytes)
-    {
-        if (ptr[dev]) (void) hipFree(ptr[dev]);
-        ptr[dev] = nullptr;
-        size[dev] = 0;
-        *err = hipMalloc(&ptr[dev], bytes);
-        if (*err != hipSuccess) { ptr[dev] = nullptr; return nullptr; }
-        size[dev] = bytes;
-    }
-    return ptr[dev];
-}
-
 template <typename FP, bool MATRIX>
 hipError_t launch_t(int num_sources, int num_stations, int offset_out,
         const void* jones, const void* I, const void* Q, const void* U,
@@ -259,7 +239,8 @@ hipError_t launch_t(int num_sources, int num_stations, int offset_out,
     per = ((per + 63) / 64) * 64;
     chunks = (num_sources + per - 1) / per;
     hipError_t err = hipSuccess;
-    double* partial = (double*) acorr_workspace(
+    std::lock_guard<std::mutex> guard(ws_launch_lock());
+    double* partial = (double*) ws_acquire_here(WS_ACORR, stream,
             (size_t) chunks * num_stations * NT * sizeof(double), &err);
     if (err != hipSuccess) return err;
     hipLaunchKernelGGL((acorr_partial_kernel<FP, MATRIX>),

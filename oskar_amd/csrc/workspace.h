@@ -1,16 +1,19 @@
 /*
- * Device workspaces of the correlator kernels, one per (device, stream,
- * kind).  Calls on different streams get different buffers, so concurrent
- * correlations on two streams do not share partial sums; calls on one
- * stream are ordered by the stream and reuse its buffer.  A buffer grows
- * (hipFree, which waits for the device, then hipMalloc) when a call needs
- * more; buffers live until the process ends.
+ * Device workspaces of the kernels, one per (device, stream, kind).  Calls
+ * on different streams get different buffers, so concurrent calls on two
+ * streams do not share partial sums; calls on one stream are ordered by the
+ * stream and reuse its buffer.  A buffer grows (hipFree, which waits for the
+ * device, then hipMalloc) when a call needs more.  Buffers live until the
+ * process ends, or until more than a thousand others have been used since
+ * (streams that come and go).
  */
 #ifndef OSKAR_AMD_WORKSPACE_H_
 #define OSKAR_AMD_WORKSPACE_H_
 
 #include <hip/hip_runtime.h>
 #include <stddef.h>
+
+#include <mutex>
 
 namespace oskar_amd {
 
@@ -20,6 +23,7 @@ enum WorkspaceKind
     WS_FACT_SOURCES,         /* shared-beam factorised: stations, sources */
     WS_FACT_PARTIALS,        /* shared-beam factorised: FP32 part tiles */
     WS_FACT_STATIONS,        /* per-station factorised: everything */
+    WS_ACORR,                /* auto-correlator: FP64 partial sums */
     WS_KINDS
 };
 
@@ -27,6 +31,14 @@ enum WorkspaceKind
  * with *err set. */
 void* ws_acquire(int kind, int dev, hipStream_t stream, size_t bytes,
         hipError_t* err);
+
+/* The same on the current device. */
+void* ws_acquire_here(int kind, hipStream_t stream, size_t bytes,
+        hipError_t* err);
+
+/* Held from acquiring a buffer to the last launch that uses it, so that
+ * host threads which share a stream do not interleave their launches. */
+std::mutex& ws_launch_lock();
 
 } /* namespace oskar_amd */
 

@@ -1,6 +1,4 @@
 /* Per-(kind, device, stream) device workspaces (see workspace.h). */
-#include <mutex>
-
 #include "workspace.h"
 
 namespace oskar_amd {
@@ -13,12 +11,15 @@ struct Entry
     hipStream_t stream;
     void* ptr;
     size_t size;
+    unsigned long long used;     /* when it was last acquired */
 };
 
 constexpr int MAX_ENTRIES = 1024;
 Entry g_entries[MAX_ENTRIES];
 int g_count = 0;
+unsigned long long g_clock = 0;
 std::mutex g_lock;
+std::mutex g_launch_lock;
 
 } /* namespace */
 
@@ -38,18 +39,22 @@ void* ws_acquire(int kind, int dev, hipStream_t stream, size_t bytes,
     }
     if (!e)
     {
-        if (g_count == MAX_ENTRIES)
+        if (g_count < MAX_ENTRIES) e = &g_entries[g_count++];
+        else
         {
-            *err = hipErrorOutOfMemory;
-            return nullptr;
+            /* The least recently used (hipFree waits for its device). */
+            e = &g_entries[0];
+            for (int i = 1; i < MAX_ENTRIES; ++i)
+                if (g_entries[i].used < e->used) e = &g_entries[i];
+            if (e->ptr) (void) hipFree(e->ptr);
         }
-        e = &g_entries[g_count++];
         e->kind = kind;
         e->dev = dev;
         e->stream = stream;
         e->ptr = nullptr;
         e->size = 0;
     }
+    e->used = ++g_clock;
     if (e->size < bytes)
     {
         if (e->ptr) (void) hipFree(e->ptr);
@@ -66,5 +71,16 @@ void* ws_acquire(int kind, int dev, hipStream_t stream, size_t bytes,
     *err = hipSuccess;
     return e->ptr;
 }
+
+void* ws_acquire_here(int kind, hipStream_t stream, size_t bytes,
+        hipError_t* err)
+{
+    int dev = 0;
+    *err = hipGetDevice(&dev);
+    return *err == hipSuccess ? ws_acquire(kind, dev, stream, bytes, err) :
+            nullptr;
+}
+
+std::mutex& ws_launch_lock() { return g_launch_lock; }
 
 } /* namespace oskar_amd */

@@ -38,7 +38,8 @@ def test_dftw(hip, num_in, typed):
     idx = np.arange(num_in, dtype=np.int32) % 2 if typed else np.zeros(
         num_in, np.int32)
     data = np.stack([np.ones(2 * x.size), np.zeros(2 * x.size)], 1).ravel()
-    got = gpu_dftw("d", 0, 0, 1.0, w, one, zero, None, x, np.zeros(x.size), None, idx,
+    got = gpu_dftw("d", 0, 0, 1.0, w, one, zero, None, x,
+                   np.zeros(x.size), None, idx,
                    data).reshape(-1, 2)
     want = np.stack([np.cos(x), np.sin(x)], 1)
     tol = 2.0 ** -105 * np.abs(x) + 3e-16 + 2.0 ** -53 * num_in
