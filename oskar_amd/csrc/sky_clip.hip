@@ -35,6 +35,9 @@
 #include <algorithm>
 
 #include "private.h"
+#include "workspace.h"
+
+using namespace oskar_amd;
 
 namespace {
 
@@ -396,27 +399,12 @@ void sky_copy_kernel(int num, int cap_in, int cap_out,
     }
 }
 
-/* Per-device block-count buffer, grown on demand (hipFree waits for the
- * device, so launches that still read the old one have finished). */
-int* counts_buffer(size_t n, hipError_t* err)
+/* Block counts of a call: a workspace of the stream.  The caller holds
+ * ws_launch_lock() over the launches that use it. */
+int* counts_buffer(size_t n, hipStream_t s, hipError_t* err)
 {
-    static void* ptr[64];
-    static size_t size[64];
-    int dev = 0;
-    *err = hipGetDevice(&dev);
-    if (*err != hipSuccess) return nullptr;
-    if (dev < 0 || dev >= 64) { *err = hipErrorInvalidDevice; return nullptr; }
-    const size_t bytes = (n > 0 ? n : 1) * sizeof(int);
-    if (size[dev] < bytes)
-    {
-        if (ptr[dev]) (void) hipFree(ptr[dev]);
-        ptr[dev] = nullptr;
-        size[dev] = 0;
-        *err = hipMalloc(&ptr[dev], bytes);
-        if (*err != hipSuccess) { ptr[dev] = nullptr; return nullptr; }
-        size[dev] = bytes;
-    }
-    return (int*) ptr[dev];
+    return (int*) ws_acquire_here(WS_SKY_COUNTS, s,
+            (n > 0 ? n : 1) * sizeof(int), err);
 }
 
 template <typename FP>
@@ -444,7 +432,8 @@ hipError_t clip_t(int num_in, const void* l, const void* m, const void* n,
 {
     const int nb = (num_in + TILE - 1) / TILE;
     hipError_t err = hipSuccess;
-    int* counts = counts_buffer((size_t) nb, &err);
+    std::lock_guard<std::mutex> guard(ws_launch_lock());
+    int* counts = counts_buffer((size_t) nb, s, &err);
     if (err != hipSuccess) return err;
     if (nb > 0)
     {
@@ -506,7 +495,8 @@ extern "C" int oskar_amd_prefix_sum_launch(int num, const int* in, int* out,
     hipStream_t s = (hipStream_t) stream;
     const int nb = (num + TILE - 1) / TILE;
     hipError_t err = hipSuccess;
-    int* counts = counts_buffer((size_t) nb, &err);
+    std::lock_guard<std::mutex> guard(ws_launch_lock());
+    int* counts = counts_buffer((size_t) nb, s, &err);
     if (err != hipSuccess) return oskar_amd_hip_status((int) err);
     /* 16-byte loads and stores need 16-byte aligned rows of 8 values. */
     const int vec = !(((uintptr_t) in & 15) || ((uintptr_t) out & 15));

@@ -24,6 +24,7 @@ enum WorkspaceKind
     WS_FACT_PARTIALS,        /* shared-beam factorised: FP32 part tiles */
     WS_FACT_STATIONS,        /* per-station factorised: everything */
     WS_ACORR,                /* auto-correlator: FP64 partial sums */
+    WS_SKY_COUNTS,           /* horizon clip, prefix sum: tiles' counts */
     WS_KINDS
 };
 

@@ -9,8 +9,10 @@ import pytest
 
 from gpu_util import sync_check
 from oskar_amd import capi, lib
-from oskar_amd.mem import (OSKAR_COMPLEX, OSKAR_GPU, OSKAR_MATRIX,
-                           OSKAR_SINGLE, Jones, Mem, check_status)
+from oskar_amd.mem import (OSKAR_COMPLEX, OSKAR_GPU, OSKAR_INT, OSKAR_MATRIX,
+                           OSKAR_SINGLE, Jones, Mem, Sky, StationWork,
+                           Telescope, check_status)
+from test_sky_gpu import I_JY, SCRATCH_L, SCRATCH_M, SCRATCH_N, make_sky
 from test_xcorr_seam_gpu import _stream_create, _stream_destroy
 
 pytestmark = pytest.mark.gpu
@@ -40,8 +42,60 @@ class Acorr:
         return [self.vis.numpy()]
 
 
+class Prefix:
+    def __init__(self, seed, num):
+        self.num = num
+        self.src = Mem.from_numpy(np.random.default_rng(seed).integers(
+            0, 9, num).astype(np.int32), OSKAR_INT)
+        self.out = Mem(OSKAR_INT, OSKAR_GPU, num + 1)
+
+    def clear(self):
+        self.out.clear()
+
+    def run(self, status):
+        lib.oskar_prefix_sum(self.num, self.src.ptr, self.out.ptr,
+                             C.byref(status))
+
+    def result(self):
+        return [self.out.numpy()]
+
+
+class Clip:
+    def __init__(self, seed, num):
+        rng = np.random.default_rng(seed)
+        P = OSKAR_SINGLE
+        v = rng.normal(size=(3, num))
+        v /= np.linalg.norm(v, axis=0)
+        self.sky = make_sky(P, num, [
+            (I_JY, rng.uniform(0.1, 9, num)), (SCRATCH_L, v[0]),
+            (SCRATCH_M, v[1]), (SCRATCH_N, v[2])])
+        self.sky.set_reference(1.1, -0.6)
+        self.tel = Telescope(P, OSKAR_GPU, 4)
+        s = C.c_int(0)
+        lib.oskar_telescope_resize_station_array(self.tel.ptr, 1, C.byref(s))
+        lib.oskar_station_set_position(
+            lib.oskar_telescope_station(self.tel.ptr, 0), 0.3, -0.5, 0.0,
+            0.0, 0.0, 0.0)
+        self.out, self.work = Sky(P, OSKAR_GPU, 10), StationWork(P, OSKAR_GPU)
+
+    def clear(self):
+        pass
+
+    def run(self, status):
+        lib.oskar_sky_horizon_clip(self.out.ptr, self.sky.ptr, self.tel.ptr,
+                                   0.8, self.work.ptr, C.byref(status))
+
+    def result(self):
+        return [np.array([self.out.attr(Sky.NUM_SOURCES)])] + [
+            self.out.get_column(c) for c in (I_JY, SCRATCH_N)]
+
+
 def make(which):
-    return Acorr(1, 300, 20000), Acorr(2, 257, 30000)
+    if which == "acorr":
+        return Acorr(1, 300, 20000), Acorr(2, 257, 30000)
+    if which == "prefix_sum":
+        return Prefix(1, 3000001), Prefix(2, 2500000)
+    return Clip(1, 700001), Clip(2, 900000)
 
 
 def serial(calls, which):
@@ -61,7 +115,7 @@ def same(calls, want):
             assert np.array_equal(a, b)
 
 
-@pytest.mark.parametrize("which", ["acorr"])
+@pytest.mark.parametrize("which", ["acorr", "prefix_sum", "clip"])
 def test_two_streams(hip, which):
     calls = make(which)
     want = serial(calls, which)
@@ -85,7 +139,7 @@ def test_two_streams(hip, which):
             _stream_destroy(st)
 
 
-@pytest.mark.parametrize("which", ["acorr"])
+@pytest.mark.parametrize("which", ["acorr", "prefix_sum", "clip"])
 @pytest.mark.parametrize("own", [0, 1])
 def test_two_threads(hip, which, own):
     """Two host threads, each on a stream of its own or both on the null
