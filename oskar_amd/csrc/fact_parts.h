@@ -58,6 +58,40 @@ inline int part_sources(int num_sources, int num_stations, int max_part,
             std::max((long long) unit, (part + unit - 1) / unit * unit));
 }
 
+/* Whether the units of a batch take part_sources(), which sizes the parts of
+ * a unit as if it had the chip to itself, in place of parts of max_part.
+ *
+ * max_part: rounds of workgroups, each as long as the longest part, 1.1 us
+ * per step of a round that is not full and 1.25 us of a full one.
+ * part_sources: the work in full rounds, and 0.03 us per tile and part for
+ * the partial sums.  Past two rounds of max_part little is idle: no (200
+ * units of 97 stations x 12,007 sources: 2835 against 3578 us).  Measured, us (max_part -> part_sources): 97 stations x
+ * 12,007 sources, 16 units 1095 -> 335, 64 units 1170 -> 1177, 170 units 2490
+ * -> 3086; 30 x 2,000, 64 units 319 -> 152, 512 units 371 -> 1127; 300 x 500,
+ * 32 units 191 -> 299.  Where it does not pay it also costs memory: 512 units
+ * of 30 x 2,000 took 3.2 GB of partial sums for 0.1 GB. */
+template <typename Sources>
+bool part_sources_pay(int num_units, Sources sources, int num_stations,
+        int max_part, int unit)
+{
+    const double tiles = (double) part_tiles(num_stations);
+    double items = 0.0, work = 0.0, partials = 0.0, longest = 0.0;
+    for (int u = 0; u < num_units; ++u)
+    {
+        const int S = sources(u);
+        if (S <= 0) continue;
+        const int part = part_sources(S, num_stations, max_part, unit);
+        items += tiles * (double) (((long long) S + max_part - 1) / max_part);
+        partials += tiles * (double) (((long long) S + part - 1) / part);
+        work += tiles * (S / 8.0);
+        longest = std::max(longest, std::min(S, max_part) / 8.0);
+    }
+    if (items >= 2 * PART_SLOTS) return false;
+    const double whole = items <= PART_SLOTS ? 1.1 * longest :
+            1.25 * longest * ceil(items / PART_SLOTS);
+    return 1.25 * work / PART_SLOTS + 0.03 * partials < whole;
+}
+
 } /* namespace oskar_amd */
 
 #endif /* OSKAR_AMD_FACT_PARTS_H_ */

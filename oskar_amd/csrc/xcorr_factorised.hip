@@ -1638,19 +1638,17 @@ hipError_t batch_upload(Batch* b, int nu, int use_casa,
     const size_t nb = (size_t) N * (N - 1) / 2;
     const size_t vis_elem = (b->precision == OSKAR_DOUBLE ? 64 : 32);
 
-    /* A batch of less than two rounds of workgroups at the configured part
-     * size takes the one-call path's part sizes (smaller ones, which cost
-     * more partial sums, for units that leave the chip idle). */
-    long long full = 0;
-    for (int u = 0; u < nu; ++u)
-        full += part_tiles(N) * ((b->units[u].num_sources + max_part - 1) /
-                max_part);
+    /* The one-call path's part sizes, for batches that leave the chip idle
+     * at the configured size. */
+    const bool pay = part_sources_pay(nu,
+            [&](int u) { return b->units[u].num_sources; }, N, max_part,
+            KSRC);
     std::vector<int> part(nu);
     for (int u = 0; u < nu; ++u)
     {
         const int S = b->units[u].num_sources;
-        part[u] = full < 2 * PART_SLOTS && S > 0 ?
-                part_sources(S, N, max_part, KSRC) : max_part;
+        part[u] = pay && S > 0 ? part_sources(S, N, max_part, KSRC) :
+                max_part;
     }
 
     /* Workspace layout per unit: [cmax 256 B][stations][src][cmat][partial]. */
