@@ -931,23 +931,28 @@ __device__ __forceinline__ void block_max_to(float mx, unsigned int* cmax,
                 __HIP_MEMORY_SCOPE_AGENT);
 }
 
-/* Sum over parts in FP64 of 64 baselines (p, q0 + 0..63) of station row p,
- * scale removal, and accumulation into vis[offset_out + b] for baselines
- * inside the uv filter.  Wave g of the workgroup adds the g-th quarter of
- * the parts (consecutive lanes read consecutive partials) and the quarters
- * are added in order, so that a row of a small array keeps 256 threads
- * busy. */
-constexpr int RED_Q = 64;
+/* Sum over parts in FP64 of the baselines (p, q0 ..) of station row p that
+ * a workgroup of 256 takes at once, scale removal, and accumulation into
+ * vis[offset_out + b] for baselines inside the uv filter.  GROUPS groups
+ * of threads add a share of the parts each (consecutive lanes read consecutive
+ * partials) and the shares are added in order: 4 groups of 64 baselines keep
+ * 256 threads busy on a row of a small array; with fewer than RED_PARTS parts
+ * (large arrays, full batches) three of them would idle and every thread takes
+ * a baseline (one part each, 110 units of 256 stations x 500 sources: a batch
+ * of 427 -> 407 us; 40 of 512 x 500: 585 -> 530 us). */
+constexpr int RED_PARTS = 8;
+template <int GROUPS> constexpr int RED_Q = 256 / GROUPS;
 
-template <typename FP, class TL>
+template <typename FP, class TL, int GROUPS>
 __device__ __forceinline__ void reduce_row(int N, int p, int q0, int tiles,
         int parts, int use_casa, const float* partial,
         const unsigned int* cmax, const double* st_uvw, double uv_min,
         double uv_max, int offset_out, Cplx<FP>* vis,
-        double (*sums)[8][RED_Q])
+        double (*sums)[8][64])
 {
-    constexpr int TP = TL::TP, TQ = TL::TQ, TW = TL::TW;
-    const int lane = threadIdx.x % RED_Q, quarter = threadIdx.x / RED_Q;
+    static_assert(GROUPS == 1 || GROUPS == 4, "sums holds 3 x 8 x 64");
+    constexpr int TP = TL::TP, TQ = TL::TQ, TW = TL::TW, Q = RED_Q<GROUPS>;
+    const int lane = threadIdx.x % Q, group = threadIdx.x / Q;
     const int q = q0 + lane;
     const int ib = p / TP, pl = p - ib * TP;
     const int t0 = row_first_tile(ib, N, TP, TQ);
@@ -956,10 +961,10 @@ __device__ __forceinline__ void reduce_row(int N, int p, int q0, int tiles,
     {
         const int jb = q / TQ, ql = q - jb * TQ;
         const int t = t0 + jb;
-        const int per = (parts + 3) / 4;
-        const int k1 = min(parts, (quarter + 1) * per);
+        const int per = (parts + GROUPS - 1) / GROUPS;
+        const int k1 = min(parts, (group + 1) * per);
 #pragma unroll 2
-        for (int k = quarter * per; k < k1; ++k)
+        for (int k = group * per; k < k1; ++k)
         {
             const float* b = partial + ((size_t) k * tiles + t) *
                     (size_t) (2 * TP * TW) + (size_t) pl * TW + ql;
@@ -971,24 +976,28 @@ __device__ __forceinline__ void reduce_row(int N, int p, int q0, int tiles,
             }
         }
     }
-    if (quarter > 0)
+    if constexpr (GROUPS > 1)
     {
-#pragma unroll
-        for (int ik = 0; ik < 4; ++ik)
+        if (group > 0)
         {
-            sums[quarter - 1][ik][lane] = vr[ik];
-            sums[quarter - 1][4 + ik][lane] = vi[ik];
+#pragma unroll
+            for (int ik = 0; ik < 4; ++ik)
+            {
+                sums[group - 1][ik][lane] = vr[ik];
+                sums[group - 1][4 + ik][lane] = vi[ik];
+            }
         }
+        __syncthreads();
+        if (group > 0) return;
     }
-    __syncthreads();
-    if (quarter > 0 || q >= p) return;
+    if (q >= p) return;
     /* uv filter on the baseline length in wavelengths. */
     const double du = gld(st_uvw + 3 * p) - gld(st_uvw + 3 * q);
     const double dv = gld(st_uvw + 3 * p + 1) - gld(st_uvw + 3 * q + 1);
     const double len = sqrt(du * du + dv * dv);
     if (len < uv_min || len > uv_max) return;
 #pragma unroll
-    for (int h = 0; h < 3; ++h)
+    for (int h = 0; h < GROUPS - 1; ++h)
 #pragma unroll
         for (int ik = 0; ik < 4; ++ik)
         {
@@ -1109,16 +1118,16 @@ __global__ void fact_stations_kernel(int n, const FP* u, const FP* v,
     }
 }
 
-template <typename FP, class TL>
+template <typename FP, class TL, int GROUPS>
 __global__ __launch_bounds__(256)
 void fact_reduce_kernel(int N, int num_tiles, int num_parts, int use_casa,
         const float* partial, const unsigned int* cmax, const double* st_uvw,
         double uv_min, double uv_max, int offset_out, Cplx<FP>* vis)
 {
-    __shared__ double sums[3][8][RED_Q];
-    const int p = blockIdx.x, q0 = blockIdx.y * RED_Q;
+    __shared__ double sums[GROUPS > 1 ? 3 : 1][8][64];
+    const int p = blockIdx.x, q0 = blockIdx.y * RED_Q<GROUPS>;
     if (q0 >= p) return;
-    reduce_row<FP, TL>(N, p, q0, num_tiles, num_parts, use_casa, partial,
+    reduce_row<FP, TL, GROUPS>(N, p, q0, num_tiles, num_parts, use_casa, partial,
             cmax, st_uvw, uv_min, uv_max, offset_out, vis, sums);
 }
 
@@ -1270,16 +1279,24 @@ template <typename FP, class TL>
 __global__ __launch_bounds__(256)
 void fact_batch_reduce_kernel(const BatchHeader* H, const UnitDesc* D)
 {
-    __shared__ double sums[3][8][RED_Q];
+    __shared__ double sums[3][8][64];
     const int N = H->num_stations, rows = H->num_units * N;
     for (int r = blockIdx.x; r < rows; r += gridDim.x)
     {
         const int u = r / N, p = r - u * N;
         const UnitDesc& d = D[u];
         if (d.num_parts == 0) continue;      /* no sources: untouched */
-        for (int q0 = 0; q0 < p; q0 += RED_Q)
+        if (d.num_parts < RED_PARTS)
         {
-            reduce_row<FP, TL>(N, p, q0, H->num_tiles, d.num_parts,
+            for (int q0 = 0; q0 < p; q0 += RED_Q<1>)
+                reduce_row<FP, TL, 1>(N, p, q0, H->num_tiles, d.num_parts,
+                        H->use_casa, d.partial, d.cmax, d.st, d.uv_min,
+                        d.uv_max, d.offset_out, (Cplx<FP>*) d.vis, sums);
+            continue;
+        }
+        for (int q0 = 0; q0 < p; q0 += RED_Q<4>)
+        {
+            reduce_row<FP, TL, 4>(N, p, q0, H->num_tiles, d.num_parts,
                     H->use_casa, d.partial, d.cmax, d.st, d.uv_min,
                     d.uv_max, d.offset_out, (Cplx<FP>*) d.vis, sums);
             __syncthreads();              /* sums is reused */
@@ -1445,7 +1462,6 @@ int fact_launch_shape(int dev, int precision, int mode, int use_casa,
     A.cmax = cmax;
     A.partial = partial;
     const dim3 grid(tiles, parts);
-    const dim3 rgrid(N, (N + RED_Q - 1) / RED_Q);
     mark(dev, 1, stream);
     if (mode == 1)
         hipLaunchKernelGGL((fact_xcorr_kernel<BodyB>), grid,
@@ -1457,14 +1473,22 @@ int fact_launch_shape(int dev, int precision, int mode, int use_casa,
     if (err != hipSuccess) return (int) err;
 
     mark(dev, 2, stream);
+#define FACT_REDUCE(FP, GROUPS) hipLaunchKernelGGL( \
+        (fact_reduce_kernel<FP, TL, GROUPS>), \
+        dim3(N, (N + RED_Q<GROUPS> - 1) / RED_Q<GROUPS>), dim3(256), 0, \
+        stream, N, tiles, parts, use_casa, partial, cmax, st, uv_min, uv_max, \
+        offset_out, (Cplx<FP>*) vis)
     if (precision == OSKAR_DOUBLE)
-        hipLaunchKernelGGL((fact_reduce_kernel<double, TL>), rgrid,
-                dim3(256), 0, stream, N, tiles, parts, use_casa, partial,
-                cmax, st, uv_min, uv_max, offset_out, (Cplx<double>*) vis);
+    {
+        if (parts < RED_PARTS) FACT_REDUCE(double, 1);
+        else FACT_REDUCE(double, 4);
+    }
     else
-        hipLaunchKernelGGL((fact_reduce_kernel<float, TL>), rgrid,
-                dim3(256), 0, stream, N, tiles, parts, use_casa, partial,
-                cmax, st, uv_min, uv_max, offset_out, (Cplx<float>*) vis);
+    {
+        if (parts < RED_PARTS) FACT_REDUCE(float, 1);
+        else FACT_REDUCE(float, 4);
+    }
+#undef FACT_REDUCE
     mark(dev, 3, stream);
     return (int) hipGetLastError();
 }

@@ -59,3 +59,13 @@ def test_units(hip, ns, nsrc, units, limit_mb):
             assert rel_rms(got[u], want) < 1e-5
         if units < 8:
             assert np.array_equal(got[k], one)
+
+
+@pytest.mark.parametrize("prec", ["f", "d"])
+@pytest.mark.parametrize("ns,nsrc", [(300, 20), (1100, 60)])
+def test_rows_of_few_parts(hip, prec, ns, nsrc):
+    """One call of one part: rows of up to five workgroups, a baseline per
+    thread (20 and 60 sources: 2e-5, as for other handfuls)."""
+    c = make_case(ns + nsrc, ns, nsrc)
+    want = oracle_direct(rounded(c, prec), 150e6)
+    assert rel_rms(run(c, prec, 0, 150e6), want) < 2e-5
