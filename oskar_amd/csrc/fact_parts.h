@@ -31,7 +31,12 @@ inline long long part_tiles(int num_stations)
  *    written and read (4 TB/s); least at sqrt(12.5 (S / 8) / tiles) parts,
  *    and no more than one round of workgroups.
  *  - Otherwise: as many parts as whole rounds hold (512 stations x 1M
- *    sources: 128 parts in 9 rounds instead of 123 in 8.65). */
+ *    sources: 128 parts in 9 rounds instead of 123 in 8.65).  Where those are
+ *    no more than parts of max_part, a short last part can end the last round
+ *    sooner than equal ones: it does if all work in full rounds and that part
+ *    take less than the rounds of equal parts (2048 x 20,000, 3 parts in 3.1
+ *    rounds: 3734 against 4005 us; 1500 x 40,000, 5 parts in 2.93: 3837
+ *    against 3786, equal). */
 inline int part_sources(int num_sources, int num_stations, int max_part,
         int unit)
 {
@@ -50,6 +55,10 @@ inline int part_sources(int num_sources, int num_stations, int max_part,
         const long long rounds = (tiles * least + PART_SLOTS - 1) /
                 PART_SLOTS;
         parts = std::max(least, PART_SLOTS * rounds / tiles);
+        const double last = (double) num_sources - (least - 1.0) * max_part;
+        if (parts == least && (double) tiles * num_sources / PART_SLOTS +
+                last < (double) rounds * ((double) num_sources / parts))
+            return max_part;
     }
     /* The parts are a grid's y. */
     parts = std::min(parts, std::max(least, 65535LL));
