@@ -172,6 +172,31 @@ __host__ __device__ inline int blocks_in_row(int N, bool casa, int ia,
     return a_last > 0 ? (a_last - 1) / BLOCK_B + 1 : 0;
 }
 
+/* Blocks of the rows before row ia: of every row but the last, 2 ia + 2, or
+ * in the CASA order the whole row's blocks less 2 ia. */
+__host__ __device__ inline int blocks_before(int N, bool casa, int ia)
+{
+    const int row = (N + BLOCK_B - 1) / BLOCK_B;
+    return casa ? ia * (row + 1 - ia) : ia * (ia + 1);
+}
+
+/* The row of a block of the list, by the root of blocks_before(), whose
+ * rounding is put right (a search row by row took 20 us of scalar code per
+ * workgroup at 3000 stations). */
+__host__ __device__ inline int block_row(int N, bool casa, int block)
+{
+    const float row = (float) ((N + BLOCK_B - 1) / BLOCK_B + 1);
+    int ia = casa ? (int) (0.5f * (row - sqrtf(fmaxf(row * row -
+            4.0f * (float) block, 0.0f)))) :
+            (int) (0.5f * (sqrtf(4.0f * (float) block + 1.0f) - 1.0f));
+#if defined(__HIP_DEVICE_COMPILE__)
+    ia = __builtin_amdgcn_readfirstlane(ia);
+#endif
+    while (ia > 0 && blocks_before(N, casa, ia) > block) --ia;
+    while (blocks_before(N, casa, ia + 1) <= block) ++ia;
+    return ia;
+}
+
 /* FP64 matrices without the Gaussian factor fit three waves per SIMD (168
  * VGPRs and 52 KB of LDS: 1.25 -> 1.19 ms for 255 stations x 10,007
  * sources); with it they would spill (30 x 277 sources: 21.7 -> 24.6 us). */
@@ -204,18 +229,11 @@ void xcorr_direct_kernel(XcorrArgs<FP> A, int blocks)
     const int xq = total / 8, xr = total % 8, xcd = wg % 8;
     const int item = xcd * xq + min(xcd, xr) + wg / 8;
     const int split = item / blocks;
-    int a0, b0;
-    {
-        int block = item % blocks, ia = 0, ib0 = 0;
-        for (;; ++ia)
-        {
-            const int c = blocks_in_row(N, A.use_casa != 0, ia, &ib0);
-            if (block < c) break;
-            block -= c;
-        }
-        a0 = ia * BLOCK_A;
-        b0 = (ib0 + block) * BLOCK_B;
-    }
+    const bool casa = A.use_casa != 0;
+    const int block = item % blocks, ia = block_row(N, casa, block);
+    const int a0 = ia * BLOCK_A;
+    const int b0 = (block - blocks_before(N, casa, ia)) * BLOCK_B +
+            (casa ? a0 : 0);
     const int tid = threadIdx.x;
     const int la = tid >> 3;
     /* Second stations lb and lb + 8: the eight lanes of a wave that share
