@@ -587,15 +587,30 @@ hipError_t launch_t(XcorrArgs<FP> A, hipStream_t stream, double* fixed)
     if (blocks == 0 || A.num_sources <= 0) return hipSuccess;
     /* Splits: about 12 rounds of four workgroups per CU, so that the last
      * round's idle time is small, with at least 8 tiles of sources each
-     * (the prologue and the partial sums cost about one), or one where that
-     * leaves the chip idle, and down to LEAST sources each while there is less
-     * than a round (30 stations x 277 sources in FP64: 8 workgroups of four
-     * tiles 80 us, 36 of one 21.6 us, 140 of 4 sources 17.7 us). */
-    int splits = (12 * 1024 + blocks - 1) / blocks;
-    const int max_splits = max(1, max(A.num_sources / (8 * G::TILE),
-            min((A.num_sources + G::LEAST - 1) / G::LEAST, 1024 / blocks)));
-    splits = max(1, min(splits, min(max_splits, 256)));
+     * (the prologue and the partial sums cost about one).  Where that leaves
+     * the chip idle, more while there is less than a round, down to LEAST
+     * sources each (30 stations x 277 sources in FP64: 8 workgroups of four
+     * tiles 80 us, 36 of one 21.6 us, 140 of 4 sources 17.7 us), as long as a
+     * split saves more than its partial sums cost: going from k - 1 to k
+     * saves `each` us per source / (k (k - 1)), a split's sums take their
+     * bytes at 1.1 TB/s (written scattered and read again), and the second
+     * kernel 3 us (512 x 20 FP32 matrices: 22 us as one split, 36 as two; 300
+     * x 32 FP64: 25, 23 as two, 36 as eight; 512 x 32: 32 and 50 as three). */
+    constexpr double each = MATRIX ? (sizeof(FP) == 8 ? 0.65 : 0.43) :
+            (sizeof(FP) == 8 ? 0.25 : 0.14);
+    constexpr int round = MATRIX && sizeof(FP) == 8 ? 768 : 1024;
     const size_t nb = (size_t) N * (N - 1) / 2;
+    const double sums = nb * G::NR * sizeof(double) / 1.1e6;
+    const double saved = each * A.num_sources;
+    int few = saved > 2.0 * (3.0 + 2.0 * sums) ?
+            (int) (0.5 + sqrt(saved / sums + 0.25)) : 1;
+    /* Whole units of LEAST sources, the nearest number per split. */
+    const int units = (A.num_sources + G::LEAST - 1) / G::LEAST;
+    const int unit_split = max(1, (2 * units + few) / (2 * few));
+    few = min((units + unit_split - 1) / unit_split, round / blocks);
+    int splits = (12 * 1024 + blocks - 1) / blocks;
+    const int max_splits = max(1, max(A.num_sources / (8 * G::TILE), few));
+    splits = max(1, min(splits, min(max_splits, 256)));
     /* One split writes vis directly and needs no partial sums. */
     splits = max(1, (int) min((size_t) splits,
             XCORR_PARTIAL_BYTES / (nb * G::NR * sizeof(double))));

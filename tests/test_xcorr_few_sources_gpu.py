@@ -34,3 +34,13 @@ def compare(prec, casa, gauss, matrix, ns, nsrc, bs):
                                 3001])
 def test_station_blocks(hip, ns, casa):
     compare("d", casa, 1, 0, ns, 2 if ns > 2000 else 5, 0)
+
+
+@pytest.mark.parametrize("prec", ["f", "d"])
+@pytest.mark.parametrize("matrix", [0, 1])
+@pytest.mark.parametrize("ns,nsrc", [(512, 20), (300, 33), (300, 100),
+                                     (200, 64), (101, 131), (64, 33)])
+def test_splits(hip, prec, matrix, ns, nsrc):
+    """One split where its partial sums would cost more than they save,
+    several with remainders otherwise."""
+    compare(prec, ns % 2, 1, matrix, ns, nsrc, 1)
