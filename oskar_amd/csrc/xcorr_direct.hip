@@ -369,6 +369,14 @@ void xcorr_direct_kernel(XcorrArgs<FP> A, int blocks)
 #pragma unroll
             for (int r = 0; r < NR; ++r) t[k][r] = (FP) 0;
 
+        /* The extended sources of the tile, one bit each: a branch per source
+         * that waits for no LDS read. */
+        uint64_t extended = 0;
+        if (GAUSS)
+        {
+            static_assert(TILE <= 64, "a bit per source");
+            extended = __ballot(lane < TILE && sExt[lane % TILE].w != (FP) 0);
+        }
         /* Two sources per iteration in the FP32 scalar form; one in the
          * matrix form (more registers would leave three waves per SIMD)
          * and in FP64. */
@@ -384,9 +392,9 @@ void xcorr_direct_kernel(XcorrArgs<FP> A, int blocks)
             FP sm[2] = {(FP) 1, (FP) 1};
             if (GAUSS)
             {
-                const Quad<FP> e = sExt[s];
-                if (__any(e.w != (FP) 0))
+                if (extended >> s & 1u)
                 {
+                    const Quad<FP> e = sExt[s];
 #pragma unroll
                     for (int k = 0; k < 2; ++k)
                         sm[k] = gauss_exp(e.x * bt[k].uu2 +
