@@ -1,7 +1,7 @@
 /*
  * Direct cross-correlation kernel for gfx950 (the "plain" visibility path)
  * with a Gaussian or smearing factor per baseline; without one the sum is a
- * matrix product (xcorr_product.hip).
+ * matrix product (xcorr_product.hip), but for few sources.
  *
  * Computes, for every baseline (p > q) outside the uv filter,
  *     V_pq += sum_s smear_s(pq) * J_first(s) B_s J_second(s)^H
@@ -604,8 +604,11 @@ hipError_t launch_t(XcorrArgs<FP> A, hipStream_t stream, double* fixed)
      * bytes at 1.1 TB/s (written scattered and read again), and the second
      * kernel 3 us (512 x 20 FP32 matrices: 22 us as one split, 36 as two; 300
      * x 32 FP64: 25, 23 as two, 36 as eight; 512 x 32: 32 and 50 as three). */
-    constexpr double each = MATRIX ? (sizeof(FP) == 8 ? 0.65 : 0.43) :
-            (sizeof(FP) == 8 ? 0.25 : 0.14);
+    constexpr double each = GAUSS || BS || TS ?
+            (MATRIX ? (sizeof(FP) == 8 ? 0.65 : 0.43) :
+            (sizeof(FP) == 8 ? 0.25 : 0.14)) :
+            (MATRIX ? (sizeof(FP) == 8 ? 0.45 : 0.3) :
+            (sizeof(FP) == 8 ? 0.1 : 0.08));
     constexpr int round = MATRIX && sizeof(FP) == 8 ? 768 : 1024;
     const size_t nb = (size_t) N * (N - 1) / 2;
     const double sums = nb * G::NR * sizeof(double) / 1.1e6;
@@ -654,17 +657,34 @@ hipError_t launch_t(XcorrArgs<FP> A, hipStream_t stream, double* fixed)
     return hipGetLastError();
 }
 
+/* Whether the per-baseline kernel sums few sources sooner than the product,
+ * whose workgroups are few (64 x 64 stations of scalars each) and take long
+ * stages.  Product -> per baseline, us, FP32: scalars 200 stations x 16 sources
+ * 17.6 -> 12, 512 x 64 21 -> 12.5, 512 x 128 21 -> 18.5, 1000 x 64 23 -> 19
+ * (but 700 x 96 23 -> 22 and 1100 x 64 24 -> 24); matrices 200 x 16 17 -> 12,
+ * 300 x 32 20 -> 17, 3000 x 16 175 -> 124 (but 1100 x 24 51 -> 50, 200 x 48
+ * 19 -> 19). */
+template <bool MATRIX> bool few_sources(int num_sources, int num_stations)
+{
+    if (MATRIX)
+        return num_sources <= 16 || (num_sources <= 32 && num_stations <= 512);
+    return (num_sources <= 64 && num_stations <= 1024) ||
+            (num_sources <= 128 && num_stations <= 512);
+}
+
 template <typename FP, bool MATRIX>
 hipError_t dispatch(const XcorrArgs<FP>& A, bool gauss, bool bs, bool ts,
         hipStream_t s, double* fixed)
 {
-    /* No factor depends on the baseline: one matrix product. */
-    if (!gauss && !bs && !ts)
+    /* No factor depends on the baseline: one matrix product, but for few
+     * sources. */
+    if (!gauss && !bs && !ts && !few_sources<MATRIX>(A.num_sources,
+            A.num_stations))
         return xcorr_product_launch<FP, MATRIX>(A, s, fixed);
 #define XC_CASE(G_, B_, T_) if (gauss == G_ && bs == B_ && ts == T_) \
         return launch_t<FP, MATRIX, G_, B_, T_>(A, s, fixed);
-    XC_CASE(false, false, true)  XC_CASE(false, true, false)
-    XC_CASE(false, true, true)
+    XC_CASE(false, false, false) XC_CASE(false, false, true)
+    XC_CASE(false, true, false)  XC_CASE(false, true, true)
     XC_CASE(true, false, false)  XC_CASE(true, false, true)
     XC_CASE(true, true, false)   XC_CASE(true, true, true)
 #undef XC_CASE

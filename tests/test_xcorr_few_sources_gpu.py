@@ -44,3 +44,42 @@ def test_splits(hip, prec, matrix, ns, nsrc):
     """One split where its partial sums would cost more than they save,
     several with remainders otherwise."""
     compare(prec, ns % 2, 1, matrix, ns, nsrc, 1)
+
+
+@pytest.mark.parametrize("prec", ["f", "d"])
+@pytest.mark.parametrize("matrix,ns,nsrc", [
+    (1, 513, 16), (1, 513, 17), (1, 512, 32), (1, 512, 33), (1, 3, 32),
+    (0, 1024, 64), (0, 1025, 64), (0, 513, 65), (0, 512, 128), (0, 512, 129),
+    (0, 2, 128)])
+def test_kernel_of_few_sources(hip, prec, matrix, ns, nsrc):
+    """Both sides of the rule that leaves few sources without factors to the
+    per-baseline kernel."""
+    for casa in (0, 1):
+        compare(prec, casa, 0, matrix, ns, nsrc, 0)
+
+
+@pytest.mark.parametrize("prec", ["f", "d"])
+@pytest.mark.parametrize("matrix", [0, 1])
+@pytest.mark.parametrize("ns", [2, 3, 8, 9, 16, 17, 31, 32, 33, 48, 49, 64,
+                                65, 97])
+def test_edges_of_the_product(hip, prec, matrix, ns):
+    """The product's tiles and remainders of its stages, with more sources
+    than the per-baseline kernel takes."""
+    compare(prec, ns % 2, 0, matrix, ns, 129 + 5 * (ns % 13), 0)
+
+
+@pytest.mark.parametrize("prec", ["f", "d"])
+def test_infinite_scalars_of_the_product(hip, prec):
+    """An infinite value in the last source (the one that pads a stage)
+    leaves every baseline of the other stations unchanged."""
+    ns, nsrc, bad = 50, 161, 20
+    g = rounded(random_sky(np.random.default_rng(4), ns, nsrc), prec)
+    want = gpu_cross_correlate(prec, 0, 0, 0, g, 0, 0).reshape(-1, 2)
+    j = g["jones_s"].copy().reshape(ns, nsrc, 2)
+    j[bad, -1, :] = np.inf
+    g["jones_s"] = j.ravel()
+    got = gpu_cross_correlate(prec, 0, 0, 0, g, 0, 0).reshape(-1, 2)
+    q, p = np.triu_indices(ns, 1)
+    other = (p != bad) & (q != bad)
+    assert np.array_equal(got[other], want[other])
+    assert not np.any(np.isfinite(got[~other]).all(axis=-1))
