@@ -528,22 +528,20 @@ __device__ __forceinline__ bool acc_place(int N, int p0, int q0, int rf,
     return *p < N && *p > *q;
 }
 
-/* vis += (re, im) of element (i, k) of baseline (p, q), inside the uv
- * filter. */
+/* The two reals of vis that element (i, k) of baseline (p, q) adds to, or
+ * NULL outside the uv filter. */
 template <typename FP, bool MATRIX>
-__device__ __forceinline__ void add_to_vis(const XcorrArgs<FP>& A, int p,
-        int q, int i, int k, double re, double im)
+__device__ __forceinline__ FP* vis_place(const XcorrArgs<FP>& A, int p, int q,
+        int i, int k)
 {
     using G = Geo<FP, MATRIX>;
     BaselineTerms<FP, false> t;
     t.init(A, p, q);
-    if (t.uv_len < A.uv_min || t.uv_len > A.uv_max) return;
+    if (t.uv_len < A.uv_min || t.uv_len > A.uv_max) return nullptr;
     /* CASA: element [i][k] = conj(V[k][i]). */
     const int el = MATRIX ? (A.use_casa ? 2 * k + i : 2 * i + k) : 0;
-    FP* o = (FP*) A.vis + ((size_t) A.offset_out +
+    return (FP*) A.vis + ((size_t) A.offset_out +
             baseline_index(A.num_stations, p, q)) * G::NR + 2 * el;
-    o[0] += (FP) re;
-    o[1] += (FP) (A.use_casa ? -im : im);
 }
 
 template <typename FP, bool MATRIX>
@@ -633,26 +631,53 @@ void xcorr_product_kernel(XcorrArgs<FP> A, int tiles)
         __syncthreads();
     }
     if (!role.active) return;
-    double* part = A.num_splits == 1 ? nullptr : A.partial +
-            (((size_t) split * tiles + tile) * 4 + wave) * WAVE_VALUES +
-            lane;
-#pragma unroll
-    for (int i = 0; i < 16; ++i)
+    if (A.num_splits > 1)
     {
-        const int r = i / 8, c = (i / 4) % 2, v = i % 4;
-        const double vr = tot.re[r][c][v], vi = tot.im[r][c][v];
-        if (part)
+        double* part = A.partial +
+                (((size_t) split * tiles + tile) * 4 + wave) * WAVE_VALUES +
+                lane;
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
         {
-            part[(i * 2 + 0) * 64] = vr;
-            part[(i * 2 + 1) * 64] = vi;
+            const int r = i / 8, c = (i / 4) % 2, v = i % 4;
+            part[(i * 2 + 0) * 64] = tot.re[r][c][v];
+            part[(i * 2 + 1) * 64] = tot.im[r][c][v];
         }
-        else
+        return;
+    }
+    /* One split: vis itself, eight values at a time, all loaded before the
+     * first is stored (a load and a store at a time are one chain: 3000
+     * stations x 16 sources of FP64 matrices 290 -> 255 us, 512 x 60 38.2 ->
+     * 36.6).  Through the LDS to consecutive accesses it was 10 % slower:
+     * every lane then has the terms of twice as many baselines to form. */
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+    {
+        FP* at[8];
+        FP old[8][2];
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
         {
             int p, q, ei, ek;
-            if (acc_place<FP, MATRIX>(N, wp0, wq0, r, c, v, lane, &p, &q,
-                    &ei, &ek))
-                add_to_vis<FP, MATRIX>(A, p, q, ei, ek, vr, vi);
+            at[j] = acc_place<FP, MATRIX>(N, wp0, wq0, h, j / 4, j % 4,
+                    lane, &p, &q, &ei, &ek) ?
+                    vis_place<FP, MATRIX>(A, p, q, ei, ek) : nullptr;
         }
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (at[j])
+            {
+                old[j][0] = at[j][0];
+                old[j][1] = at[j][1];
+            }
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (at[j])
+            {
+                const double im = tot.im[h][j / 4][j % 4];
+                at[j][0] = old[j][0] + (FP) tot.re[h][j / 4][j % 4];
+                at[j][1] = old[j][1] + (FP) (A.use_casa ? -im : im);
+            }
     }
 }
 
@@ -708,7 +733,12 @@ void xcorr_product_reduce_kernel(XcorrArgs<FP> A, int tiles)
     if (acc_place<FP, MATRIX>(N, ib * G::BST + role.wp * G::WST,
             jb * G::BST + role.wq * G::WST, reg >> 3, (reg >> 2) & 1,
             reg & 3, lane, &p, &q, &i, &k))
-        add_to_vis<FP, MATRIX>(A, p, q, i, k, re, im);
+    {
+        FP* o = vis_place<FP, MATRIX>(A, p, q, i, k);
+        if (!o) return;
+        o[0] += (FP) re;
+        o[1] += (FP) (A.use_casa ? -im : im);
+    }
 }
 
 } /* namespace */
