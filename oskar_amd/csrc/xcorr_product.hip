@@ -683,15 +683,18 @@ void xcorr_product_kernel(XcorrArgs<FP> A, int tiles)
 
 /* Adds the splits in a fixed order and scatters the sums to vis.
  * Workgroup (x, y): accumulator register x = (rf, cf, v) of sub-tile y; its
- * four waves add a quarter of the splits each (consecutive lanes on
+ * GROUPS waves add a share of the splits each (consecutive lanes on
  * consecutive partials; the partials of all waves that share the sub-tile),
- * the quarters are then added in order. */
-template <typename FP, bool MATRIX>
-__global__ __launch_bounds__(NT)
+ * the shares are then added in order.  4 waves; 16 where there are few
+ * sub-tiles, whose many splits (hundreds, of up to four waves each) would be
+ * long chains on a chip that is idle (2 stations x 100,000 FP32 scalars 62 ->
+ * 58 us, 64 x 2,000 in FP64 20 -> 18). */
+template <typename FP, bool MATRIX, int GROUPS>
+__global__ __launch_bounds__(64 * GROUPS)
 void xcorr_product_reduce_kernel(XcorrArgs<FP> A, int tiles)
 {
     using G = Geo<FP, MATRIX>;
-    __shared__ double sums[3][2][64];
+    __shared__ double sums[GROUPS - 1][2][64];
     const int N = A.num_stations;
     const int tile = blockIdx.y / 4, u = blockIdx.y % 4;
     int ib, jb;
@@ -700,31 +703,31 @@ void xcorr_product_reduce_kernel(XcorrArgs<FP> A, int tiles)
             true);
     if (u >= role.live) return;
     const int reg = blockIdx.x;                 /* (rf * 2 + cf) * 4 + v */
-    const int lane = threadIdx.x & 63, quarter = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, group = threadIdx.x >> 6;
     const size_t stride = (size_t) tiles * 4 * WAVE_VALUES;
     const double* part = A.partial + ((size_t) tile * 4 + u) * WAVE_VALUES +
             (size_t) reg * 128 + lane;
-    const int per = (A.num_splits + 3) / 4;
-    const int k1 = min(A.num_splits, (quarter + 1) * per);
+    const int per = (A.num_splits + GROUPS - 1) / GROUPS;
+    const int k1 = min(A.num_splits, (group + 1) * per);
     double re = 0.0, im = 0.0;
     for (int h = 0; h < role.step; ++h)
     {
 #pragma unroll 8
-        for (int s = quarter * per; s < k1; ++s)
+        for (int s = group * per; s < k1; ++s)
         {
             re += part[s * stride];
             im += part[s * stride + 64];
         }
         part += (size_t) role.live * WAVE_VALUES;
     }
-    if (quarter > 0)
+    if (group > 0)
     {
-        sums[quarter - 1][0][lane] = re;
-        sums[quarter - 1][1][lane] = im;
+        sums[group - 1][0][lane] = re;
+        sums[group - 1][1][lane] = im;
     }
     __syncthreads();
-    if (quarter > 0) return;
-    for (int h = 0; h < 3; ++h)
+    if (group > 0) return;
+    for (int h = 0; h < GROUPS - 1; ++h)
     {
         re += sums[h][0][lane];
         im += sums[h][1][lane];
@@ -788,8 +791,13 @@ hipError_t xcorr_product_launch(XcorrArgs<FP> A, hipStream_t stream,
             dim3((unsigned) (tiles * splits)), dim3(NT), 0, stream, A, tiles);
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess || splits == 1) return err;
-    hipLaunchKernelGGL((xcorr_product_reduce_kernel<FP, MATRIX>),
-            dim3(16, (unsigned) (tiles * 4)), dim3(NT), 0, stream, A, tiles);
+    const dim3 grid(16, (unsigned) (tiles * 4));
+    if (tiles <= 3)
+        hipLaunchKernelGGL((xcorr_product_reduce_kernel<FP, MATRIX, 16>),
+                grid, dim3(64 * 16), 0, stream, A, tiles);
+    else
+        hipLaunchKernelGGL((xcorr_product_reduce_kernel<FP, MATRIX, 4>),
+                grid, dim3(64 * 4), 0, stream, A, tiles);
     return hipGetLastError();
 }
 

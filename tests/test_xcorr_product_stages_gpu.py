@@ -103,3 +103,24 @@ def test_pairs_of_stages(hip, prec, matrix, ns, nsrc, splits, pairs):
         tol = 2 * t * u * mag + 2 * u * (np.abs(init.reshape(-1, nr)) +
                                          np.abs(want))
         assert np.all(err <= tol), np.max(err / tol)
+
+
+@pytest.mark.parametrize("prec", ["f", "d"])
+@pytest.mark.parametrize("matrix", [0, 1])
+@pytest.mark.parametrize("ns,nsrc", [(2, 20001), (5, 6007), (17, 6007),
+                                     (33, 5003), (64, 3001), (65, 3001),
+                                     (96, 2500), (97, 2500)])
+def test_many_splits_of_few_stations(hip, prec, matrix, ns, nsrc):
+    """Up to three tiles: hundreds of splits, each the sum of up to four
+    waves, added by 16 waves; more tiles by four."""
+    g = rounded(random_sky(np.random.default_rng(ns + nsrc), ns, nsrc), prec)
+    u = 2.0 ** (-53 if prec == "d" else -24)
+    nr = 8 if matrix else 2
+    for casa in (0, 1):
+        got = gpu_cross_correlate(prec, casa, 0, matrix, g, 0, 0).reshape(
+            -1, nr)
+        want, mag = product(g, ns, nsrc, matrix, casa)
+        t = (16 if matrix else 4) * (nsrc if prec == "d" else 32) + 8
+        err = np.abs(got - want)
+        tol = 2 * t * u * mag + 2 * u * np.abs(want)
+        assert np.all(err <= tol), np.max(err / tol)
