@@ -55,13 +55,12 @@ void oskar_cross_correlate(
  * device memory: code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc.  Arguments, checks, errors and results
  * as oskar_cross_correlate(); the split-source partial sums go to a fixed
- * 256 MiB array that every device holds until the process ends, instead of
- * a workspace the library allocates.  No input is rejected for its size:
- * when the partials of the usual split count do not fit, the sources are
- * split fewer times (down to one split, which adds to vis directly and
- * uses no scratch), so results then differ from oskar_cross_correlate()'s
- * by the FP64 summation order only.  Up to 512 stations the split count,
- * and so every result bit, is that of oskar_cross_correlate().  Every call
+ * 256 MiB array, which a device holds from the first call until the process
+ * ends, instead of a workspace the library allocates.  No input is rejected
+ * for its size: when the partials of the usual split count do not fit, the
+ * sources are split fewer times (down to one split, which adds to vis
+ * directly and uses no scratch).  oskar_cross_correlate()'s workspace is no
+ * larger, so the split count, and every result bit, is the same.  Every call
  * on one device shares that device's array: calls that overlap on one
  * device (two streams or two host threads) race and must be serialised by
  * the caller.

@@ -52,21 +52,12 @@
 #include <math.h>
 #include <stdint.h>
 
-#include <mutex>
-
 #include "device_common.h"
 #include "private.h"
 #include "workspace.h"
 #include "xcorr_common.h"
 
 using namespace oskar_amd;
-
-/* Split partials of the allocation-free entry point: a fixed array in
- * every device's code object.  Host code never passes this name to a
- * kernel: it is a host-side stand-in, not a device address; the device
- * address comes from hipGetSymbolAddress (scratch_address below). */
-static __device__ __align__(256)
-        double scratch[XCORR_PARTIAL_BYTES / sizeof(double)];
 
 namespace {
 
@@ -556,31 +547,6 @@ void* workspace_get(size_t bytes, hipStream_t stream, hipError_t* err)
     return ws_acquire(WS_XCORR_SPLIT, dev, stream, bytes, err);
 }
 
-/* Device address of `scratch` on the current device, looked up once per
- * device (with that device current) and kept. */
-constexpr int MAX_DEVICES = 64;
-std::mutex g_scratch_lock;
-void* g_scratch_ptr[MAX_DEVICES];
-
-hipError_t scratch_address(double** out)
-{
-    int dev = 0;
-    hipError_t err = hipGetDevice(&dev);
-    if (err != hipSuccess) return err;
-    if (dev < 0 || dev >= MAX_DEVICES) return hipErrorInvalidDevice;
-    std::lock_guard<std::mutex> guard(g_scratch_lock);
-    if (!g_scratch_ptr[dev])
-    {
-        void* p = nullptr;
-        err = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-        if (err != hipSuccess) return err;
-        if (!p) return hipErrorInvalidSymbol;
-        g_scratch_ptr[dev] = p;
-    }
-    *out = (double*) g_scratch_ptr[dev];
-    return hipSuccess;
-}
-
 /* fixed: the device's scratch array (allocation-free entry point); NULL:
  * the per-stream workspace. */
 template <typename FP, bool MATRIX, bool GAUSS, bool BS, bool TS>
@@ -731,7 +697,7 @@ hipError_t build_and_launch(int matrix, const oskar_XcorrParams* p,
     double* fixed = nullptr;
     if (no_alloc)
     {
-        const hipError_t err = scratch_address(&fixed);
+        const hipError_t err = xcorr_scratch(&fixed);
         if (err != hipSuccess) return err;
     }
     if (matrix)
