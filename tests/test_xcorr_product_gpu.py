@@ -1,8 +1,11 @@
-"""The matrix-core product of the direct correlator (point sources without
-smearing): sizes at the edges of its tiles (32 stations of matrices or 64 of
-scalars per workgroup, halves of those per wave, 16 rows per MFMA block), of
-its source stages (8 or 16 k-steps) and of its pipeline (pairs of stages),
-one split and many.
+"""The direct correlator for point sources without smearing: sizes at the
+edges of the matrix-core product's tiles (32 stations of matrices or 64 of
+scalars per workgroup, halves of those per wave, 16 rows per MFMA block) and
+of its source stages (8 or 16 k-steps), one split and many, and of the
+per-baseline kernel, which takes up to 32 sources of matrices and 128 of
+scalars on these arrays.  The product's pipeline (pairs of full stages) is in
+test_xcorr_product_stages_gpu, its edges with more sources in
+test_xcorr_few_sources_gpu.
 
 Tolerance: a value is a sum of T products of reals (T = 16 per source for
 matrices: 2 x 2 complex products on each of J B and M J^H; 4 for scalars),
@@ -91,10 +94,11 @@ def test_infinite_values_stay_with_their_station(hip, prec, matrix):
 
 @pytest.mark.parametrize("prec", ["f", "d"])
 @pytest.mark.parametrize("matrix", [0, 1])
-def test_jones_aligned_to_a_real_only(hip, prec, matrix):
+@pytest.mark.parametrize("nsrc", [30, 50, 150])
+def test_jones_aligned_to_a_real_only(hip, prec, matrix, nsrc):
     """The raw-pointer entry points take Jones arrays with the alignment of
-    one real."""
-    ns, nsrc = 40, 50
+    one real, in both kernels."""
+    ns = 40
     rng = np.random.default_rng(5)
     g = rounded(random_sky(rng, ns, nsrc), prec)
     P = OSKAR_DOUBLE if prec == "d" else OSKAR_SINGLE

@@ -6,7 +6,7 @@ Checked against oskar_cross_correlate on the same inputs, on two calls in a
 row, the second with a smaller input (the array keeps the first call's
 partials, which must not leak into the second's result):
   1. 512 stations x 3,000 sources, FP64 matrix Jones, Gaussian sources,
-     bandwidth and time smearing (8 source splits, which fill the 64 MiB
+     bandwidth and time smearing (23 source splits, 193 MB of the 256 MiB
      array): every value identical to oskar_cross_correlate's;
   2. 64 stations x 1,000 sources, FP32 scalar Jones, point sources: every
      value identical.
@@ -14,10 +14,13 @@ Both also accumulate into non-zero visibilities at an offset, and the
 check order and error codes of oskar_cross_correlate hold (an FP32 vis for
 FP64 Jones is a type mismatch, with vis untouched).
 
-At 600 stations the usual 6 splits of FP64 matrix partials (69 MB) do not
-fit the array, so the entry point splits the sources 5 times: the result
-equals oskar_cross_correlate's to the FP64 summation order (max difference
-below 1e-12 of the largest value).
+Where the usual splits' partials do not fit the array (nor the workspace of
+oskar_cross_correlate, which has the same limit), the sources are split fewer
+times: 1,000 stations x 1,700 sources of FP64 matrices with factors want 12
+splits of 32 MB, of which 8 fit; 1,000 x 7,200 point sources want 8 of 34.6 MB
+in the product, of which 7 fit, and 3,000 x 7,600 scalars 4 of 74 MB, of which
+3 fit.  Both entry points against the CPU oracle on the baselines of a
+dozen stations from all over the array.
 """
 import ctypes as C
 import math
@@ -30,6 +33,7 @@ from oskar_amd import capi, lib
 from oskar_amd.mem import (OSKAR_COMPLEX, OSKAR_DOUBLE, OSKAR_GPU,
                            OSKAR_MATRIX, OSKAR_SINGLE, Jones, Mem,
                            Telescope)
+from test_xcorr_gpu import oracle_run
 
 pytestmark = pytest.mark.gpu
 
@@ -103,11 +107,47 @@ def test_no_alloc_checks_like_oskar_cross_correlate(hip):
     assert np.array_equal(vis.numpy(), init.astype(np.float32))
 
 
-def test_no_alloc_fewer_splits_when_scratch_is_short(hip):
-    rng = np.random.default_rng(600)
-    print("no_alloc capped: 600 st x 2000 src FP64 matrix Gaussian BS TS",
-          flush=True)
-    got, want, init = both("d", 1, 1, inputs(rng, 600, 2000), 1, 1, 0)
-    scale = float(np.max(np.abs(want - init)))
-    assert scale > 0.0
-    assert float(np.max(np.abs(got - want))) <= 1e-12 * scale
+def splits_that_fit(gauss, matrix, ns, nsrc, prec):
+    """(wanted, fitting) splits by the launch rules."""
+    if gauss:
+        nb = ns * (ns - 1) // 2
+        rows = -(-ns // 32)
+        blocks = sum(((min(32 * i + 32, ns) - 2) // 16 + 1)
+                     for i in range(rows))
+        return (min(-(-12 * 1024 // blocks), nsrc // 128),
+                (256 << 20) // (nb * 64))
+    side = -(-ns // (32 if matrix else 64))
+    tiles = side * (side + 1) // 2
+    stages = -(-nsrc // ((8 if prec == "d" else 16) * (1 if matrix else 2)))
+    return (int(math.sqrt(stages / (0.026 * tiles))),
+            (256 << 20) // (tiles * 65536))
+
+
+@pytest.mark.parametrize("prec,gauss,matrix,ns,nsrc", [
+    ("d", 1, 1, 1000, 1700), ("d", 0, 1, 1000, 7200),
+    ("d", 0, 0, 3000, 7600)])
+def test_no_alloc_fewer_splits_when_scratch_is_short(hip, prec, gauss,
+                                                     matrix, ns, nsrc):
+    wanted, fit = splits_that_fit(gauss, matrix, ns, nsrc, prec)
+    assert 1 < fit < wanted
+    print("no_alloc capped:", prec, gauss, matrix, ns, nsrc, flush=True)
+    rng = np.random.default_rng(ns)
+    g = inputs(rng, ns, nsrc)
+    nr = 8 if matrix else 2
+    got, want, init = both(prec, gauss, matrix, g, gauss, gauss, 0)
+    assert np.array_equal(got, want)
+    # The oracle on a sub-array.
+    few = np.sort(rng.choice(ns - 2, 10, replace=False) + 1)
+    few = np.concatenate([[0], few, [ns - 1]])
+    h = dict(g)
+    for k in "uvwxy":
+        h[k] = g[k][few]
+    h["jones_m"] = g["jones_m"].reshape(ns, nsrc, 8)[few].ravel()
+    h["jones_s"] = g["jones_s"].reshape(ns, nsrc, 2)[few].ravel()
+    ref = oracle_run("d", 0, gauss, matrix, h, gauss, gauss).reshape(-1, nr)
+    q, p = np.triu_indices(few.size, 1)
+    p, q = few[p], few[q]
+    at = q * (ns - 1) - (q - 1) * q // 2 + p - q - 1
+    sums = (got - init).reshape(-1, nr)[at]
+    scale = float(np.max(np.abs(ref)))
+    assert float(np.max(np.abs(sums - ref))) <= 1e-12 * scale
