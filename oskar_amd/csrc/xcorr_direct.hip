@@ -1,7 +1,7 @@
 /*
  * Direct cross-correlation kernel for gfx950 (the "plain" visibility path)
  * with a Gaussian or smearing factor per baseline; without one the sum is a
- * matrix product (xcorr_product.hip), but for few sources.
+ * matrix product (xcorr_product.hip), but for few sources or stations.
  *
  * Computes, for every baseline (p > q) outside the uv filter,
  *     V_pq += sum_s smear_s(pq) * J_first(s) B_s J_second(s)^H
@@ -623,19 +623,23 @@ hipError_t launch_t(XcorrArgs<FP> A, hipStream_t stream, double* fixed)
     return hipGetLastError();
 }
 
-/* Whether the per-baseline kernel sums few sources sooner than the product,
- * whose workgroups are few (64 x 64 stations of scalars each) and take long
- * stages.  Product -> per baseline, us, FP32: scalars 200 stations x 16 sources
+/* Whether the per-baseline kernel is done with few sources or stations sooner
+ * than the product, whose workgroups are few (64 x 64 stations of scalars each)
+ * and take long stages.  Product -> per baseline, us, FP32: scalars 200 stations x 16 sources
  * 17.6 -> 12, 512 x 64 21 -> 12.5, 512 x 128 21 -> 18.5, 1000 x 64 23 -> 19
  * (but 700 x 96 23 -> 22 and 1100 x 64 24 -> 24); matrices 200 x 16 17 -> 12,
  * 300 x 32 20 -> 17, 3000 x 16 175 -> 124 (but 1100 x 24 51 -> 50, 200 x 48
- * 19 -> 19). */
-template <bool MATRIX> bool few_sources(int num_sources, int num_stations)
+ * 19 -> 19).  Arrays of up to 32 stations of scalars are a corner of one of its
+ * tiles: 2 x 100,000 FP32 58 -> 39, FP64 72 -> 47, 32 x 30,000 35 -> 26 and 47
+ * -> 29 (but 32 x 100,000 53 -> 57, 64 x 10,000 24 -> 24). */
+template <bool MATRIX> bool is_few(int num_sources, int num_stations)
 {
     if (MATRIX)
         return num_sources <= 16 || (num_sources <= 32 && num_stations <= 512);
     return (num_sources <= 64 && num_stations <= 1024) ||
-            (num_sources <= 128 && num_stations <= 512);
+            (num_sources <= 128 && num_stations <= 512) ||
+            (num_sources <= 65536 && num_stations <= 32) ||
+            (num_sources <= 131072 && num_stations <= 16);
 }
 
 template <typename FP, bool MATRIX>
@@ -643,8 +647,8 @@ hipError_t dispatch(const XcorrArgs<FP>& A, bool gauss, bool bs, bool ts,
         hipStream_t s, double* fixed)
 {
     /* No factor depends on the baseline: one matrix product, but for few
-     * sources. */
-    if (!gauss && !bs && !ts && !few_sources<MATRIX>(A.num_sources,
+     * sources or stations. */
+    if (!gauss && !bs && !ts && !is_few<MATRIX>(A.num_sources,
             A.num_stations))
         return xcorr_product_launch<FP, MATRIX>(A, s, fixed);
 #define XC_CASE(G_, B_, T_) if (gauss == G_ && bs == B_ && ts == T_) \

@@ -687,8 +687,8 @@ void xcorr_product_kernel(XcorrArgs<FP> A, int tiles)
  * consecutive partials; the partials of all waves that share the sub-tile),
  * the shares are then added in order.  4 waves; 16 where there are few
  * sub-tiles, whose many splits (hundreds, of up to four waves each) would be
- * long chains on a chip that is idle (2 stations x 100,000 FP32 scalars 62 ->
- * 58 us, 64 x 2,000 in FP64 20 -> 18). */
+ * long chains on a chip that is idle (64 stations x 2,000 FP64 scalars 20 ->
+ * 18 us, 30 x 2,000 matrices 23 -> 21). */
 template <typename FP, bool MATRIX, int GROUPS>
 __global__ __launch_bounds__(64 * GROUPS)
 void xcorr_product_reduce_kernel(XcorrArgs<FP> A, int tiles)

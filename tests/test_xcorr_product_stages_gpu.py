@@ -112,7 +112,8 @@ def test_pairs_of_stages(hip, prec, matrix, ns, nsrc, splits, pairs):
                                      (96, 2500), (97, 2500)])
 def test_many_splits_of_few_stations(hip, prec, matrix, ns, nsrc):
     """Up to three tiles: hundreds of splits, each the sum of up to four
-    waves, added by 16 waves; more tiles by four."""
+    waves, added by 16 waves; more tiles by four.  (Scalars of up to 32
+    stations take the per-baseline kernel.)"""
     g = rounded(random_sky(np.random.default_rng(ns + nsrc), ns, nsrc), prec)
     u = 2.0 ** (-53 if prec == "d" else -24)
     nr = 8 if matrix else 2
