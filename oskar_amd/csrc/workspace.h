@@ -4,8 +4,7 @@
  * streams do not share partial sums; calls on one stream are ordered by the
  * stream and reuse its buffer.  A buffer grows (hipFree, which waits for the
  * device, then hipMalloc) when a call needs more.  Buffers live until the
- * process ends, or until more than a thousand others have been used since
- * (streams that come and go).
+ * process ends: a captured graph may hold their addresses.
  */
 #ifndef OSKAR_AMD_WORKSPACE_H_
 #define OSKAR_AMD_WORKSPACE_H_

@@ -1,4 +1,6 @@
 /* Per-(kind, device, stream) device workspaces (see workspace.h). */
+#include <new>
+
 #include "workspace.h"
 
 namespace oskar_amd {
@@ -11,13 +13,10 @@ struct Entry
     hipStream_t stream;
     void* ptr;
     size_t size;
-    unsigned long long used;     /* when it was last acquired */
+    Entry* next;
 };
 
-constexpr int MAX_ENTRIES = 1024;
-Entry g_entries[MAX_ENTRIES];
-int g_count = 0;
-unsigned long long g_clock = 0;
+Entry* g_entries = nullptr;
 std::mutex g_lock;
 std::mutex g_launch_lock;
 
@@ -27,34 +26,20 @@ void* ws_acquire(int kind, int dev, hipStream_t stream, size_t bytes,
         hipError_t* err)
 {
     std::lock_guard<std::mutex> guard(g_lock);
-    Entry* e = nullptr;
-    for (int i = 0; i < g_count; ++i)
-    {
-        Entry& x = g_entries[i];
-        if (x.kind == kind && x.dev == dev && x.stream == stream)
-        {
-            e = &x;
-            break;
-        }
-    }
+    Entry* e = g_entries;
+    while (e && !(e->kind == kind && e->dev == dev && e->stream == stream))
+        e = e->next;
     if (!e)
     {
-        if (g_count < MAX_ENTRIES) e = &g_entries[g_count++];
-        else
+        e = new (std::nothrow) Entry{kind, dev, stream, nullptr, 0,
+                g_entries};
+        if (!e)
         {
-            /* The least recently used (hipFree waits for its device). */
-            e = &g_entries[0];
-            for (int i = 1; i < MAX_ENTRIES; ++i)
-                if (g_entries[i].used < e->used) e = &g_entries[i];
-            if (e->ptr) (void) hipFree(e->ptr);
+            *err = hipErrorOutOfMemory;
+            return nullptr;
         }
-        e->kind = kind;
-        e->dev = dev;
-        e->stream = stream;
-        e->ptr = nullptr;
-        e->size = 0;
+        g_entries = e;
     }
-    e->used = ++g_clock;
     if (e->size < bytes)
     {
         if (e->ptr) (void) hipFree(e->ptr);

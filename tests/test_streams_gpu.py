@@ -173,3 +173,26 @@ def test_two_threads(hip, which, own):
         for st in streams:
             if st:
                 _stream_destroy(st)
+
+
+def test_more_streams_than_ever(hip):
+    """1,100 streams, one after another: none is refused a buffer."""
+    a = Acorr(3, 5, 300)
+    want = serial([a], "acorr")
+    s = C.c_int(0)
+    streams = [_stream_create() for _ in range(1100)]
+    try:
+        for st in streams:
+            a.clear()
+            sync_check("clear")
+            lib.oskar_hip_set_stream(st)
+            a.run(s)
+            check_status(s, "acorr")
+            lib.oskar_hip_set_stream(None)
+            sync_check("acorr")
+        same([a], want)
+    finally:
+        lib.oskar_hip_set_stream(None)
+        sync_check("acorr")
+        for st in streams:
+            _stream_destroy(st)
