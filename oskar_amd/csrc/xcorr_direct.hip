@@ -41,11 +41,11 @@
  * Bound: vector instructions.  FP32 matrices with all factors take 82 per
  * evaluation, 40 of them the contraction (163 with library sines, divisions
  * and both sinc branches, 92 with the sinc's last form past MID), and the
- * vector unit is busy throughout: 512 stations x 20,000 sources 10.86 ->
- * 5.21 ms (5.73 without the form up to WIDE).  FP64 with both smearings
- * takes 82 (565), vector unit 64 % busy at three waves per SIMD: 255 x
- * 10,007 sources 4.69 -> 1.19 ms.  Scalars with bandwidth smearing in FP32,
- * 351 x 50,001: 2.51 -> 1.35 ms (1.43 with the flux in an LDS
+ * vector unit is busy throughout: 512 stations x 20,000 sources 10.8 ->
+ * 5.2 ms (5.73 without the form up to WIDE).  FP64 with both smearings
+ * takes 82 (565), vector unit 74 % busy at three waves per SIMD: 255 x
+ * 10,007 sources 4.62 -> 1.20 ms.  Scalars with bandwidth smearing in FP32,
+ * 351 x 50,001: 2.52 -> 1.37 ms (1.43 with the flux in an LDS
  * read of its own: LDS was active 71 % of the time).
  */
 #include <hip/hip_runtime.h>
