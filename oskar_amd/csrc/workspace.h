@@ -32,7 +32,11 @@ enum WorkspaceKind
 void* ws_acquire(int kind, int dev, hipStream_t stream, size_t bytes,
         hipError_t* err);
 
-/* The same on the current device. */
+/* The same on the current device, for kernels whose calls may be captured on
+ * a stream that has not run them before: under capture, where nothing can be
+ * allocated, the buffer is one that all captures of the device share, made by
+ * an earlier call of at least this size on any stream, and never freed or
+ * moved, since graphs hold its address. */
 void* ws_acquire_here(int kind, hipStream_t stream, size_t bytes,
         hipError_t* err);
 

@@ -17,6 +17,17 @@ struct Entry
 };
 
 Entry* g_entries = nullptr;
+
+/* Buffers for captured calls, newest first. */
+struct Capture
+{
+    int kind, dev;
+    void* ptr;
+    size_t size;
+    Capture* next;
+};
+
+Capture* g_captures = nullptr;
 std::mutex g_lock;
 std::mutex g_launch_lock;
 
@@ -62,8 +73,36 @@ void* ws_acquire_here(int kind, hipStream_t stream, size_t bytes,
 {
     int dev = 0;
     *err = hipGetDevice(&dev);
-    return *err == hipSuccess ? ws_acquire(kind, dev, stream, bytes, err) :
-            nullptr;
+    if (*err != hipSuccess) return nullptr;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (stream)
+    {
+        *err = hipStreamIsCapturing(stream, &capture);
+        if (*err != hipSuccess) return nullptr;
+    }
+    Capture* c = nullptr;
+    {
+        std::lock_guard<std::mutex> guard(g_lock);
+        for (c = g_captures; c && !(c->kind == kind && c->dev == dev);)
+            c = c->next;
+        if (!c || c->size < bytes)
+        {
+            /* Newest first, at least twice the last; the last stays. */
+            Capture* n = new (std::nothrow) Capture{kind, dev, nullptr,
+                    c && 2 * c->size > bytes ? 2 * c->size : bytes,
+                    g_captures};
+            *err = n ? hipMalloc(&n->ptr, n->size > 0 ? n->size : 1) :
+                    hipErrorOutOfMemory;
+            if (*err != hipSuccess)
+            {
+                delete n;
+                return nullptr;
+            }
+            g_captures = c = n;
+        }
+    }
+    if (capture != hipStreamCaptureStatusNone) return c->ptr;
+    return ws_acquire(kind, dev, stream, bytes, err);
 }
 
 std::mutex& ws_launch_lock() { return g_launch_lock; }

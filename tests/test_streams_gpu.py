@@ -13,7 +13,7 @@ from oskar_amd.mem import (OSKAR_COMPLEX, OSKAR_GPU, OSKAR_INT, OSKAR_MATRIX,
                            OSKAR_SINGLE, Jones, Mem, Sky, StationWork,
                            Telescope, check_status)
 from test_sky_gpu import I_JY, SCRATCH_L, SCRATCH_M, SCRATCH_N, make_sky
-from test_xcorr_seam_gpu import _stream_create, _stream_destroy
+from test_xcorr_seam_gpu import _hip, _stream_create, _stream_destroy
 
 pytestmark = pytest.mark.gpu
 
@@ -196,3 +196,38 @@ def test_more_streams_than_ever(hip):
         sync_check("acorr")
         for st in streams:
             _stream_destroy(st)
+
+
+@pytest.mark.parametrize("which", ["acorr", "prefix_sum"])
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_capture_on_a_new_stream(hip, which, mode):
+    """A call warmed on the null stream is captured on a stream that has not
+    run it (each capture mode); replays give the call's own result, also after
+    a larger call."""
+    x = Acorr(1, 60, 3000) if which == "acorr" else Prefix(1, 100001)
+    larger = Acorr(2, 512, 9000) if which == "acorr" else Prefix(2, 5000001)
+    want = serial([x], which)
+    api, graph, run = _hip(), C.c_void_p(), C.c_void_p()
+    s = C.c_int(0)
+    stream = _stream_create()
+    try:
+        lib.oskar_hip_set_stream(stream)
+        assert api.hipStreamBeginCapture(stream, mode) == 0
+        x.run(s)
+        assert api.hipStreamEndCapture(stream, C.byref(graph)) == 0
+        check_status(s, which)
+        assert api.hipGraphInstantiate(C.byref(run), graph, None, None,
+                                       C.c_size_t(0)) == 0
+        lib.oskar_hip_set_stream(None)
+        for k in range(4):
+            if k == 2:
+                serial([larger], which)
+            x.clear()
+            sync_check("clear")
+            assert api.hipGraphLaunch(run, stream) == 0
+            assert api.hipStreamSynchronize(stream) == 0
+            same([x], want)
+    finally:
+        lib.oskar_hip_set_stream(None)
+        sync_check(which)
+        _stream_destroy(stream)
